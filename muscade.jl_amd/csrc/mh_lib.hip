@@ -174,6 +174,8 @@ struct Ctx {
     int64_t cnu = 0;
     double* d_cbuf = nullptr;    // D | L | U (3·cnb·B²) | b (cnb·B) | pair couplings (4·cnp)
     double* d_csaved = nullptr;  // cnp × (3B+1): original rows of the held dofs
+    double* d_cred = nullptr;    // the block systems of the later phases of the reduction
+    std::vector<chain::System> csys;   // one per phase; the first is d_cbuf
     double* d_dx = nullptr;      // nX: Δx of the last solve
     unsigned* d_cflag = nullptr;
     unsigned* h_cflag = nullptr; // pinned
@@ -232,7 +234,7 @@ void free_graph(Ctx* c, int slot) {
 void free_graph(Ctx* c) { for (int k = 0; k < 4; ++k) free_graph(c, k); }
 void free_chain(Ctx* c) {
     dfree(c->d_cpos); dfree(c->d_chpos); dfree(c->d_cdum); dfree(c->d_cbuf); dfree(c->d_csaved); dfree(c->d_dx);
-    dfree(c->d_cslot); dfree(c->d_cunc); c->cnu = 0;
+    dfree(c->d_cslot); dfree(c->d_cunc); dfree(c->d_cred); c->csys.clear(); c->cnu = 0;
     dfree(c->d_cflag);
     if (c->h_cflag) { (void)hipHostFree(c->h_cflag); c->h_cflag = nullptr; }
     for (auto& e : c->cev) if (e) { (void)hipEventDestroy(e); e = nullptr; }
@@ -2955,19 +2957,15 @@ int enqueue_chain_solve(Ctx* c, const double* rhs, bool timed = true, bool fused
     if (c->cnp) hipLaunchKernelGGL(pair_kernel<B>, dim3(cgrid(c->cnp)), dim3(kCB), 0, s, c->cnp, c->d_chpos, pc, D, L,
                                    U, b, c->d_csaved, c->d_cflag);
     if (timed) HIPCHK(c, hipEventRecord(c->cev[1], s));
-    int64_t top = 1;
-    for (int64_t st = 1; st < nb; st *= 2) {
-        const int64_t nel = (nb - st + 2 * st - 1) / (2 * st), nkeep = (nb + 2 * st - 1) / (2 * st);
-        hipLaunchKernelGGL(factor_kernel<B>, dim3(cgrid(nel)), dim3(kCB), 0, s, nb, st, D, L, U, b, c->d_cflag);
-        hipLaunchKernelGGL(update_kernel<B>, dim3(cgrid(nkeep * B)), dim3(kCB), 0, s, nb, st, D, L, U, b);
-        top = 2 * st;
-    }
-    hipLaunchKernelGGL(top_kernel<B>, dim3(1), dim3(64), 0, s, D, b, c->d_cflag);
+    const auto& sy = c->csys;
+    const size_t np = sy.size();
+    auto chunks = [](const System& x) { return dim3((unsigned)((x.n + chain::kChunk - 1) / chain::kChunk)); };
+    for (size_t p = 0; p + 1 < np; ++p)
+        hipLaunchKernelGGL(reduce_kernel<B>, chunks(sy[p]), dim3(kReduceThreads), 0, s, sy[p], sy[p + 1], c->d_cflag);
+    hipLaunchKernelGGL(top_kernel<B>, dim3(1), dim3(kTopThreads), 0, s, sy[np - 1], c->d_cflag);
     if (timed) HIPCHK(c, hipEventRecord(c->cev[2], s));
-    for (int64_t st = top / 2; st >= 1; st /= 2) {
-        const int64_t nel = (nb - st + 2 * st - 1) / (2 * st);
-        hipLaunchKernelGGL(back_kernel<B>, dim3(cgrid(nel * B)), dim3(kCB), 0, s, nb, st, L, U, b);
-    }
+    for (size_t p = np - 1; p-- > 0;)
+        hipLaunchKernelGGL(back_kernel<B>, chunks(sy[p]), dim3(chain::kChunk * B), 0, s, sy[p], (const double*)sy[p + 1].b);
     hipLaunchKernelGGL(unpack_kernel<B>, dim3(cgrid(c->nX)), dim3(kCB), 0, s, c->nX, nb, c->d_cpos, c->d_chpos, pc,
                        c->d_csaved, b, c->d_dx);
     if (timed) HIPCHK(c, hipEventRecord(c->cev[3], s));
@@ -3060,6 +3058,24 @@ int mh_chain_prepare(mh_ctx* c, int B, int64_t nblock, const int64_t* pos, int64
     HIPCHK(c, hipMalloc(&c->d_cflag, chain::kStatusBytes));
     HIPCHK(c, hipHostMalloc((void**)&c->h_cflag, chain::kStatusBytes, hipHostMallocDefault));
     for (auto& e : c->cev) HIPCHK(c, hipEventCreate(&e));
+    {   // the phases of the reduction: each leaves the first block of every chunk to the next
+        chain::System x;
+        const int64_t BB = (int64_t)B * B;
+        x.n = nblock; x.D = c->d_cbuf; x.L = x.D + nblock * BB; x.U = x.L + nblock * BB; x.b = x.U + nblock * BB;
+        c->csys.push_back(x);
+        int64_t tot = 0;
+        for (int64_t m = nblock; m > chain::kTopBlocks;) { m = (m + chain::kChunk - 1) / chain::kChunk; tot += m * (4 * BB + 2 * B); }
+        if (tot) HIPCHK(c, hipMalloc(&c->d_cred, sizeof(double) * tot));
+        double* w = c->d_cred;
+        while (x.n > chain::kTopBlocks) {
+            x.n = (x.n + chain::kChunk - 1) / chain::kChunk;
+            x.stride *= chain::kChunk;
+            x.D = w; x.D2 = x.D + x.n * BB; x.L = x.D2 + x.n * BB; x.U = x.L + x.n * BB;
+            x.b = x.U + x.n * BB; x.b2 = x.b + x.n * B;
+            w = x.b2 + x.n * B;
+            c->csys.push_back(x);
+        }
+    }
     if (c->nX) HIPCHK(c, copy_sync(c, c->d_cpos, p32.data(), sizeof(int32_t) * c->nX, hipMemcpyHostToDevice));
     if (npair) HIPCHK(c, copy_sync(c, c->d_chpos, h32.data(), sizeof(int32_t) * npair, hipMemcpyHostToDevice));
     if (ndummy) HIPCHK(c, copy_sync(c, c->d_cdum, d32.data(), sizeof(int32_t) * ndummy, hipMemcpyHostToDevice));
