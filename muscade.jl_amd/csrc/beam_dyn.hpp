@@ -513,39 +513,6 @@ template <int NT, bool E> MH_HD void dyn_seed(const double (*X)[12], const doubl
     }
 }
 
-// Value pass: the frozen loads of the dynamic element, eg[gp] = dL_gp·fₑ(gp) and
-// mtot = Σ_gp dL_gp·mₑ, for beam_static<true>. X: ND rows of 12 element dofs.
-// kb (optional, stride ks): the ε-free kinematics that dyn_translation_direction reads, the
-// kDynBase numbers ∂ⁿrₛₘ(i,j)/∂tⁿ at n·9 + i + 3j (n < 3) and ẋ_gp,i at 27 + 3·gp + i.
-constexpr int kDynBase = 39;
-template <int ND> MH_HD void dyn_frozen_loads(const BeamGeo& G, const BeamDynSection& D, const double (*X)[12],
-                                              const double* U, v3* eg, v3& mtot, double* kb = nullptr,
-                                              int64_t ks = 1) {
-    Jet<ND, false> Xj[12];
-    dyn_seed<ND, false>(X, nullptr, nullptr, -1, Xj);
-    DynKin<false> k;
-    dyn_kinematics<ND, false>(G, Xj, k);
-    if (kb) {
-#pragma unroll
-        for (int q = 0; q < 9; ++q) {
-            kb[q * ks] = k.r0[q].v[0];
-            kb[(9 + q) * ks] = k.r1[q].v[0];
-            kb[(18 + q) * ks] = k.r2[q].v[0];
-        }
-#pragma unroll
-        for (int g = 0; g < 4; ++g)
-#pragma unroll
-            for (int i = 0; i < 3; ++i) kb[(27 + 3 * g + i) * ks] = k.xd[g][i].v[0];
-    }
-    Jet<1, false> fe[4][3], me[3];
-    dyn_loads<false>(k, D, U, fe, me);
-    mtot = mk(0., 0., 0.);
-    for (int g = 0; g < 4; ++g) {
-        eg[g] = G.dL[g] * mk(fe[g][0].v[0], fe[g][1].v[0], fe[g][2].v[0]);
-        mtot = mtot + G.dL[g] * mk(me[0].v[0], me[1].v[0], me[2].v[0]);
-    }
-}
-
 // Requestables of the element (BeamElement.jl:28-64,151-174) at X (ND time levels), what
 // getresult extracts (src/Output.jl:131-181). getresult evaluates the element on plain
 // values, so the time jets carry no solver partials and every square is exact (no
@@ -660,111 +627,6 @@ MH_HD void gauge_jets(const BeamGeo& G, const double* X0, int i, int j, Jet<2, t
     q[3] = (2. / L) * (-vl.a[1]);
 }
 
-// One trial direction (see dyn_seed): the ε-derivatives of the loads (DF, Dm) and,
-// for a δX direction, the column of the Jacobians of x_gp and vₛₘ w.r.t. X₀ (Jx, Jv).
-struct DynDir { double DF[4][3]; double Dm[3]; double Jx[4][3]; double Jv[3]; };
-// ROTE = false only for δX along a translation dof (0..2, 6..8): rₛₘ and vₛₘ then carry no ε.
-template <int ND, bool ROTE = true>
-MH_HD void dyn_direction(const BeamGeo& G, const BeamDynSection& D, const double (*X)[12], const double* U,
-                         const double* scale, const double* c, int dir, DynDir& o, double w0 = 1.,
-                         const double* lam = nullptr) {
-    Jet<ND, true> Xj[12];
-    dyn_seed<ND, true>(X, scale, c, dir, Xj, w0, lam);
-    DynKin<true> k;
-    dyn_kinematics<ND, true, ROTE>(G, Xj, k);
-    Jet<1, true> fe[4][3], me[3];
-    dyn_loads<true>(k, D, U, fe, me);
-    for (int g = 0; g < 4; ++g)
-        for (int q = 0; q < 3; ++q) { o.DF[g][q] = fe[g][q].e[0]; o.Jx[g][q] = k.xe[g][q]; }
-    for (int q = 0; q < 3; ++q) o.Dm[q] = me[q].e[0];
-    if constexpr (ROTE) {
-        v3 jv = dyn_vsm_e(k.r0);
-        o.Jv[0] = jv.x; o.Jv[1] = jv.y; o.Jv[2] = jv.z;
-    } else {
-        o.Jv[0] = 0.; o.Jv[1] = 0.; o.Jv[2] = 0.;
-    }
-}
-// The δX direction along a translation dof (dir 0..2, 6..8) in closed form, from the
-// kinematics jets k of any direction of the same element (only their ε-free parts are read).
-// Along a translation rₛₘ and vₛₘ carry no ε, so with the seed σ = (w0·s, a₁s, b₁s) on dof
-// component c of node 1 (η = −½) or node 2 (η = +½):
-//   x_gp,ε = (η·M_gp(:,c) + ½·e_c) ⊛ σ,   M_gp = rₛₘ·diag(ya, yu, yu)·rₛₘᵀ   (Leibniz products
-// of time jets), the loads vary through ẋ and ẍ alone, and the roll couple mₑ not at all:
-//   DFᵢ = μ·ẍᵢ,ε + Σⱼ r₀(i,j)·(Caⱼ·(r₀ᵀẍ_ε)ⱼ + (Clⱼ + 2Cqⱼ|(r₀ᵀẋ)ⱼ|)·(r₀ᵀẋ_ε)ⱼ).
-// The same numbers as dyn_direction<ND, false>(…, dir, …) up to rounding.
-template <int ND>
-MH_HD void dyn_translation_direction(const BeamGeo& G, const BeamDynSection& D, const double* kb, int64_t ks,
-                                     const double* scale, const double* c, int dir, DynDir& o, double w0 = 1.) {
-    const bool node2 = dir >= 6;
-    const int cc = node2 ? dir - 6 : dir;
-    const double eta = node2 ? 0.5 : -0.5;
-    const double s = scale[dir];
-    const double sg0 = w0 * s, sg1 = ND > 1 ? c[0] * s : 0., sg2 = ND > 2 ? c[3] * s : 0.;
-    // R[n][i + 3j]: ∂ⁿrₛₘ(i,j)/∂tⁿ
-    double R[3][9];
-#pragma unroll
-    for (int q = 0; q < 9; ++q) { R[0][q] = kb[q * ks]; R[1][q] = kb[(9 + q) * ks]; R[2][q] = kb[(18 + q) * ks]; }
-    // Wᵢⱼ = rₛₘ(i,j) ⊛ rₛₘ(c,j): the gp-independent products of M_gp(i,c) = Σⱼ Yⱼ Wᵢⱼ
-    // row cc of R by selects (an index known only at run time would put R in scratch memory)
-    double Rc[3][3];
-#pragma unroll
-    for (int m = 0; m < 3; ++m)
-#pragma unroll
-        for (int j = 0; j < 3; ++j) Rc[m][j] = cc == 0 ? R[m][3 * j] : (cc == 1 ? R[m][3 * j + 1] : R[m][3 * j + 2]);
-    double W[3][3][3];
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            const int a = i + 3 * j;
-            W[i][j][0] = R[0][a] * Rc[0][j];
-            W[i][j][1] = R[1][a] * Rc[0][j] + R[0][a] * Rc[1][j];
-            W[i][j][2] = (R[2][a] * Rc[0][j] + 2. * (R[1][a] * Rc[1][j])) + R[0][a] * Rc[2][j];
-        }
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-        const double z = G.zgp[g];
-        const double Y[3] = {2. * z, -4. * (z * z * z) + 3. * z, -4. * (z * z * z) + 3. * z};
-        double xd[3], xdd[3];
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
-            double m[3];
-#pragma unroll
-            for (int n = 0; n < 3; ++n) m[n] = eta * ((Y[0] * W[i][0][n] + Y[1] * W[i][1][n]) + Y[2] * W[i][2][n]);
-            if (i == cc) m[0] = m[0] + 0.5;
-            o.Jx[g][i] = m[0] * sg0;
-            xd[i] = ND > 1 ? m[1] * sg0 + m[0] * sg1 : 0.;
-            xdd[i] = ND > 2 ? (m[2] * sg0 + 2. * (m[1] * sg1)) + m[0] * sg2 : 0.;
-        }
-        double fl[3];
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            const double l1 = (kb[(27 + 3 * g) * ks] * R[0][3 * j] + kb[(28 + 3 * g) * ks] * R[0][3 * j + 1]) +
-                              kb[(29 + 3 * g) * ks] * R[0][3 * j + 2];
-            const double l1e = (xd[0] * R[0][3 * j] + xd[1] * R[0][3 * j + 1]) + xd[2] * R[0][3 * j + 2];
-            const double l2e = (xdd[0] * R[0][3 * j] + xdd[1] * R[0][3 * j + 1]) + xdd[2] * R[0][3 * j + 2];
-            fl[j] = D.Ca[j] * l2e + (D.Cl[j] + 2. * (D.Cq[j] * fabs(l1))) * l1e;
-        }
-#pragma unroll
-        for (int i = 0; i < 3; ++i)
-            o.DF[g][i] = D.mu * xdd[i] + ((R[0][i] * fl[0] + R[0][i + 3] * fl[1]) + R[0][i + 6] * fl[2]);
-    }
-#pragma unroll
-    for (int q = 0; q < 3; ++q) { o.Dm[q] = 0.; o.Jv[q] = 0.; }
-}
-// Row i of the load-variation part of the tangent along direction d:
-// Σ_gp dL_gp·(∂x_gp/∂X₀ᵢ · DF_gp + ∂vₛₘ/∂X₀ᵢ · Dm)   (Jx_i, Jv_i: column i of the Jacobians,
-// from the δX direction i, so already × scale.X[i] — the scaling of row i of R)
-MH_HD double dyn_row(const BeamGeo& G, const double (*Jx_i)[3], const double* Jv_i, const DynDir& d) {
-    double s = 0.;
-    for (int g = 0; g < 4; ++g) {
-        double t = (Jx_i[g][0] * d.DF[g][0] + Jx_i[g][1] * d.DF[g][1]) + Jx_i[g][2] * d.DF[g][2];
-        t = t + ((Jv_i[0] * d.Dm[0] + Jv_i[1] * d.Dm[1]) + Jv_i[2] * d.Dm[2]);
-        s = s + t * G.dL[g];
-    }
-    return s;
-}
-
 // ---- adjoint (vector-Jacobian products) of the residual ------------------------
 // For L = Λ·R the load part of ∂L/∂X⁽ᵈ⁾ₖ is Σ_gp dL (y_gp·∂fₑ/∂X⁽ᵈ⁾ₖ + y_v·∂mₑ/∂X⁽ᵈ⁾ₖ) with
 // y_gp = J_x,gp Λ and y_v = J_v Λ, the derivatives of x_gp and vₛₘ along Λ.
@@ -779,74 +641,11 @@ MH_HD void dyn_y(const BeamGeo& G, const double (*X)[12], const double* lam, Dyn
     v3 jv = dyn_vsm_e(k.r0);
     o.yv[0] = jv.x; o.yv[1] = jv.y; o.yv[2] = jv.z;
 }
-MH_HD double dyn_ycontract(const BeamGeo& G, const DynY& y, const DynDir& d) {
-    double s = 0.;
-    for (int g = 0; g < 4; ++g) {
-        double t = (y.y[g][0] * d.DF[g][0] + y.y[g][1] * d.DF[g][1]) + y.y[g][2] * d.DF[g][2];
-        t = t + ((y.yv[0] * d.Dm[0] + y.yv[1] * d.Dm[1]) + y.yv[2] * d.Dm[2]);
-        s = s + t * G.dL[g];
-    }
-    return s;
-}
 // ∂L/∂U (U-dofs: fₑ - U, per length): -Σ_gp dL y_gp
 MH_HD v3 dyn_vjp_u(const BeamGeo& G, const DynY& y) {
     v3 s = mk(0., 0., 0.);
     for (int g = 0; g < 4; ++g) s = s + G.dL[g] * mk(y.y[g][0], y.y[g][1], y.y[g][2]);
     return mk(-s.x, -s.y, -s.z);
-}
-// Whole dynamic element on one thread (host checks): gX[der][k] = Σ_i Λᵢ ∂Rᵢ/∂X⁽ᵈᵉʳ⁾ₖ (unscaled)
-// for der < ND, gU = Λ·∂R/∂U.
-template <int ND> MH_HD int dyn_vjp_element(const BeamGeo& G, const BeamSection& S, const BeamDynSection& D,
-                                            const double (*X)[12], const double* U, const double* lam, double (*gX)[12],
-                                            double* gU) {
-    v3 eg[4], mtot;
-    dyn_frozen_loads<ND>(G, D, X, U, eg, mtot);
-    BeamOut out;
-    beam_static<true>(G, S, mk(0., 0., 0.), X[0], out, eg, mtot);
-    DynY y;
-    dyn_y(G, X, lam, y);
-    const double one[12] = {1., 1., 1., 1., 1., 1., 1., 1., 1., 1., 1., 1.};
-    int nan = out.nan;
-    for (int der = 0; der < ND; ++der) {
-        double c[6] = {der == 1 ? 1. : 0., 0., 0., der == 2 ? 1. : 0., 0., 0.};
-        for (int k = 0; k < 12; ++k) {
-            DynDir d;
-            dyn_direction<ND>(G, D, X, U, one, c, k, d, der == 0 ? 1. : 0.);
-            double g = dyn_ycontract(G, y, d);
-            if (der == 0)
-                for (int i = 0; i < 12; ++i) g = g + compact_entry(out.Kc, k, i) * lam[i];
-            gX[der][k] = g;
-            nan |= g != g;
-        }
-    }
-    v3 gu = dyn_vjp_u(G, y);
-    gU[0] = gu.x; gU[1] = gu.y; gU[2] = gu.z;
-    return nan;
-}
-
-// Whole element on one thread (host checks): scaled R, K = ∂R/∂δX (12×12,
-// column-major) and, for :step, dRr = ∂R/∂δr. c = Newmark (a₁,a₂,a₃,b₁,b₂,b₃).
-template <int ND> MH_HD int dyn_element(const BeamGeo& G, const BeamSection& S, const BeamDynSection& D,
-                                        const double (*X)[12], const double* U, const double* scale, const double* c,
-                                        double* R, double* K, double* dRr) {
-    v3 eg[4], mtot;
-    dyn_frozen_loads<ND>(G, D, X, U, eg, mtot);
-    BeamOut out;
-    beam_static<true>(G, S, mk(0., 0., 0.), X[0], out, eg, mtot);
-    DynDir dir[12];
-    for (int k = 0; k < 12; ++k) dyn_direction<ND>(G, D, X, U, scale, c, k, dir[k]);
-    for (int i = 0; i < 12; ++i) R[i] = out.R[i] * scale[i];
-    for (int k = 0; k < 12; ++k)
-        for (int i = 0; i < 12; ++i)
-            K[i + 12 * k] = compact_entry(out.Kc, i, k) * (scale[i] * scale[k]) + dyn_row(G, dir[i].Jx, dir[i].Jv, dir[k]);
-    if (dRr) {
-        DynDir r;
-        dyn_direction<ND>(G, D, X, U, scale, c, 12, r);
-        for (int i = 0; i < 12; ++i) dRr[i] = dyn_row(G, dir[i].Jx, dir[i].Jv, r);
-    }
-    int nan = out.nan;
-    for (int i = 0; i < 144; ++i) nan |= K[i] != K[i];
-    return nan;
 }
 
 }  // namespace mh

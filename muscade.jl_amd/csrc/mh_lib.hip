@@ -35,6 +35,7 @@
 #include "../../include/muscade_hip.h"
 #include "beam_math.hpp"
 #include "beam_dyn.hpp"
+#include "beam_dir.hpp"
 #include "bar_math.hpp"
 #include "chain_solve.hpp"
 
@@ -57,6 +58,7 @@ struct Group {
     int64_t kbase = 0, rbase = 0;
     int64_t kper = 0;            // Kbuf entries per element (45 for static beams, nX² otherwise)
     int64_t kcbase = 0;          // dynamic beams: offset of the compact static part in Kc
+    int64_t recbase = 0;         // dynamic beams: offset of the records
     int64_t ubase = 0;           // U-dof groups: offset of the per-element ∂L/∂U entries
     int64_t kdbase = 0, kubase = 0;   // AssemblyDirect: offsets of the ∂R/∂X⁽ᵈ⁾ and ∂R/∂U blocks
     bool compact = false;
@@ -95,8 +97,7 @@ struct Ctx {
     bool coded = false;          // ksrc carries multiplier codes (compact groups present)
     int64_t nK = 0, nP = 0, nR = 0, nnz = 0;
     double* d_Kc = nullptr;      // dynamic beams: scaled compact static part, 45 per element
-    double* d_Kb = nullptr;      // dynamic beams (SweepX): ε-free kinematics, mh::kDynBase per element
-    double* d_ybuf = nullptr;    // dynamic beams (adjoint): y = (J_x Λ, J_v Λ), 15 per element
+    double* d_rec = nullptr;     // dynamic beams: the elements' records (mh::DynRec), in tiles of kDynTile
     double* d_c6 = nullptr;      // SweepX: the Newmark coefficients of the current call (6)
     double* h_c6 = nullptr;      // pinned staging of d_c6
     double* d_Kbuf = nullptr;
@@ -256,7 +257,7 @@ void free_prepared(Ctx* c) {
     free_graph(c);
     free_chain(c);
     free_big(c);
-    dfree(c->d_Kbuf); dfree(c->d_Rbuf); dfree(c->d_dRbuf); dfree(c->d_nzval); dfree(c->d_rhs); dfree(c->d_Kc); dfree(c->d_Kb); dfree(c->d_ybuf);
+    dfree(c->d_Kbuf); dfree(c->d_Rbuf); dfree(c->d_dRbuf); dfree(c->d_nzval); dfree(c->d_rhs); dfree(c->d_Kc); dfree(c->d_rec);
     dfree(c->d_colptr); dfree(c->d_rowval); dfree(c->d_kseg); dfree(c->d_ksrc); dfree(c->d_rseg); dfree(c->d_rsrc);
     dfree(c->d_useg); dfree(c->d_usrc); dfree(c->d_gbuf); dfree(c->d_gX); dfree(c->d_gubuf); dfree(c->d_gU);
     dfree(c->d_aseg); dfree(c->d_asrc); dfree(c->d_gabuf); dfree(c->d_gA); dfree(c->d_crhs);
@@ -465,7 +466,8 @@ struct BeamDynArgs {
     double* dR;         // ∂R/∂δr (:step)
     unsigned long long* flag;
     unsigned long long gtag;
-    double* Kb = nullptr;   // value pass → direction pass: ε-free kinematics, mh::kDynBase × nele (SoA)
+    double* rec = nullptr;   // value pass → direction passes: number q of element e at
+                             // (e / kDynTile · kDynRec + q) · kDynTile + e % kDynTile
 };
 
 template <int ND, bool UDOF>
@@ -491,8 +493,12 @@ __device__ __forceinline__ void dyn_load(const BeamDynArgs& a, int64_t e, mh::Be
     }
 }
 
-// Value pass, one element per lane: the frozen loads of the time jets, then the
-// residual and the compact tangent of Π with those loads held fixed.
+// Value pass, one element per lane: the element's record and the frozen loads from the time jets,
+// then the residual and the compact tangent of Π with those loads held fixed.
+constexpr int kDynTile = 64;   // elements whose records lie together
+constexpr int kDynRecMax = mh::kDynRec<3>;
+static_assert(kBeamBlock % kDynTile == 0, "whole tiles per workgroup");
+int64_t rec_numbers(int64_t nele) { return (nele + kDynTile - 1) / kDynTile * kDynTile * kDynRecMax; }
 template <int ND, bool UDOF>
 __global__ __launch_bounds__(kBeamBlock) void beam_dyn_value_kernel(BeamDynArgs a) {
     __shared__ double tile[kBeamBlock * mh::kCompact];
@@ -509,7 +515,8 @@ __global__ __launch_bounds__(kBeamBlock) void beam_dyn_value_kernel(BeamDynArgs 
         double X[ND][12], U[3];
         dyn_load<ND, UDOF>(a, e, G, S, D, X, U);
         mh::v3 eg[4], mtot;
-        mh::dyn_frozen_loads<ND>(G, D, X, U, eg, mtot, a.Kb ? a.Kb + e : nullptr, n);
+        double* rec = a.rec + e / kDynTile * (kDynTile * mh::kDynRec<ND>) + e % kDynTile;
+        mh::dyn_record<ND>(G, D, X, U, [&](int q, double v) { rec[q * kDynTile] = v; }, eg, mtot);
         mh::BeamOut out;
         mh::beam_static<true>(G, S, mh::mk(0., 0., 0.), X[0], out, eg, mtot, hmsh + tid, kBeamBlock);
         if (a.R) {
@@ -587,103 +594,172 @@ __global__ __launch_bounds__(kBlock) void beam_gauge_derivs_kernel(BeamDynArgs a
     }
 }
 
-// Direction pass, one wave per workgroup of kDirElemsW(STEP) elements, after the value pass
-// (which leaves the compact static part in Kc and the ε-free kinematics in Kb). One lane per
-// rotation dof of an element (δX of dofs 3..5, 9..11) and, on :step, one for δr. A lane first
-// evaluates the δX direction of one translation dof (0..2, 6..8) in closed form from Kb
-// (mh::dyn_translation_direction: along a translation the rotation chain carries no ε), then
-// propagates the time jets with its own ε seed. The lanes of an element exchange the Jacobian
-// columns of x_gp and vₛₘ (and the translation load derivatives) through LDS, and each lane
-// forms the columns k of its directions, K[:,k] = (compact static part) +
-// Σ_gp dL·(J_xᵀ ∂fₑ/∂ε + J_vᵀ ∂mₑ/∂ε), in LDS (the workgroup then writes its elements' K blocks
-// as one contiguous range), or ∂R/∂δr.
-constexpr int kDirLanes = 16;              // the adjoint and DirectXUA kernels: 16 lanes per element
-constexpr int kDirElems = 16;
-constexpr int kDirBlock = kDirLanes * kDirElems;
-constexpr int kDirWBlock = 64;             // SweepX direction pass: one wave
-template <bool STEP> constexpr int kDirPerW = STEP ? 7 : 6;             // lanes per element
-template <bool STEP> constexpr int kDirElemsW = kDirWBlock / kDirPerW<STEP>;   // 9 on :step, 10 on :iter
-template <int ND, bool UDOF, bool STEP>
-__global__ __launch_bounds__(kDirWBlock) void beam_dyn_dir_kernel(BeamDynArgs a) {
-    constexpr int per = kDirPerW<STEP>, NE = kDirElemsW<STEP>;
-    __shared__ double Jsh[NE][12][15];      // per dof: Jx (4 gp × 3), Jv (3)
-    __shared__ double DFt[NE][6][12];       // per translation dof: ∂fₑ/∂ε (4 gp × 3); ∂mₑ/∂ε = 0
-    __shared__ double Ksh[NE][144];         // the elements' K blocks, written out as one contiguous range
-    const int64_t e0 = xcd_tile(a.per_xcd) * NE;
-    if (e0 >= a.nele) return;   // whole workgroup leaves together
-    const int el = threadIdx.x / per, j = threadIdx.x - el * per;
-    const int dir = j < 3 ? 3 + j : (j < 6 ? 6 + j : 12);        // r of node 1, r of node 2, δr
-    const int dir_t = j < 3 ? j : j + 3;                          // t of node 1, t of node 2 (j < 6)
-    const int64_t e = e0 + el;
+// Direction passes, after the value pass, which leaves the compact static part in Kc and the records:
+// a workgroup of four waves per tile of elements. Lane 6e + j of element e owns one rotation dof (3..5,
+// 9..11) and one translation dof (0..2, 6..8); on :step the fourth wave has one lane per element for δr.
+// Records, node rotations and sections are staged in LDS, where the six lanes read them as they need
+// them; the rows of the load part's Jacobian are exchanged there, the columns go straight to memory.
+// Bound: FP64 latency at two waves per SIMD, then HBM. A direction of second order is about 2,200
+// FP64 instructions, against 12,700 operations in time jets with an ε seed, which took 450 registers
+// (one wave per SIMD). The tile of K leaves through LDS: stored by its lanes, every line of it was
+// written in 16 requests to L2 (663 µs against 485). 383,000 elements, second order, :iter: 1384 µs
+// with jets, 485 now.
+constexpr int kDirLanes = 256;
+constexpr int kDirTile = kDirLanes / 6;    // elements of a workgroup: 42 (LDS: two workgroups per CU)
+constexpr int kStepTile = kDirLanes / 8;   // on :step 32, three waves of directions and one of δr
+// An element in LDS. An odd number of doubles: no bank is favoured.
+template <int ND> struct DynElem {
+    mh::DynRec<ND> rec;
+    double V[ND][6];   // node rotations on time levels
+    mh::BeamDynSection sec;
+};
+static_assert(sizeof(DynElem<1>) / 8 % 2 == 1 && sizeof(DynElem<2>) / 8 % 2 == 1 && sizeof(DynElem<3>) / 8 % 2 == 1, "odd");
+// Lane j of an element: its rotation dof (node j/3, component j%3) and translation dof likewise.
+__device__ __forceinline__ int rot_dof(int j) { return j < 3 ? 3 + j : 6 + j; }
+__device__ __forceinline__ int tr_dof(int j) { return j < 3 ? j : 3 + j; }
+
+template <int ND, int T, class Args>
+__device__ __forceinline__ void stage_elements(const Args& a, int64_t e0, DynElem<ND>* __restrict__ lds) {
+    constexpr int kSec = sizeof(mh::BeamDynSection) / sizeof(double), kRows = kDirLanes / T;
     const int64_t n = a.nele;
-    const bool live = el < NE && e < n;
-    mh::BeamGeo G;
-    mh::DynDir d;
-    if (live) {
-        mh::BeamSection S;
-        mh::BeamDynSection D;
-        double X[ND][12], U[3];
-        dyn_load<ND, UDOF>(a, e, G, S, D, X, U);
-        if (j < 6) {
-            mh::DynDir dt;
-            mh::dyn_translation_direction<ND>(G, D, a.Kb + e, n, a.scale, a.dc ? a.dc : a.c, dir_t, dt);
+    const int el = threadIdx.x % T, q0 = threadIdx.x / T;
+    const int64_t e = e0 + el;
+    if (q0 < kRows && e < n) {
+        const double* src = a.rec + e / kDynTile * (mh::kDynRec<ND> * kDynTile) + e % kDynTile;
+        double* dst = reinterpret_cast<double*>(&lds[el].rec);
+#pragma unroll 6
+        for (int q = q0; q < mh::kDynRec<ND>; q += kRows) dst[q] = src[q * kDynTile];
+        for (int k = q0; k < 6; k += kRows) {
+            const int32_t q = a.idx[rot_dof(k) * n + e];
 #pragma unroll
-            for (int g = 0; g < 4; ++g)
-#pragma unroll
-                for (int q = 0; q < 3; ++q) { Jsh[el][dir_t][3 * g + q] = dt.Jx[g][q]; DFt[el][j][3 * g + q] = dt.DF[g][q]; }
-#pragma unroll
-            for (int q = 0; q < 3; ++q) Jsh[el][dir_t][12 + q] = 0.;
+            for (int d = 0; d < ND; ++d) lds[el].V[d][k] = a.X[d][q];
         }
-        mh::dyn_direction<ND, true>(G, D, X, U, a.scale, a.dc ? a.dc : a.c, dir, d);
-        if (dir < 12) {
-#pragma unroll
-            for (int g = 0; g < 4; ++g)
-#pragma unroll
-                for (int q = 0; q < 3; ++q) Jsh[el][dir][3 * g + q] = d.Jx[g][q];
-#pragma unroll
-            for (int q = 0; q < 3; ++q) Jsh[el][dir][12 + q] = d.Jv[q];
+        for (int i = q0; i < kSec; i += kRows) {   // mu, iota1, w, then (Ca, Cl, Cq) per axis
+            const int c = (i - 3) / 3, q = (i - 3) % 3;
+            (&lds[el].sec.mu)[i] = a.sec[(i < 3 ? 4 + i : 7 + 3 * q + c) * n + e];
         }
     }
     __syncthreads();
+}
+// Column of the symmetric static part from the compact block (beam_math.hpp): of rotation dof r
+// (0..5) or of translation dof (node m, component c). t1, t2: the translation rows of node 1, 2; v: the
+// rotation rows.
+__device__ __forceinline__ void static_rot_col(const double* __restrict__ kc, int r, mh::v3& t1, mh::v3& t2, double (&v)[6]) {
+    const mh::v3 t = mh::mk(0.5 * kc[6 + r], 0.5 * kc[12 + r], 0.5 * kc[18 + r]);
+    t1 = mh::mk(-t.x, -t.y, -t.z);
+    t2 = t;
+#pragma unroll
+    for (int i = 0; i < 6; ++i) v[i] = kc[24 + mh::sym6(i, r)];
+}
+__device__ __forceinline__ void static_tr_col(const double* __restrict__ kc, int m, int c, mh::v3& t1, mh::v3& t2, double (&v)[6]) {
+    const mh::v3 q = mh::mk(0.25 * kc[mh::sym3(0, c)], 0.25 * kc[mh::sym3(1, c)], 0.25 * kc[mh::sym3(2, c)]);
+    const mh::v3 nq = mh::mk(-q.x, -q.y, -q.z);
+    t1 = m ? nq : q;
+    t2 = m ? q : nq;
+    const double h = m ? 0.5 : -0.5;
+#pragma unroll
+    for (int i = 0; i < 6; ++i) v[i] = h * kc[6 + 6 * c + i];
+}
+// One column: the translation rows t1, t2 and rotation rows v of an element's 12.
+__device__ __forceinline__ bool store_col(double* __restrict__ dst, mh::v3 t1, mh::v3 t2, const double (&v)[6]) {
+    const double c[12] = {t1.x, t1.y, t1.z, v[0], v[1], v[2], t2.x, t2.y, t2.z, v[3], v[4], v[5]};
+    bool nan = false;
+#pragma unroll
+    for (int i = 0; i < 12; ++i) { dst[i] = c[i]; nan = nan || c[i] != c[i]; }
+    return nan;
+}
+__device__ __forceinline__ mh::v3 had(const double* s, mh::v3 a) { return mh::mk(s[0] * a.x, s[1] * a.y, s[2] * a.z); }
+
+template <int ND, bool STEP>
+__global__ __launch_bounds__(kDirLanes, 2) void beam_dyn_dir_kernel(BeamDynArgs a) {
+    constexpr int T = STEP ? kStepTile : kDirTile;
+    // the records, then the columns of the tile: K goes to memory in whole lines
+    constexpr int kCol = 145;
+    __shared__ union Tile { DynElem<ND> lds[T]; double K[T * kCol]; __device__ Tile() {} } tile;
+    DynElem<ND>* lds = tile.lds;
+    __shared__ mh::DirRow rows[T][6];
+    __shared__ double path[STEP ? T : 1][ND][12];
+    const int64_t e0 = xcd_tile(a.per_xcd) * T;
+    if (e0 >= a.nele) return;   // whole workgroup leaves together
+    stage_elements<ND, T>(a, e0, lds);
+    const int tid = threadIdx.x;
+    const bool dr = STEP && tid >= 6 * T;
+    const int el = dr ? tid - 6 * T : tid / 6, j = dr ? 6 : tid - el * 6;
+    const int64_t e = e0 + el, n = a.nele;
+    const bool live = el < T && e < n;
+    const mh::DynRec<ND>& R = lds[live ? el : 0].rec;
+    const mh::BeamDynSection& S = lds[live ? el : 0].sec;
+    const double (*V)[6] = lds[live ? el : 0].V;
+    const double* cf = a.dc ? a.dc : a.c;
+    const int nd = j / 3, k = j - 3 * nd;
+    mh::DirCol cr, ct;
+    mh::v3 r1, r2, t1, t2;   // translation rows of the two columns
     if (live) {
-        double col[12], colt[12];
-        int nan = 0;
-#pragma unroll
-        for (int i = 0; i < 12; ++i) {
-            const double(*Jx)[3] = (const double(*)[3])(&Jsh[el][i][0]);
-            col[i] = mh::dyn_row(G, Jx, &Jsh[el][i][12], d);
-            if (dir < 12) {
-                double t = 0.;
-#pragma unroll
-                for (int g = 0; g < 4; ++g)
-                    t = t + ((Jx[g][0] * DFt[el][j][3 * g] + Jx[g][1] * DFt[el][j][3 * g + 1]) +
-                             Jx[g][2] * DFt[el][j][3 * g + 2]) * G.dL[g];
-                double m;
-                int slot = mh::compact_slot(i, dir, &m);
-                col[i] = m * a.Kc[e * mh::kCompact + slot] + col[i];
-                slot = mh::compact_slot(i, dir_t, &m);
-                colt[i] = m * a.Kc[e * mh::kCompact + slot] + t;
-                nan |= colt[i] != colt[i];
-            }
-            nan |= col[i] != col[i];
-        }
-        if (dir < 12) {
-#pragma unroll
-            for (int i = 0; i < 12; ++i) Ksh[el][12 * dir + i] = col[i];
-#pragma unroll
-            for (int i = 0; i < 12; ++i) Ksh[el][12 * dir_t + i] = colt[i];
+        if (!dr) {
+            double sg[3];
+            const double sr = a.scale[rot_dof(j)], st = a.scale[tr_dof(j)];
+            sg[0] = sr; sg[1] = cf[0] * sr; sg[2] = cf[3] * sr;
+            mh::DirRow row;
+            mh::rotation_direction<ND>(S, R, V, nd, k, sg, row, cr);
+            rows[el][j] = row;
+            mh::translation_rows<ND>(R, cr, r1, r2);
+            MH_PHASE();
+            sg[0] = st; sg[1] = cf[0] * st; sg[2] = cf[3] * st;
+            mh::translation_direction<ND>(S, R, nd, k, sg, ct);
+            mh::translation_rows<ND>(R, ct, t1, t2);
         } else {
+            double (*dX)[12] = path[STEP ? el : 0];
 #pragma unroll
-            for (int i = 0; i < 12; ++i) a.dR[i * n + e] = col[i];
+            for (int i = 0; i < 12; ++i) {
+                const int32_t q = a.idx[i * n + e];
+                const double x1 = a.X[1][q], x2 = ND > 2 ? a.X[2][q] : 0.;
+                dX[0][i] = 0.;
+                dX[1][i] = ND > 2 ? cf[1] * x1 + cf[2] * x2 : cf[1] * x1;
+                if constexpr (ND > 2) dX[2][i] = cf[4] * x1 + cf[5] * x2;
+            }
+            MH_PHASE();
+            mh::DirRow row;
+            mh::full_direction<ND>(S, R, V, dX, row, cr);
+            mh::translation_rows<ND>(R, cr, r1, r2);
         }
-        if (nan) atomicMin(a.flag, a.gtag | (unsigned long long)e);
+    }
+    MH_PHASE();
+    mh::v3 s1, s2, q1, q2;
+    double sr[6], st[6];
+    if (live && !dr) {
+        const double* kc = a.Kc + e * mh::kCompact;
+        static_rot_col(kc, j, s1, s2, sr);
+        static_tr_col(kc, nd, k, q1, q2, st);
     }
     __syncthreads();
-    // the workgroup's elements are consecutive: their K blocks form one contiguous range
-    const int64_t nv = (n - e0 < NE ? n - e0 : NE) * 144;
+    bool nan = false;
+    if (live) {
+        double vr[6], vt[6];
+#pragma unroll
+        for (int i = 0; i < 6; ++i) {
+            const mh::DirRow& w = rows[el][i];
+            vr[i] = mh::rotation_row(w, cr);
+            if (!dr) vt[i] = mh::rotation_row(w, ct);
+        }
+        r1 = had(a.scale, r1); r2 = had(a.scale + 6, r2);
+        if (dr) {
+            const double c[12] = {r1.x, r1.y, r1.z, vr[0], vr[1], vr[2], r2.x, r2.y, r2.z, vr[3], vr[4], vr[5]};
+#pragma unroll
+            for (int i = 0; i < 12; ++i) { a.dR[i * n + e] = c[i]; nan = nan || c[i] != c[i]; }
+        } else {
+            t1 = had(a.scale, t1); t2 = had(a.scale + 6, t2);
+            double* K = tile.K + el * kCol;
+#pragma unroll
+            for (int i = 0; i < 6; ++i) { vr[i] = sr[i] + vr[i]; vt[i] = st[i] + vt[i]; }
+            nan = store_col(K + 12 * rot_dof(j), s1 + r1, s2 + r2, vr);
+            nan = store_col(K + 12 * tr_dof(j), q1 + t1, q2 + t2, vt) || nan;
+        }
+    }
+    __syncthreads();
+    const int64_t nv = (n - e0 < T ? n - e0 : T) * 144;
     double* dst = a.K + e0 * 144;
-    const double* src = &Ksh[0][0];
-    for (int64_t f = threadIdx.x; f < nv; f += kDirWBlock) dst[f] = src[f];
+    for (int f = tid; f < nv; f += kDirLanes) dst[f] = tile.K[f + f / 144];
+    if (nan) atomicMin(a.flag, a.gtag | (unsigned long long)e);
 }
 
 // ---- Bar3D -----------------------------------------------------------------
@@ -768,9 +844,7 @@ struct VjpArgs {
     const double* lam;
     double t;
     const double* Kc;    // dynamic beams: unscaled compact static part (value pass)
-    const double* Kb;    // dynamic beams: ε-free kinematics (value pass), mh::kDynBase per element
-    double* yb;          // dynamic beams: y = (J_x Λ, J_v Λ), 15 per element (yb[q*nele + e])
-    double one[12] = {1., 1., 1., 1., 1., 1., 1., 1., 1., 1., 1., 1.};   // unit dof scales
+    const double* rec;   // dynamic beams: the elements' records (value pass)
     double* g;           // g[der*gstride + i*nele + e]
     int64_t gstride;
     double* gu;          // gu[q*nele + e] (U-dof groups)
@@ -878,100 +952,69 @@ __global__ __launch_bounds__(kBeamBlock) void beam_vjp_a_kernel(VjpArgs a, int m
     }
 }
 
-// Dynamic beams, after the value pass with unit scales (the compact static part in Kc, the
-// ε-free kinematics in Kb), one element per lane: y = (J_x Λ, J_v Λ), the derivatives of x_gp
-// (4 × 3) and vₛₘ (3) along Λ (a first-order jet seeded with Λ), 15 numbers per element into
-// yb (yb[q·n + e]); the static part (Kc Λ)ₖ of ∂L/∂Xₖ into g; ∂L/∂U = −Σ_gp dL y_gp with U-dofs.
+// Dynamic beams, after the value pass with unit scales: a workgroup per tile of elements and lanes
+// as in the direction pass. A lane differentiates the loads along X⁽ᵈ⁾ₖ of its two dofs for every
+// time order d, contracts with y = J Λ (formed by each lane: it costs less than exchanging it), and
+// adds the static part (Kc Λ)ₖ for d = 0; the first lane of an element gives ∂L/∂U = −Σ_gp dL y_gp.
 template <int ND, bool UDOF>
-__global__ __launch_bounds__(kBlock) void beam_dyn_y_kernel(VjpArgs a) {
-    const int64_t e = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    const int64_t n = a.nele;
-    if (e >= n) return;
-    mh::BeamGeo G;
-    mh::BeamSection S;
-    mh::BeamDynSection D;
-    double X[ND][12], U[3], lam[12];
-    {
-        BeamDynArgs b;
-        b.nele = a.nele; b.idx = a.idx; b.uidx = a.uidx; b.nodes = a.nodes; b.xyz = a.xyz; b.o2 = a.o2; b.sec = a.sec;
-        for (int d = 0; d < 3; ++d) b.X[d] = a.X[d];
-        b.U = a.U;
-        dyn_load<ND, UDOF>(b, e, G, S, D, X, U);
+__global__ __launch_bounds__(kDirLanes, 2) void beam_dyn_vjp_kernel(VjpArgs a) {
+    __shared__ DynElem<ND> lds[kDirTile];
+    __shared__ mh::DirLam ys[kDirTile];
+    const int64_t e0 = xcd_tile(a.per_xcd) * kDirTile;
+    if (e0 >= a.nele) return;   // whole workgroup leaves together
+    stage_elements<ND, kDirTile>(a, e0, lds);
+    const int el = threadIdx.x / 6, j = threadIdx.x - el * 6;
+    const int64_t e = e0 + el, n = a.nele;
+    const bool live = el < kDirTile && e < n;
+    const mh::DynRec<ND>& R = lds[live ? el : 0].rec;
+    const mh::BeamDynSection& S = lds[live ? el : 0].sec;
+    const double (*V)[6] = lds[live ? el : 0].V;
+    const int nd = j / 3, k = j - 3 * nd;
+    double gr0 = 0., gt0 = 0.;
+    if (live) {
+        mh::DirLam y;
+        double lam[12];
+#pragma unroll
+        for (int i = 0; i < 12; ++i) lam[i] = a.lam[a.idx[i * n + e]];
+        mh::lambda_row<ND>(R, V, lam, y);
+        if (j == 0) ys[el] = y;
+        if (UDOF && j == 0) {
+            const mh::v3 gu = mh::row_load<ND>(R, y.r) + (0.5 * R.L) * mh::mk(lam[0] + lam[6], lam[1] + lam[7], lam[2] + lam[8]);
+            a.gu[e] = -gu.x; a.gu[n + e] = -gu.y; a.gu[2 * n + e] = -gu.z;
+        }
+        const mh::v3 l1 = mh::mk(lam[0], lam[1], lam[2]), l2 = mh::mk(lam[6], lam[7], lam[8]);
+        const double lr[6] = {lam[3], lam[4], lam[5], lam[9], lam[10], lam[11]};
+        const double* kc = a.Kc + e * mh::kCompact;
+        mh::v3 s1, s2;
+        double sv[6];
+        static_rot_col(kc, j, s1, s2, sv);
+        gr0 = mh::dot(s1, l1) + mh::dot(s2, l2);
+#pragma unroll
+        for (int i = 0; i < 6; ++i) gr0 = gr0 + sv[i] * lr[i];
+        static_tr_col(kc, nd, k, s1, s2, sv);
+        gt0 = mh::dot(s1, l1) + mh::dot(s2, l2);
+#pragma unroll
+        for (int i = 0; i < 6; ++i) gt0 = gt0 + sv[i] * lr[i];
     }
-#pragma unroll
-    for (int i = 0; i < 12; ++i) lam[i] = a.lam[a.idx[i * n + e]];
-    mh::DynY y;
-    mh::dyn_y(G, X, lam, y);
-#pragma unroll
-    for (int g = 0; g < 4; ++g)
-#pragma unroll
-        for (int q = 0; q < 3; ++q) a.yb[(3 * g + q) * n + e] = y.y[g][q];
-#pragma unroll
-    for (int q = 0; q < 3; ++q) a.yb[(12 + q) * n + e] = y.yv[q];
-    if (UDOF) {
-        const mh::v3 gu = mh::dyn_vjp_u(G, y);
-        a.gu[e] = gu.x; a.gu[n + e] = gu.y; a.gu[2 * n + e] = gu.z;
+    __syncthreads();
+    if (!live) return;
+    const mh::DirLam& y = ys[el];
+    bool nan = false;
+#pragma unroll 1
+    for (int der = 0; der < ND; ++der) {
+        const double sg[3] = {der == 0 ? 1. : 0., der == 1 ? 1. : 0., der == 2 ? 1. : 0.};
+        mh::DirRow row;
+        mh::DirCol col;
+        mh::rotation_direction<ND>(S, R, V, nd, k, sg, row, col);
+        const double gr = (der == 0 ? gr0 : 0.) + mh::lambda_contract(y, col);
+        MH_PHASE();
+        mh::translation_direction<ND>(S, R, nd, k, sg, col);
+        const double gt = (der == 0 ? gt0 : 0.) + mh::lambda_contract(y, col);
+        a.g[der * a.gstride + tr_dof(j) * n + e] = gt;
+        a.g[der * a.gstride + rot_dof(j) * n + e] = gr;
+        nan = nan || gt != gt || gr != gr;
     }
-    const double* kc = a.Kc + e * mh::kCompact;
-#pragma unroll
-    for (int k = 0; k < 12; ++k) {
-        double g = 0.;
-#pragma unroll
-        for (int i = 0; i < 12; ++i) g = g + mh::compact_entry(kc, k, i) * lam[i];
-        a.g[k * n + e] = g;
-    }
-}
-
-// Then one launch per time-derivative order DER: one wave per workgroup of kDirElemsW<false>
-// elements, 6 lanes per element, lane j owning one translation dof (0..2, 6..8) and one
-// rotation dof (3..5, 9..11) as in the direction pass. A lane differentiates the loads along
-// X⁽ᴰᴱᴿ⁾ₖ of its two dofs — the rotation on time jets, then the translation in closed form — and
-// contracts with y: ∂L/∂X⁽ᴰᴱᴿ⁾ₖ = Σ_gp dL (y_gp·∂fₑ/∂ε + y_v·∂mₑ/∂ε), added to the static part
-// for DER = 0. (All orders in one launch keep three jet passes' state live at once and spill
-// about 2 KB per lane.)
-template <int ND, bool UDOF, int DER>
-__global__ __launch_bounds__(kDirWBlock) void beam_dyn_vjp_kernel(VjpArgs a) {
-    constexpr int per = kDirPerW<false>, NE = kDirElemsW<false>;
-    const int64_t e0 = xcd_tile(a.per_xcd) * NE;
-    const int el = threadIdx.x / per, j = threadIdx.x - el * per;
-    const int64_t e = e0 + el;
-    const int64_t n = a.nele;
-    if (el >= NE || e >= n) return;
-    const int dir_t = j < 3 ? j : j + 3;     // t of node 1, t of node 2
-    const int dir_r = j < 3 ? 3 + j : 6 + j; // r of node 1, r of node 2
-    mh::BeamGeo G;
-    mh::BeamSection S;
-    mh::BeamDynSection D;
-    double X[ND][12], U[3];
-    {
-        BeamDynArgs b;
-        b.nele = a.nele; b.idx = a.idx; b.uidx = a.uidx; b.nodes = a.nodes; b.xyz = a.xyz; b.o2 = a.o2; b.sec = a.sec;
-        for (int d = 0; d < 3; ++d) b.X[d] = a.X[d];
-        b.U = a.U;
-        dyn_load<ND, UDOF>(b, e, G, S, D, X, U);
-    }
-    // the rotation direction first, while nothing else is live
-    const double c[6] = {DER == 1 ? 1. : 0., 0., 0., DER == 2 ? 1. : 0., 0., 0.};
-    constexpr double w0 = DER == 0 ? 1. : 0.;
-    mh::DynDir d;
-    mh::DynY y;
-    mh::dyn_direction<ND, true>(G, D, X, U, a.one, c, dir_r, d, w0);
-#pragma unroll
-    for (int g = 0; g < 4; ++g)
-#pragma unroll
-        for (int q = 0; q < 3; ++q) y.y[g][q] = a.yb[(3 * g + q) * n + e];
-#pragma unroll
-    for (int q = 0; q < 3; ++q) y.yv[q] = a.yb[(12 + q) * n + e];
-    double gr = mh::dyn_ycontract(G, y, d);
-    mh::dyn_translation_direction<ND>(G, D, a.Kb + e, n, a.one, c, dir_t, d, w0);
-    double gt = mh::dyn_ycontract(G, y, d);
-    if constexpr (DER == 0) {   // the static part, from the y kernel
-        gt = a.g[dir_t * n + e] + gt;
-        gr = a.g[dir_r * n + e] + gr;
-    }
-    a.g[DER * a.gstride + dir_t * n + e] = gt;
-    a.g[DER * a.gstride + dir_r * n + e] = gr;
-    if ((gt != gt) | (gr != gr)) atomicMin(a.flag, a.gtag | (unsigned long long)e);
+    if (nan) atomicMin(a.flag, a.gtag | (unsigned long long)e);
 }
 
 template <int ND, bool UDOF>
@@ -1042,6 +1085,7 @@ struct DirectArgs {
     double t, dt;
     double sX[12], sU[3], sL[12];
     const double* Kc;     // beams: unscaled compact static part (value pass)
+    const double* rec;    // beams: the elements' records (value pass)
     double* Kd;           // Kd[d*nKd + kdbase + e*nX² + i + nX·k]
     int64_t nKd;
     double* KU;           // KU[kubase + e*nX*3 + i + nX·c]
@@ -1051,86 +1095,79 @@ struct DirectArgs {
     unsigned long long gtag;
 };
 
-// Beams, 16 lanes per element: the X₀ pass of lane k gives column k of J_x, J_v (LDS) and
-// of ∂R/∂X₀; lanes then differentiate the loads along X′ₖ and X″ₖ for the other orders;
-// lane 12 forms ∂R/∂U = -Σ dL J_xᵀ.
+// Beams, after the value pass with unit scales: a workgroup per tile of elements and lanes as in
+// the SweepX direction pass. The X₀ pass gives the Jacobian's rows (LDS) and ∂R/∂X₀; then the loads
+// are differentiated along X′ₖ and X″ₖ; ∂R/∂U = −Σ_gp dL J_xᵀ, a lane its two rows.
 template <int ND, bool UDOF>
-__global__ __launch_bounds__(kDirBlock) void beam_direct_kernel(DirectArgs a) {
-    __shared__ double Jsh[kDirElems][12][15];
-    const int64_t e0 = xcd_tile(a.per_xcd) * kDirElems;
+__global__ __launch_bounds__(kDirLanes, 2) void beam_direct_kernel(DirectArgs a) {
+    __shared__ DynElem<ND> lds[kDirTile];
+    __shared__ mh::DirRow rows[kDirTile][6];
+    const int64_t e0 = xcd_tile(a.per_xcd) * kDirTile;
     if (e0 >= a.nele) return;   // whole workgroup leaves together
-    const int el = threadIdx.x / kDirLanes, k = threadIdx.x % kDirLanes;
-    const int64_t e = e0 + el;
+    stage_elements<ND, kDirTile>(a, e0, lds);
     const int64_t n = a.nele;
-    const bool live = e < n && k <= 12;
-    mh::BeamGeo G;
-    const double one[12] = {1., 1., 1., 1., 1., 1., 1., 1., 1., 1., 1., 1.};
-    mh::DynDir d0;
-    // the element's data from memory (again for the higher time orders, rather than held
-    // live across the barrier)
-    auto load = [&](mh::BeamGeo& Gl, mh::BeamDynSection& Dl, double (*Xl)[12], double* Ul) {
-        mh::BeamSection S;
-        BeamDynArgs b;
-        b.nele = a.nele; b.idx = a.idx; b.uidx = a.uidx; b.nodes = a.nodes; b.xyz = a.xyz; b.o2 = a.o2; b.sec = a.sec;
-        for (int d = 0; d < 3; ++d) b.X[d] = a.X[d];
-        b.U = a.U;
-        dyn_load<ND, UDOF>(b, e, Gl, S, Dl, Xl, Ul);
-    };
-    if (live) {
-        mh::BeamDynSection D;
-        double X[ND][12], U[3];
-        load(G, D, X, U);
-        if (k < 12) {
-            const double c0[6] = {0., 0., 0., 0., 0., 0.};
-            mh::dyn_direction<ND>(G, D, X, U, one, c0, k, d0, 1.);
-#pragma unroll
-            for (int g = 0; g < 4; ++g)
-#pragma unroll
-                for (int q = 0; q < 3; ++q) Jsh[el][k][3 * g + q] = d0.Jx[g][q];
-#pragma unroll
-            for (int q = 0; q < 3; ++q) Jsh[el][k][12 + q] = d0.Jv[q];
+    const int m = n - e0 < kDirTile ? (int)(n - e0) : kDirTile, lane = threadIdx.x < 6 * m ? threadIdx.x : 6 * m - 1;
+    const bool live = threadIdx.x < 6 * m;   // the others repeat the last lane and store nothing
+    const int el = lane / 6, j = lane - el * 6;
+    const int64_t e = e0 + el;
+    const mh::DynRec<ND>& R = lds[el].rec;
+    const mh::BeamDynSection& S = lds[el].sec;
+    const double (*V)[6] = lds[el].V;
+    const int nd = j / 3, k = j - 3 * nd, ir = rot_dof(j), it = tr_dof(j);
+    bool nan = false;
+#pragma unroll 1
+    for (int der = 0; der < ND; ++der) {
+        const double sg[3] = {der == 0 ? 1. : 0., der == 1 ? 1. : 0., der == 2 ? 1. : 0.};
+        mh::DirCol cr, ct;
+        mh::v3 r1, r2, t1, t2, s1, s2;
+        {
+            mh::DirRow row;
+            mh::rotation_direction<ND>(S, R, V, nd, k, sg, row, cr);
+            if (der == 0) rows[el][j] = row;
         }
+        mh::translation_rows<ND>(R, cr, r1, r2);
+        MH_PHASE();
+        mh::translation_direction<ND>(S, R, nd, k, sg, ct);
+        mh::translation_rows<ND>(R, ct, t1, t2);
+        __syncthreads();
+        MH_PHASE();
+        double vr[6], vt[6], sv[6];
+#pragma unroll
+        for (int i = 0; i < 6; ++i) {
+            vr[i] = mh::rotation_row(rows[el][i], cr);
+            vt[i] = mh::rotation_row(rows[el][i], ct);
+        }
+        if (der == 0) {
+            const double* kc = a.Kc + e * mh::kCompact;
+            static_rot_col(kc, j, s1, s2, sv);
+            r1 = s1 + r1; r2 = s2 + r2;
+#pragma unroll
+            for (int i = 0; i < 6; ++i) vr[i] = sv[i] + vr[i];
+            static_tr_col(kc, nd, k, s1, s2, sv);
+            t1 = s1 + t1; t2 = s2 + t2;
+#pragma unroll
+            for (int i = 0; i < 6; ++i) vt[i] = sv[i] + vt[i];
+        }
+        const double fr = a.sX[ir], ft = a.sX[it];
+#pragma unroll
+        for (int i = 0; i < 6; ++i) { vr[i] = (vr[i] * fr) * a.dt; vt[i] = (vt[i] * ft) * a.dt; }
+        if (!live) continue;
+        double* K = a.Kd + der * a.nKd + e * 144;
+        nan = store_col(K + 12 * ir, a.dt * (fr * r1), a.dt * (fr * r2), vr) || nan;
+        nan = store_col(K + 12 * it, a.dt * (ft * t1), a.dt * (ft * t2), vt) || nan;
     }
-    __syncthreads();
     if (!live) return;
-    int nan = 0;
-    if (k == 12) {
-        if (UDOF) {
-            double* dst = a.KU + e * 36;
-            for (int c = 0; c < 3; ++c)
-                for (int i = 0; i < 12; ++i) {
-                    double s = 0.;
-                    for (int g = 0; g < 4; ++g) s = s + Jsh[el][i][3 * g + c] * G.dL[g];
-                    dst[i + 12 * c] = ((-s) * a.sU[c]) * a.dt;
-                    nan |= dst[i + 12 * c] != dst[i + 12 * c];
-                }
-        }
-    } else {
-        // column k of the block of each time order; d0 (order 0) is consumed first, so that it is
-        // not live through the directions of the higher orders
-        auto rows = [&](int der, const mh::DynDir& d, const mh::BeamGeo& Gx) {
-            double* dst = a.Kd + der * a.nKd + e * 144 + 12 * k;
-            for (int i = 0; i < 12; ++i) {
-                double v = mh::dyn_row(Gx, (const double(*)[3])(&Jsh[el][i][0]), &Jsh[el][i][12], d);
-                if (der == 0) {
-                    double m;
-                    const int slot = mh::compact_slot(i, k, &m);
-                    v = m * a.Kc[e * mh::kCompact + slot] + v;
-                }
-                dst[i] = (v * a.sX[k]) * a.dt;
-                nan |= dst[i] != dst[i];
-            }
-        };
-        rows(0, d0, G);
-        for (int der = 1; der < ND; ++der) {
-            mh::BeamGeo Gd;
-            mh::BeamDynSection D;
-            double X[ND][12], U[3];
-            load(Gd, D, X, U);
-            mh::DynDir d;
-            const double c[6] = {der == 1 ? 1. : 0., 0., 0., der == 2 ? 1. : 0., 0., 0.};
-            mh::dyn_direction<ND>(Gd, D, X, U, one, c, k, d, 0.);
-            rows(der, d, Gd);
+    if (UDOF) {
+        const mh::v3 ur = mh::row_load<ND>(R, rows[el][j]);
+        const mh::v3 ut = (0.5 * R.L) * mh::mk(k == 0 ? 1. : 0., k == 1 ? 1. : 0., k == 2 ? 1. : 0.);
+        double* dst = a.KU + e * 36;
+        const double cr[3] = {ur.x, ur.y, ur.z}, ct[3] = {ut.x, ut.y, ut.z};
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const double x = ((-cr[c]) * a.sU[c]) * a.dt, y = ((-ct[c]) * a.sU[c]) * a.dt;
+            dst[ir + 12 * c] = x;
+            dst[it + 12 * c] = y;
+            nan = nan || x != x || y != y;
         }
     }
     if (nan) atomicMin(a.flag, a.gtag | (unsigned long long)e);
@@ -1514,12 +1551,12 @@ void launch_dyn(BeamDynArgs& a, bool step, hipStream_t s) {
         a.per_xcd = (ntile + kXCD - 1) / kXCD;
         hipLaunchKernelGGL((beam_dyn_value_kernel<ND, UDOF>), dim3((unsigned)(a.per_xcd * kXCD)), dim3(kBeamBlock), 0, s, a);
     }
-    const int NE = step ? kDirElemsW<true> : kDirElemsW<false>;
-    const int64_t ntile = (a.nele + NE - 1) / NE;
+    const int tile = step ? kStepTile : kDirTile;
+    const int64_t ntile = (a.nele + tile - 1) / tile;
     a.per_xcd = (ntile + kXCD - 1) / kXCD;
     const dim3 gr((unsigned)(a.per_xcd * kXCD));
-    if (step) hipLaunchKernelGGL((beam_dyn_dir_kernel<ND, UDOF, true>), gr, dim3(kDirWBlock), 0, s, a);
-    else hipLaunchKernelGGL((beam_dyn_dir_kernel<ND, UDOF, false>), gr, dim3(kDirWBlock), 0, s, a);
+    if (step) hipLaunchKernelGGL((beam_dyn_dir_kernel<ND, true>), gr, dim3(kDirLanes), 0, s, a);
+    else hipLaunchKernelGGL((beam_dyn_dir_kernel<ND, false>), gr, dim3(kDirLanes), 0, s, a);
 }
 int launch_dyn_beams(Ctx* c, const Group& g, int OX, bool step, const double* c6, unsigned long long gtag) {
     BeamDynArgs a;
@@ -1536,7 +1573,7 @@ int launch_dyn_beams(Ctx* c, const Group& g, int OX, bool step, const double* c6
     for (int i = 0; i < 6; ++i) a.c[i] = c6[i];
     a.dc = c->d_c6;
     a.Kc = c->d_Kc + g.kcbase; a.K = c->d_Kbuf + g.kbase; a.R = c->d_Rbuf + g.rbase;
-    a.Kb = c->d_Kb + g.kcbase / mh::kCompact * mh::kDynBase;
+    a.rec = c->d_rec + g.recbase;
     a.dR = step ? c->d_dRbuf + g.rbase : nullptr;
     a.flag = c->d_flag; a.gtag = gtag;
     const bool u = g.kind == MH_KIND_BEAM_U;
@@ -1601,7 +1638,7 @@ int launch_vjp(Ctx* c, const Group& g, int nd, unsigned long long gtag) {
         for (int i = 0; i < 12; ++i) { b.sR[i] = 1.; b.scale[i] = 1.; }
         for (int i = 0; i < 6; ++i) b.c[i] = 0.;
         b.Kc = c->d_Kc + g.kcbase; b.K = nullptr; b.R = nullptr; b.dR = nullptr;
-        b.Kb = c->d_Kb + g.kcbase / mh::kCompact * mh::kDynBase;
+        b.rec = c->d_rec + g.recbase;
         b.flag = c->d_flag; b.gtag = gtag;
         const int64_t ntile = (g.nele + kBeamBlock - 1) / kBeamBlock;
         b.per_xcd = (ntile + kXCD - 1) / kXCD;
@@ -1614,39 +1651,16 @@ int launch_vjp(Ctx* c, const Group& g, int nd, unsigned long long gtag) {
             else hipLaunchKernelGGL((beam_dyn_value_kernel<3, false>), grv, dim3(kBeamBlock), 0, s, b);
         }
         a.Kc = b.Kc;
-        a.Kb = b.Kb;
-        a.yb = c->d_ybuf + g.kcbase / mh::kCompact * 15;
-        {
-            const dim3 gy((unsigned)((g.nele + kBlock - 1) / kBlock));
-            if (nd == 2) {
-                if (u) hipLaunchKernelGGL((beam_dyn_y_kernel<2, true>), gy, dim3(kBlock), 0, s, a);
-                else hipLaunchKernelGGL((beam_dyn_y_kernel<2, false>), gy, dim3(kBlock), 0, s, a);
-            } else {
-                if (u) hipLaunchKernelGGL((beam_dyn_y_kernel<3, true>), gy, dim3(kBlock), 0, s, a);
-                else hipLaunchKernelGGL((beam_dyn_y_kernel<3, false>), gy, dim3(kBlock), 0, s, a);
-            }
-        }
-        const int64_t nt = (g.nele + kDirElemsW<false> - 1) / kDirElemsW<false>;
+        a.rec = b.rec;
+        const int64_t nt = (g.nele + kDirTile - 1) / kDirTile;
         a.per_xcd = (nt + kXCD - 1) / kXCD;
         const dim3 gr((unsigned)(a.per_xcd * kXCD));
         if (nd == 2) {
-            if (u) {
-                hipLaunchKernelGGL((beam_dyn_vjp_kernel<2, true, 0>), gr, dim3(kDirWBlock), 0, s, a);
-                hipLaunchKernelGGL((beam_dyn_vjp_kernel<2, true, 1>), gr, dim3(kDirWBlock), 0, s, a);
-            } else {
-                hipLaunchKernelGGL((beam_dyn_vjp_kernel<2, false, 0>), gr, dim3(kDirWBlock), 0, s, a);
-                hipLaunchKernelGGL((beam_dyn_vjp_kernel<2, false, 1>), gr, dim3(kDirWBlock), 0, s, a);
-            }
+            if (u) hipLaunchKernelGGL((beam_dyn_vjp_kernel<2, true>), gr, dim3(kDirLanes), 0, s, a);
+            else hipLaunchKernelGGL((beam_dyn_vjp_kernel<2, false>), gr, dim3(kDirLanes), 0, s, a);
         } else {
-            if (u) {
-                hipLaunchKernelGGL((beam_dyn_vjp_kernel<3, true, 0>), gr, dim3(kDirWBlock), 0, s, a);
-                hipLaunchKernelGGL((beam_dyn_vjp_kernel<3, true, 1>), gr, dim3(kDirWBlock), 0, s, a);
-                hipLaunchKernelGGL((beam_dyn_vjp_kernel<3, true, 2>), gr, dim3(kDirWBlock), 0, s, a);
-            } else {
-                hipLaunchKernelGGL((beam_dyn_vjp_kernel<3, false, 0>), gr, dim3(kDirWBlock), 0, s, a);
-                hipLaunchKernelGGL((beam_dyn_vjp_kernel<3, false, 1>), gr, dim3(kDirWBlock), 0, s, a);
-                hipLaunchKernelGGL((beam_dyn_vjp_kernel<3, false, 2>), gr, dim3(kDirWBlock), 0, s, a);
-            }
+            if (u) hipLaunchKernelGGL((beam_dyn_vjp_kernel<3, true>), gr, dim3(kDirLanes), 0, s, a);
+            else hipLaunchKernelGGL((beam_dyn_vjp_kernel<3, false>), gr, dim3(kDirLanes), 0, s, a);
         }
     } else if (bar) {
         const dim3 gr((unsigned)((g.nele + kBarBlock - 1) / kBarBlock));
@@ -1835,10 +1849,10 @@ template <int ND>
 static void launch_direct_beam(bool u, dim3 grv, dim3 gr, hipStream_t s, const BeamDynArgs& b, const DirectArgs& a) {
     if (u) {
         hipLaunchKernelGGL((beam_dyn_value_kernel<ND, true>), grv, dim3(kBeamBlock), 0, s, b);
-        hipLaunchKernelGGL((beam_direct_kernel<ND, true>), gr, dim3(kDirBlock), 0, s, a);
+        hipLaunchKernelGGL((beam_direct_kernel<ND, true>), gr, dim3(kDirLanes), 0, s, a);
     } else {
         hipLaunchKernelGGL((beam_dyn_value_kernel<ND, false>), grv, dim3(kBeamBlock), 0, s, b);
-        hipLaunchKernelGGL((beam_direct_kernel<ND, false>), gr, dim3(kDirBlock), 0, s, a);
+        hipLaunchKernelGGL((beam_direct_kernel<ND, false>), gr, dim3(kDirLanes), 0, s, a);
     }
 }
 
@@ -1873,12 +1887,14 @@ static int launch_direct(Ctx* c, const Group& g, int nd, double dt, unsigned lon
         for (int i = 0; i < 12; ++i) { b.sR[i] = dt; b.scale[i] = 1.; }
         for (int i = 0; i < 6; ++i) b.c[i] = 0.;
         b.Kc = c->d_Kc + g.kcbase; b.K = nullptr; b.R = c->d_Rd + g.rbase; b.dR = nullptr;
+        b.rec = c->d_rec + g.recbase;
         b.flag = c->d_flag; b.gtag = gtag;
         const int64_t ntile = (g.nele + kBeamBlock - 1) / kBeamBlock;
         b.per_xcd = (ntile + kXCD - 1) / kXCD;
         const dim3 grv((unsigned)(b.per_xcd * kXCD));
         a.Kc = b.Kc;
-        const int64_t nt = (g.nele + kDirElems - 1) / kDirElems;
+        a.rec = b.rec;
+        const int64_t nt = (g.nele + kDirTile - 1) / kDirTile;
         a.per_xcd = (nt + kXCD - 1) / kXCD;
         const dim3 gr((unsigned)(a.per_xcd * kXCD));
         if (nd == 1) launch_direct_beam<1>(u, grv, gr, s, b, a);
@@ -2110,7 +2126,7 @@ int mh_prepare_sweepx(mh_ctx* c, int OX, int64_t* nnz_out) {
     free_prepared(c);
     // contribution counts and buffer offsets, in eletype order. Static beams store the
     // compact tangent; dynamic beams (K + a₁C + b₁M is not symmetric) the full block.
-    int64_t nK = 0, nP = 0, nR = 0, nKc = 0, nRU = 0, nRA = 0;
+    int64_t nK = 0, nP = 0, nR = 0, nKc = 0, nRec = 0, nRU = 0, nRA = 0;
     bool coded = false;
     for (auto& g : c->groups) {
         g.ubase = nRU;
@@ -2123,7 +2139,8 @@ int mh_prepare_sweepx(mh_ctx* c, int OX, int64_t* nnz_out) {
         g.kper = g.compact ? mh::kCompact : (int64_t)g.nX * g.nX;
         g.kbase = nK; g.rbase = nR;
         g.kcbase = nKc;
-        if (beam && OX > 0) nKc += g.nele * mh::kCompact;
+        g.recbase = nRec;
+        if (beam && OX > 0) { nKc += g.nele * mh::kCompact; nRec += rec_numbers(g.nele); }
         nK += g.nele * g.kper;
         nP += g.nele * g.nX * g.nX;
         nR += g.nele * g.nX;
@@ -2140,7 +2157,7 @@ int mh_prepare_sweepx(mh_ctx* c, int OX, int64_t* nnz_out) {
     HIPCHK(c, hipMalloc(&c->d_Rbuf, sizeof(double) * std::max<int64_t>(nR, 1)));
     HIPCHK(c, hipMalloc(&c->d_dRbuf, sizeof(double) * std::max<int64_t>(nR, 1)));
     if (nKc) HIPCHK(c, hipMalloc(&c->d_Kc, sizeof(double) * nKc));
-    if (nKc) HIPCHK(c, hipMalloc(&c->d_Kb, sizeof(double) * (nKc / mh::kCompact * mh::kDynBase)));
+    if (nRec) HIPCHK(c, hipMalloc(&c->d_rec, sizeof(double) * nRec));
     HIPCHK(c, hipMalloc(&c->d_rhs, sizeof(double) * std::max<int64_t>(nX, 1)));
     HIPCHK(c, hipMalloc(&c->d_colptr, sizeof(int32_t) * (nX + 1)));
     // ---- matrix pairs
@@ -2576,17 +2593,14 @@ int mh_vjp_lagrangian(mh_ctx* c, int OX, mh_err* err) {
         }
     }
     if (OX > 0 && !c->d_Kc) {
-        int64_t nKc = 0;
+        int64_t nKc = 0, nRec = 0;
         for (auto& g : c->groups)
-            if (g.kind == MH_KIND_BEAM || g.kind == MH_KIND_BEAM_U) { g.kcbase = nKc; nKc += g.nele * mh::kCompact; }
+            if (g.kind == MH_KIND_BEAM || g.kind == MH_KIND_BEAM_U) {
+                g.kcbase = nKc; nKc += g.nele * mh::kCompact;
+                g.recbase = nRec; nRec += rec_numbers(g.nele);
+            }
         if (nKc) HIPCHK(c, hipMalloc(&c->d_Kc, sizeof(double) * nKc));
-        if (nKc && !c->d_Kb) HIPCHK(c, hipMalloc(&c->d_Kb, sizeof(double) * (nKc / mh::kCompact * mh::kDynBase)));
-    }
-    if (OX > 0 && !c->d_ybuf) {
-        int64_t nb = 0;   // beams, in the layout of Kc
-        for (auto& g : c->groups)
-            if (g.kind == MH_KIND_BEAM || g.kind == MH_KIND_BEAM_U) nb = std::max(nb, g.kcbase / mh::kCompact + g.nele);
-        if (nb) HIPCHK(c, hipMalloc(&c->d_ybuf, sizeof(double) * 15 * nb));
+        if (nRec) HIPCHK(c, hipMalloc(&c->d_rec, sizeof(double) * nRec));
     }
     hipLaunchKernelGGL(fill_u64, dim3(1), dim3(1), 0, s, c->d_flag, ~0ull);
     HIPCHK(c, hipEventRecord(c->ev[0], s));
@@ -2776,17 +2790,17 @@ int mh_prepare_direct(mh_ctx* c, int OX, int OU, int IA, int64_t* nnz4) {
     free_prepared(c);
     // A-dofs reach the device only through A-scaled beams: their section follows A (mh_set_A)
     // and their A column comes from mh_beam_dRdA, outside these blocks
-    int64_t nR = 0, nKd = 0, nKU = 0, nKc = 0;
+    int64_t nR = 0, nKd = 0, nKU = 0, nKc = 0, nRec = 0;
     for (auto& g : c->groups) {
         if (g.kind == MH_KIND_ZERO || g.kind == MH_KIND_HOST) {
             c->err = "elements with user functions (DofCost, DofConstraint) are not evaluated on the device in AssemblyDirect";
             return MH_ERR_ARG;
         }
-        g.rbase = nR; g.kdbase = nKd; g.kubase = nKU; g.kcbase = nKc;
+        g.rbase = nR; g.kdbase = nKd; g.kubase = nKU; g.kcbase = nKc; g.recbase = nRec;
         nR += g.nele * g.nX;
         nKd += g.nele * g.nX * g.nX;
         nKU += g.nele * g.nX * g.nU;
-        if (g.kind == MH_KIND_BEAM || g.kind == MH_KIND_BEAM_U) nKc += g.nele * mh::kCompact;
+        if (g.kind == MH_KIND_BEAM || g.kind == MH_KIND_BEAM_U) { nKc += g.nele * mh::kCompact; nRec += rec_numbers(g.nele); }
     }
     if (nR >= (int64_t)UINT32_MAX || nKd >= (int64_t)UINT32_MAX) { c->err = "too many element outputs for 32-bit maps"; return MH_ERR_SIZE; }
     c->nR = nR; c->nKd = nKd; c->nKU = nKU;
@@ -2809,6 +2823,7 @@ int mh_prepare_direct(mh_ctx* c, int OX, int OU, int IA, int64_t* nnz4) {
     HIPCHK(c, hipMalloc(&c->d_Kd, sizeof(double) * std::max<int64_t>((OX + 1) * nKd, 1)));
     HIPCHK(c, hipMalloc(&c->d_KU, sizeof(double) * std::max<int64_t>(nKU, 1)));
     HIPCHK(c, hipMalloc(&c->d_Kc, sizeof(double) * std::max<int64_t>(nKc, 1)));
+    HIPCHK(c, hipMalloc(&c->d_rec, sizeof(double) * std::max<int64_t>(nRec, 1)));
     HIPCHK(c, hipMalloc(&c->d_Rd, sizeof(double) * std::max<int64_t>(nR, 1)));
     HIPCHK(c, hipMalloc(&c->d_L1x, sizeof(double) * std::max<int64_t>(nR, 1)));
     // residual-path elements (beams, bars) add nothing to L1[X] and never write their slots
