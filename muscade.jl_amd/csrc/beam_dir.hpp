@@ -21,90 +21,7 @@
 #pragma once
 #include "beam_dyn.hpp"
 
-// A phase ends: what follows is neither scheduled nor loaded before it. Without phases the compiler
-// reads a whole record into registers at once and spills (564 B a lane of the direction kernel).
-#if defined(__HIP_DEVICE_COMPILE__)
-#define MH_PHASE() do { asm volatile("" ::: "memory"); __builtin_amdgcn_sched_barrier(0); } while (0)
-#else
-#define MH_PHASE() do {} while (0)
-#endif
-
 namespace mh {
-
-// ------------------------------------------------ coefficient functions of t = θ²
-// a = sinθ/θ, b = (1−cosθ)/θ², c = (θ−sinθ)/θ³, each with its first two derivatives in t
-// (a′ = ½(c−b), b′ = (a−2b)/2t, c′ = (b−3c)/2t). Series for t < 1 (last term below 1e-18).
-struct RotFun { double a, b, c, a1, b1, c1, a2, b2, c2; };
-MH_HD RotFun rot_fun(double t) {
-    RotFun f;
-    if (t < 1.) {
-        // 1/(2k+2)!, 1/(2k+3)!
-        const double B[10] = {0.5, 1. / 24., 1. / 720., 1. / 40320., 1. / 3628800., 1. / 479001600., 1. / 87178291200.,
-                              1. / 20922789888000., 1. / 6402373705728000., 1. / 2432902008176640000.};
-        const double C[10] = {1. / 6., 1. / 120., 1. / 5040., 1. / 362880., 1. / 39916800., 1. / 6227020800.,
-                              1. / 1307674368000., 1. / 355687428096000., 1. / 121645100408832000.,
-                              1. / 51090942171709440000.};
-        const double u = -t;
-        double b = 0., b1 = 0., b2 = 0., c = 0., c1 = 0., c2 = 0.;
-#pragma unroll
-        for (int k = 9; k >= 0; --k) {
-            b = b * u + B[k]; c = c * u + C[k];
-            if (k > 0) { b1 = b1 * u - k * B[k]; c1 = c1 * u - k * C[k]; }
-            if (k > 1) { b2 = b2 * u + k * (k - 1) * B[k]; c2 = c2 * u + k * (k - 1) * C[k]; }
-        }
-        f.b = b; f.b1 = b1; f.b2 = b2; f.c = c; f.c1 = c1; f.c2 = c2;
-        f.a = 1. - t * c;
-    } else {
-        const double th = sqrt(t), h = 0.5 / t, sh = sin(0.5 * th);
-        f.a = sin(th) / th;
-        f.b = 2. * sh * sh / t;
-        f.c = (1. - f.a) / t;
-        f.b1 = (f.a - 2. * f.b) * h;
-        f.c1 = (f.b - 3. * f.c) * h;
-        const double a1 = 0.5 * (f.c - f.b);
-        f.b2 = (a1 - 4. * f.b1) * h;
-        f.c2 = (f.b1 - 5. * f.c1) * h;
-    }
-    f.a1 = 0.5 * (f.c - f.b);
-    f.a2 = 0.5 * (f.c1 - f.b1);
-    return f;
-}
-// τ = tan(θ/4)/θ and κ = ½e − ¼τ, e = (1 − (θ/2)cot(θ/2))/θ², with two derivatives in t = θ².
-struct HalfFun { double k, k1, k2, q, q1, q2; };   // τ, τ′, τ″, κ, κ′, κ″
-MH_HD HalfFun half_fun(double t) {
-    HalfFun f;
-    double e, e1, e2;
-    if (t < 1.) {
-        // tan(x)/(4x) in x² = t/16, and (1 − x cot x)/(4x²) in x² = t/4
-        const double T[10] = {1., 1. / 3., 2. / 15., 17. / 315., 62. / 2835., 1382. / 155925., 21844. / 6081075.,
-                              929569. / 638512875., 6404582. / 10854718875., 443861162. / 1856156927625.};
-        const double Q[10] = {1. / 3., 1. / 45., 2. / 945., 1. / 4725., 2. / 93555., 1382. / 638512875., 4. / 18243225.,
-                              3617. / 162820783125., 87734. / 38979295480125., 349222. / 1531329465290625.};
-        const double u = t / 16., w = t / 4.;
-        double a = 0., a1 = 0., a2 = 0., b = 0., b1 = 0., b2 = 0.;
-#pragma unroll
-        for (int k = 9; k >= 0; --k) {
-            a = a * u + T[k]; b = b * w + Q[k];
-            if (k > 0) { a1 = a1 * u + k * T[k]; b1 = b1 * w + k * Q[k]; }
-            if (k > 1) { a2 = a2 * u + k * (k - 1) * T[k]; b2 = b2 * w + k * (k - 1) * Q[k]; }
-        }
-        f.k = 0.25 * a; f.k1 = a1 / 64.; f.k2 = a2 / 1024.;
-        e = 0.25 * b; e1 = b1 / 16.; e2 = b2 / 64.;
-    } else {
-        const double th = sqrt(t), h = 0.5 / t;
-        f.k = tan(0.25 * th) / th;
-        f.k1 = (0.25 - f.k + 0.25 * f.k * f.k * t) * h;
-        f.k2 = (-3. * f.k1 + 0.5 * f.k * f.k1 * t + 0.25 * f.k * f.k) * h;
-        const double x = 0.5 * th, C = x / tan(x);
-        const double C1 = (C - C * C - 0.25 * t) * h;
-        const double C2 = (C1 - 2. * C * C1 - 0.25) * h - C1 / t;
-        e = (1. - C) / t;
-        e1 = (-C1 - e) / t;
-        e2 = (-C2 - 2. * e1) / t;
-    }
-    f.q = 0.5 * e - 0.25 * f.k; f.q1 = 0.5 * e1 - 0.25 * f.k1; f.q2 = 0.5 * e2 - 0.25 * f.k2;
-    return f;
-}
 
 // Time jets of vectors, level by level.
 template <int ND> struct TV { v3 v[ND]; };
@@ -146,8 +63,17 @@ template <int ND> MH_HD void tnorm2(const TV<ND>& v, double* t) {
 struct LostSquare { double c, g, c1, c2, g1, g2; };
 MH_HD LostSquare lost_square(v3 v, v3 vd, const RotFun& f) {   // f at |v|²
     const double t = dot(v, v), s = dot(v, vd), C = 1. - f.b * t, g = t * f.a;
-    const RotFun h = rot_fun(0.25 * t);
-    const double sd = (0.5 * h.a1) * s, q = sd * sd, qt = (0.25 * h.a2) * (sd * s), qs = h.a1 * sd;
+    double f0, f1;   // derivatives of sinc1(|v|/2) in t; b is half its square
+    if (t < 1.) {
+        const double i = 1. / sqrt(2. * f.b);
+        f0 = f.b1 * i;
+        f1 = (f.b2 - f0 * f0) * i;
+    } else {
+        const RotFun h = rot_fun(0.25 * t);
+        f0 = 0.25 * h.a1;
+        f1 = 0.0625 * h.a2;
+    }
+    const double sd = (2. * f0) * s, q = sd * sd, qt = (4. * f1) * (sd * s), qs = (4. * f0) * sd;
     LostSquare o;
     o.c = q * C; o.c1 = 2. * (qt * C) - q * f.a; o.c2 = qs * C;
     o.g = q * g; o.g1 = 2. * (qt * g) + q * (f.a + C); o.g2 = qs * g;
@@ -176,15 +102,16 @@ struct RuleRec {
     double A, B, k1, k2, k3, k, b, c;   // b, c of T(v)
     v3 y, x, u;          // ∂F/∂|v|², x, ∂(½T(v)F)/∂|v|² at fixed F
 };
-MH_HD void rule_record(const m3& rm, const v3* a, const v3* ad, const RotFun* fn, v3 v, v3 vd, RuleRec& o) {
+MH_HD void rule_record(const m3& rm, const v3* a, const v3* ad, const RotFun* fn, const RotFun& f, v3 v, v3 vd, RuleRec& o) {
     const double th = dot(v, v);
-    const RotFun f = rot_fun(th), p = rot_fun(4. * th);
 #pragma unroll
     for (int n = 0; n < 2; ++n) o.sq[n] = lost_square(a[n], ad[n], fn[n]);
     o.rm = rm;
     o.sq[2] = lost_square(v, vd, f);
-    const double S = f.a, S1 = f.a1, C = 1. - f.b * th, C1 = -0.5 * S, ip = 1. / p.a;
-    const double s = -2. * p.a1 * ip, s1 = -8. * (p.a2 - p.a1 * p.a1 * ip) * ip;
+    // p = a(4|v|²) = SC and its derivatives in |v|²
+    const double S = f.a, S1 = f.a1, C = 1. - f.b * th, C1 = -0.5 * S, ip = 1. / (S * C);
+    const double pd = S1 * C + S * C1, pdd = f.a2 * C + 2. * S1 * C1 - 0.5 * S * S1;
+    const double s = -0.5 * pd * ip, s1 = -0.5 * (pdd - pd * pd * ip) * ip;
     o.A = 1. / S; o.B = 1. / C; o.b = f.b; o.c = f.c;
     const double A1 = -S1 * o.A * o.A, B1 = -C1 * o.B * o.B;
     o.k1 = 2. * s * C * o.A - 1.;
@@ -329,83 +256,86 @@ MH_HD GpShape gp_shape(int g, double L) {
     return s;
 }
 
-// The record of an element, number q handed to put(q, value), and the loads the closed form of the
-// static part holds fixed: eg[gp] = dL_gp·fₑ, mtot = Σ_gp dL_gp·mₑ. X: ND rows of the 12 dofs.
+// The record of an element, number q handed to put(q, value), and the loads that the closed form of
+// the static part takes (beam_tangent<true>), from its frame. X: ND rows of the 12 dofs. The spin Ω and
+// vₗ's time derivatives are those of the header along the nodes' velocities, and their derivatives.
 template <int ND, class Put>
-MH_HD void dyn_record(const BeamGeo& G, const BeamDynSection& S, const double (*X)[12], const double* U, Put put, v3* eg,
-                      v3& mtot) {
+MH_HD void dyn_record(const BeamGeo& G, const BeamDynSection& S, const double (*X)[12], const double* U,
+                      const BeamFrame& f, Put put, BeamLoads& ld) {
     int q = 0;
     auto put3 = [&](v3 a) { put(q, a.x); put(q + 1, a.y); put(q + 2, a.z); q += 3; };
     const double L = G.L;
-    JM3<ND, false> rsm;
-    JV3<ND, false> dv, v1, v2;
-#pragma unroll
-    for (int c = 0; c < 3; ++c)
-#pragma unroll
-        for (int n = 0; n < ND; ++n) {
-            v1.a[c].v[n] = X[n][3 + c]; v2.a[c].v[n] = X[n][9 + c];
-            v1.a[c].e[0] = 0.; v2.a[c].e[0] = 0.;
-        }
-    dyn_rotation_chain<ND, false, true>(G, v1, v2, rsm, dv);
-    auto col = [&](int j, int n) { return mk(rsm.a[3 * j].v[n], rsm.a[3 * j + 1].v[n], rsm.a[3 * j + 2].v[n]); };
-    const v3 c0 = col(0, 0), c1 = col(1, 0), c2 = col(2, 0);
+    const v3 c0 = col(f.r, 0), c1 = col(f.r, 1), c2 = col(f.r, 2), zero = mk(0., 0., 0.);
     put3(c0); put3(c1); put3(c2);
     auto body = [&](v3 a) { return mk(dot(c0, a), dot(c1, a), dot(c2, a)); };
-    auto skew = [&](int n) {   // of r₀ᵀ·(n-th time derivative of r)
-        const v3 d0 = col(0, n), d1 = col(1, n), d2 = col(2, n);
-        return mk(0.5 * (dot(c2, d1) - dot(c1, d2)), 0.5 * (dot(c0, d2) - dot(c2, d0)), 0.5 * (dot(c1, d0) - dot(c0, d1)));
-    };
-    const v3 om = ND > 1 ? skew(ND > 1 ? 1 : 0) : mk(0., 0., 0.), omd = ND > 2 ? skew(ND > 2 ? 2 : 0) : mk(0., 0., 0.);
-    put3(om); put3(omd);
-    // body components of jets: (rᵀa)′ = rᵀa′ − Ω×(rᵀa), …
-    auto tobody = [&](const v3* g) {
-        TV<ND> t;
-        t.v[0] = body(g[0]);
-        if constexpr (ND > 1) {
-            const v3 a1 = body(g[1]);
-            t.v[1] = a1 - cross(om, t.v[0]);
-            if constexpr (ND > 2) t.v[2] = body(g[2]) - cross(omd, t.v[0]) - cross(om, t.v[1]) - cross(om, a1);
+    TV<ND> vn[2];
+    double tn[2][3], th[3];
+    const RotFun fn[2] = {f.f1, f.f2};
+#pragma unroll
+    for (int n = 0; n < ND; ++n) { vn[0].v[n] = mk(X[n][3], X[n][4], X[n][5]); vn[1].v[n] = mk(X[n][9], X[n][10], X[n][11]); }
+    tnorm2(vn[0], tn[0]);
+    tnorm2(vn[1], tn[1]);
+    const HalfFun hf = half_fun(f.fh);
+    v3 om = zero, omd = zero;
+    TV<ND> vl;
+    vl.v[0] = f.vl;
+    if constexpr (ND > 1) {
+        v3 t[2], td[2];   // rᵀT(v_n)v̇_n and rᵀ times its derivative
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const v3 v = vn[i].v[0], w = vn[i].v[1], y = cross(v, w), z = cross(v, y);
+            t[i] = body(w + fn[i].b * y + fn[i].c * z);
+            if constexpr (ND > 2) {
+                const v3 a = vn[i].v[2], yd = cross(v, a), zd = cross(w, y) + cross(v, yd);
+                td[i] = body(a + (fn[i].b1 * tn[i][1]) * y + fn[i].b * yd + (fn[i].c1 * tn[i][1]) * z + fn[i].c * zd);
+            }
         }
-        return t;
-    };
-    v3 g[ND], cs[ND];
+        const v3 dl = t[1] - t[0], y = cross(f.vl, dl), z = cross(f.vl, y);
+        om = 0.5 * (t[0] + t[1]) - hf.k * y;
+        vl.v[1] = 0.5 * dl + (4. * hf.q) * z;
+        if constexpr (ND > 2) {
+            const v3 t1 = td[0] - cross(om, t[0]), t2 = td[1] - cross(om, t[1]), dd = t2 - t1;
+            const v3 yd = cross(vl.v[1], dl) + cross(f.vl, dd), zd = cross(vl.v[1], y) + cross(f.vl, yd);
+            const double s = 8. * dot(f.vl, vl.v[1]);
+            omd = 0.5 * (t1 + t2) - (hf.k1 * s) * y - hf.k * yd;
+            vl.v[2] = 0.5 * dd + 4. * ((hf.q1 * s) * z + hf.q * zd);
+        }
+    }
+    put3(om); put3(omd);
+    // d in body components: (rᵀa)′ = rᵀa′ − Ω×(rᵀa), …
+    TV<ND> d;
+    v3 cs[ND];
+    d.v[0] = f.d;
 #pragma unroll
     for (int n = 0; n < ND; ++n) {
         const v3 u1 = mk(X[n][0], X[n][1], X[n][2]), u2 = mk(X[n][6], X[n][7], X[n][8]);
         cs[n] = 0.5 * (u1 + u2);
-        g[n] = n == 0 ? (u2 + 0.5 * G.tgm) - cs[n] : u2 - cs[n];
+        if (n == 1) d.v[n] = body(u2 - cs[n]) - cross(om, d.v[0]);
+        if (n == 2) {
+            const v3 a1 = d.v[n - 1] + cross(om, d.v[0]);
+            d.v[n] = body(u2 - cs[n]) - cross(omd, d.v[0]) - cross(om, d.v[n - 1]) - cross(om, a1);
+        }
     }
-    const TV<ND> d = tobody(g);
 #pragma unroll
-    for (int n = 0; n < ND; ++n) { put3(d.v[n]); g[n] = mk(dv.a[0].v[n], dv.a[1].v[n], dv.a[2].v[n]); }
-    const TV<ND> vl = tobody(g);
+    for (int n = 0; n < ND; ++n) put3(d.v[n]);
 #pragma unroll
     for (int n = 0; n < ND; ++n) put3(vl.v[n]);
-    double t[3], k[ND];
+    double k[ND];
     auto putn = [&]() {
 #pragma unroll
         for (int n = 0; n < ND; ++n) put(q + n, k[n]);
         q += ND;
     };
-    TV<ND> vn[2];
-    RotFun fn[2];
-#pragma unroll
-    for (int n = 0; n < ND; ++n) { vn[0].v[n] = mk(X[n][3], X[n][4], X[n][5]); vn[1].v[n] = mk(X[n][9], X[n][10], X[n][11]); }
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-        tnorm2(vn[i], t);
-        fn[i] = rot_fun(t[0]);
-        tcompose<ND>(fn[i].b, fn[i].b1, fn[i].b2, t, k); putn();
-        tcompose<ND>(fn[i].c, fn[i].c1, fn[i].c2, t, k); putn();
+        tcompose<ND>(fn[i].b, fn[i].b1, fn[i].b2, tn[i], k); putn();
+        tcompose<ND>(fn[i].c, fn[i].c1, fn[i].c2, tn[i], k); putn();
     }
-    {
-        tnorm2(vl, t);
+    tnorm2(vl, th);
 #pragma unroll
-        for (int n = 0; n < ND; ++n) t[n] *= 4.;
-        const HalfFun f = half_fun(t[0]);
-        tcompose<ND>(f.k, f.k1, f.k2, t, k); putn();
-        tcompose<ND>(f.q, f.q1, f.q2, t, k); putn();
-    }
+    for (int n = 0; n < ND; ++n) th[n] *= 4.;
+    tcompose<ND>(hf.k, hf.k1, hf.k2, th, k); putn();
+    tcompose<ND>(hf.q, hf.q1, hf.q2, th, k); putn();
     // the power rule
     v3 ddl = mk(0., 0., 0.), dvl = ddl;   // what it takes off d″, vₗ″
     m3 Q2;
@@ -414,7 +344,7 @@ MH_HD void dyn_record(const BeamGeo& G, const BeamDynSection& S, const double (*
         auto ref = [&](v3 a) { return mulT(G.rm, a); };
         const v3 a[2] = {ref(vn[0].v[0]), ref(vn[1].v[0])}, ad[2] = {ref(vn[0].v[1]), ref(vn[1].v[1])};
         RuleRec ru;
-        rule_record(G.rm, a, ad, fn, vl.v[0], vl.v[1], ru);
+        rule_record(G.rm, a, ad, fn, f.fh, vl.v[0], vl.v[1], ru);
         const double* p = reinterpret_cast<const double*>(&ru);
 #pragma unroll
         for (int i = 0; i < 56; ++i) put(kRecBase<ND> + i, p[i]);
@@ -424,6 +354,7 @@ MH_HD void dyn_record(const BeamGeo& G, const BeamDynSection& S, const double (*
         gx = 0.5 * (ru.gam.a[5] - ru.gam.a[7]);
     }
     // loads at the Gauss points, body frame
+    ld.e0 = ld.ea = ld.eu = ld.ev = mk(0., 0., 0.);
 #pragma unroll
     for (int gp = 0; gp < 4; ++gp) {
         const GpShape h = gp_shape(gp, L);
@@ -440,17 +371,15 @@ MH_HD void dyn_record(const BeamGeo& G, const BeamDynSection& S, const double (*
         put(q + 12 + 3 * gp, xdd.x); put(q + 13 + 3 * gp, xdd.y); put(q + 14 + 3 * gp, xdd.z);
         auto bl = [&](int j, double x1, double x2) { return S.mu * x2 + (S.Ca[j] * x2 + S.Cl[j] * x1 + S.Cq[j] * (x1 * fabs(x1))); };
         const double f0 = bl(0, xd.x, xdd.x), f1 = bl(1, xd.y, xdd.y), f2 = bl(2, xd.z, xdd.z);
-        eg[gp] = h.w * (f0 * c0 + f1 * c1 + f2 * c2 + mk(-U[0], -U[1], S.w - U[2]));
+        const v3 e = h.w * (f0 * c0 + f1 * c1 + f2 * c2 + mk(-U[0], -U[1], S.w - U[2]));
+        ld.e0 = ld.e0 + e; ld.ea = ld.ea + h.ya * e; ld.eu = ld.eu + h.yu * e; ld.ev = ld.ev + h.yv * e;
     }
     q += 24;
     const double m1 = ND > 2 ? S.iota1 * (omd.x - gx) : 0.;
     put(q++, m1);
-    mtot = (m1 * L) * c0;
+    ld.m = (m1 * L) * c0;
     {
-        m3 rr;
-        rr.a[0] = c0.x; rr.a[1] = c0.y; rr.a[2] = c0.z; rr.a[3] = c1.x; rr.a[4] = c1.y; rr.a[5] = c1.z;
-        rr.a[6] = c2.x; rr.a[7] = c2.y; rr.a[8] = c2.z;
-        const v3 psi = rotvec(rr);
+        const v3 psi = rotvec(f.r);
         put3(psi);
         put(q++, exp_coef(norm3(psi)).e);
     }

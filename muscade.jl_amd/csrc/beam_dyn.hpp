@@ -38,7 +38,6 @@ template <int NT, bool E> MH_HD Jet<NT, E> jzero() {
     for (int n = 0; n < (E ? NT : 1); ++n) r.e[n] = 0.;
     return r;
 }
-template <int NT, bool E> MH_HD Jet<NT, E> jconst(double c) { Jet<NT, E> r = jzero<NT, E>(); r.v[0] = c; return r; }
 template <int NT, bool E> MH_HD Jet<NT, E> operator+(const Jet<NT, E>& a, const Jet<NT, E>& b) {
     Jet<NT, E> r;
 #pragma unroll
@@ -232,33 +231,6 @@ template <int NT, bool E, bool XSQ = false> MH_HD JM3<NT, E> jrodrigues(const JV
     for (int i = 0; i < 3; ++i) { r.a[i] = c0.a[i]; r.a[3 + i] = c1.a[i]; r.a[6 + i] = c2.a[i]; }
     return r;
 }
-// Rodrigues⁻¹(m) = spin⁻¹(m)/scac((tr m - 1)/2) (Rotations.jl:101)
-template <int NT, bool E> MH_HD JV3<NT, E> jrodrigues_inv(const JM3<NT, E>& m) {
-    using J = Jet<NT, E>;
-    J tr = (m.a[0] + m.a[4]) + m.a[8];
-    J rs = jrecip(jscac(0.5 * (tr + (-1.))));
-    JV3<NT, E> r;
-    r.a[0] = (0.5 * (m.a[5] - m.a[7])) * rs;
-    r.a[1] = (0.5 * (m.a[6] - m.a[2])) * rs;
-    r.a[2] = (0.5 * (m.a[1] - m.a[3])) * rs;
-    return r;
-}
-template <int NT, bool E> MH_HD JM3<NT, E> jmul(const JM3<NT, E>& A, const JM3<NT, E>& B) {
-    JM3<NT, E> r;
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-        for (int j = 0; j < 3; ++j) r.a[i + 3 * j] = (A.a[i] * B.a[3 * j] + A.a[i + 3] * B.a[1 + 3 * j]) + A.a[i + 6] * B.a[2 + 3 * j];
-    return r;
-}
-template <int NT, bool E> MH_HD JM3<NT, E> jmulABt(const JM3<NT, E>& A, const JM3<NT, E>& B) {
-    JM3<NT, E> r;
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-        for (int j = 0; j < 3; ++j) r.a[i + 3 * j] = (A.a[i] * B.a[j] + A.a[i + 3] * B.a[j + 3]) + A.a[i + 6] * B.a[j + 6];
-    return r;
-}
 // A ∘₁ B with a constant B
 template <int NT, bool E> MH_HD JM3<NT, E> jmul_const(const JM3<NT, E>& A, const m3& B) {
     JM3<NT, E> r;
@@ -346,18 +318,8 @@ MH_HD void dyn_rotation_chain(const BeamGeo& G, const JV3<NT, E>& v1, const JV3<
         rsm.a[3 * j + 2] = (w[2] + ah * cz) + bh * (z * s - n2 * w[2]);
     }
 }
-// A time jet with no ε part as one whose ε part is zero.
-template <int NT, bool E> MH_HD Jet<NT, E> jlift(const Jet<NT, false>& a) {
-    Jet<NT, E> r = jzero<NT, E>();
-#pragma unroll
-    for (int n = 0; n < NT; ++n) r.v[n] = a.v[n];
-    return r;
-}
-
 // Kinematics (BeamElement.jl:176-208) on time jets. Xj: the 12 element dofs as jets.
-// ROTE = false: the ε seed is on a translation dof, so the rotation chain carries no ε part
-// and is evaluated on plain time jets (about half the work of a direction).
-template <int NT, bool E, bool ROTE = true, bool XSQ = false>
+template <int NT, bool E, bool XSQ = false>
 MH_HD void dyn_kinematics(const BeamGeo& G, const Jet<NT, E>* Xj, DynKin<E>& k) {
     using J = Jet<NT, E>;
     const double L = G.L;
@@ -366,27 +328,10 @@ MH_HD void dyn_kinematics(const BeamGeo& G, const Jet<NT, E>* Xj, DynKin<E>& k) 
     for (int c = 0; c < 3; ++c) { u1.a[c] = Xj[c]; u2.a[c] = Xj[6 + c]; }
     JM3<NT, E> rsm;
     JV3<NT, E> dv;
-    if constexpr (ROTE || !E) {
-        JV3<NT, E> v1, v2;
+    JV3<NT, E> v1, v2;
 #pragma unroll
-        for (int c = 0; c < 3; ++c) { v1.a[c] = Xj[3 + c]; v2.a[c] = Xj[9 + c]; }
-        dyn_rotation_chain<NT, E, XSQ>(G, v1, v2, rsm, dv);
-    } else {
-        JV3<NT, false> w1, w2;
-#pragma unroll
-        for (int c = 0; c < 3; ++c)
-#pragma unroll
-            for (int n = 0; n < NT; ++n) { w1.a[c].v[n] = Xj[3 + c].v[n]; w2.a[c].v[n] = Xj[9 + c].v[n]; }
-#pragma unroll
-        for (int c = 0; c < 3; ++c) { w1.a[c].e[0] = 0.; w2.a[c].e[0] = 0.; }
-        JM3<NT, false> rf;
-        JV3<NT, false> df;
-        dyn_rotation_chain<NT, false, XSQ>(G, w1, w2, rf, df);
-#pragma unroll
-        for (int i = 0; i < 9; ++i) rsm.a[i] = jlift<NT, E>(rf.a[i]);
-#pragma unroll
-        for (int c = 0; c < 3; ++c) dv.a[c] = jlift<NT, E>(df.a[c]);
-    }
+    for (int c = 0; c < 3; ++c) { v1.a[c] = Xj[3 + c]; v2.a[c] = Xj[9 + c]; }
+    dyn_rotation_chain<NT, E, XSQ>(G, v1, v2, rsm, dv);
     // uₗ₂ = rₛₘᵀ(u₂ + tgₘ/2 - cₛ) - tgₑ/2,  vₗ₂ = rₛₘᵀ Δv
     JV3<NT, E> dd, cs;
     const double tg[3] = {G.tgm.x, G.tgm.y, G.tgm.z};
@@ -465,15 +410,6 @@ template <bool E> MH_HD void dyn_loads(const DynKin<E>& k, const BeamDynSection&
     for (int i = 0; i < 3; ++i) me[i] = r0[i] * m1;
 }
 
-// Left-Jacobian inverse direction of the rotation vector of rₛₘ: ∂vₛₘ/∂ε with
-// vₛₘ = Rodrigues⁻¹(rₛₘ) (BeamElement.jl:203).
-MH_HD v3 dyn_vsm_e(const Jet<1, true>* r0) {
-    JM3<1, true> m;
-#pragma unroll
-    for (int i = 0; i < 9; ++i) m.a[i] = r0[i];
-    JV3<1, true> v = jrodrigues_inv(m);
-    return mk(v.a[0].e[0], v.a[1].e[0], v.a[2].e[0]);
-}
 // Rotation vector of a rotation matrix (value only).
 MH_HD v3 rotvec(const m3& r) {
     double sc = scac((at(r, 0, 0) + at(r, 1, 1) + at(r, 2, 2) - 1.) / 2.);
@@ -557,7 +493,7 @@ template <int ND> MH_HD void dyn_requestables(const BeamGeo& G, const BeamSectio
         for (int c = 0; c < 3; ++c) out[q++] = km[c].v[d];
     // loads (values) from the time jets of the Gauss points
     DynKin<false> k;
-    dyn_kinematics<ND, false, true, true>(G, Xj, k);
+    dyn_kinematics<ND, false, true>(G, Xj, k);
     Jet<1, false> fe[4][3], me[3];
     const double U0[3] = {0., 0., 0.};
     dyn_loads<false>(k, D, U0, fe, me);
@@ -625,27 +561,6 @@ MH_HD void gauge_jets(const BeamGeo& G, const double* X0, int i, int j, Jet<2, t
     q[1] = (2. / L) * vl.a[0];
     q[2] = (2. / L) * vl.a[2];
     q[3] = (2. / L) * (-vl.a[1]);
-}
-
-// ---- adjoint (vector-Jacobian products) of the residual ------------------------
-// For L = Λ·R the load part of ∂L/∂X⁽ᵈ⁾ₖ is Σ_gp dL (y_gp·∂fₑ/∂X⁽ᵈ⁾ₖ + y_v·∂mₑ/∂X⁽ᵈ⁾ₖ) with
-// y_gp = J_x,gp Λ and y_v = J_v Λ, the derivatives of x_gp and vₛₘ along Λ.
-struct DynY { double y[4][3]; double yv[3]; };
-MH_HD void dyn_y(const BeamGeo& G, const double (*X)[12], const double* lam, DynY& o) {
-    Jet<1, true> Xj[12];
-    dyn_seed<1, true>(X, nullptr, nullptr, 13, Xj, 0., lam);
-    DynKin<true> k;
-    dyn_kinematics<1, true>(G, Xj, k);
-    for (int g = 0; g < 4; ++g)
-        for (int q = 0; q < 3; ++q) o.y[g][q] = k.xe[g][q];
-    v3 jv = dyn_vsm_e(k.r0);
-    o.yv[0] = jv.x; o.yv[1] = jv.y; o.yv[2] = jv.z;
-}
-// ∂L/∂U (U-dofs: fₑ - U, per length): -Σ_gp dL y_gp
-MH_HD v3 dyn_vjp_u(const BeamGeo& G, const DynY& y) {
-    v3 s = mk(0., 0., 0.);
-    for (int g = 0; g < 4; ++g) s = s + G.dL[g] * mk(y.y[g][0], y.y[g][1], y.y[g][2]);
-    return mk(-s.x, -s.y, -s.z);
 }
 
 }  // namespace mh

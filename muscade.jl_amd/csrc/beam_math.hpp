@@ -8,20 +8,23 @@
 //
 //   * the static residual is the gradient of Π(X) = Σ_gp dL·(½EA ε² +
 //     ½ mᵢ·κ + fₑ·x) (fₑ constant in the static case), so K is its Hessian;
-//   * Π depends on the 12 element dofs through the rotation core
-//     (v₁,v₂) ↦ (rₛₘ, Δv) and through the translations (d, cₛₘ);
-//   * first derivatives of the rotation core use spatial spins
-//     (δQ Qᵀ = spin(ω δp)); second derivatives use the symmetric second-order
-//     spin W (δ²Q Qᵀ = spin(W) + ½{spin ω_a, spin ω_b}) with composition
-//     rules for Exp, Log, products and transposes. The second-order part is
-//     never stored: it is contracted with adjoint vectors in a reverse sweep
-//     and accumulated into the 6×6 rotation block of K.
+//   * Π depends on the 12 element dofs through the corotated frame rₛₘ and the
+//     translations and rotations seen from it (BeamSpin): first and second
+//     derivatives along node spins are taken in the frame's own axes.
 //
 // Everything is `__host__ __device__` so the same code can be exercised on the
 // host in unit harnesses; the product path runs it on the GPU only.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <cmath>
+
+// A phase ends: what follows is neither scheduled nor loaded before it. Without phases the compiler
+// reads a whole record into registers at once and spills (564 B a lane of the direction kernel).
+#if defined(__HIP_DEVICE_COMPILE__)
+#define MH_PHASE() do { asm volatile("" ::: "memory"); __builtin_amdgcn_sched_barrier(0); } while (0)
+#else
+#define MH_PHASE() do {} while (0)
+#endif
 
 namespace mh {
 
@@ -139,22 +142,6 @@ MH_HD m3 rodrigues(v3 v, const ExpCoef& k) {
     at(r, 2, 2) = 1. + k.b * (a2 + b2);
     return r;
 }
-// Left Jacobian T(v) = I + b S + c S²: δRod(v) = spin(T δv) Rod(v)
-MH_HD m3 tangent_op(v3 v, const ExpCoef& k) {
-    m3 r;
-    double x = v.x, y = v.y, z = v.z;
-    double xx = x * x, yy = y * y, zz = z * z;
-    at(r, 0, 0) = 1. - k.c * (yy + zz);
-    at(r, 1, 1) = 1. - k.c * (xx + zz);
-    at(r, 2, 2) = 1. - k.c * (xx + yy);
-    at(r, 0, 1) = -k.b * z + k.c * x * y;
-    at(r, 1, 0) = k.b * z + k.c * x * y;
-    at(r, 0, 2) = k.b * y + k.c * x * z;
-    at(r, 2, 0) = -k.b * y + k.c * x * z;
-    at(r, 1, 2) = -k.b * x + k.c * y * z;
-    at(r, 2, 1) = k.b * x + k.c * y * z;
-    return r;
-}
 // T(v)⁻¹ = I - ½ S + e S²
 MH_HD m3 tangent_inv(v3 v, const ExpCoef& k) {
     m3 r;
@@ -265,243 +252,392 @@ MH_HD int compact_slot(int i, int j, double* mult) {
 struct BeamSection { double EA, EI2, EI3, GJ, w; };
 struct BeamOut { double R[12]; double Kc[kCompact]; int nan; };
 
-// Residual and compact tangent of Π = Π_int + Σ_gp e_gp·x_gp + m·vₛₘ with the loads
-// e_gp and the couple m held fixed.
-//   GEN = false: e_gp = dL_gp·fe with fe = (0,0,w) - U, m = 0 (the static element);
-//   GEN = true:  e_gp = eg[gp] (already × dL_gp) and m = mtot = Σ_gp dL_gp·mₑ, the
-//                frozen external loads of the dynamic element (inertia, added mass,
-//                damping, roll inertia). vₛₘ = Rodrigues⁻¹(rₛₘ) (BeamElement.jl:203).
-template <bool GEN = false>
-MH_HD void beam_static(const BeamGeo& G, const BeamSection& S, v3 fe, const double* X, BeamOut& out,
-                       const v3* eg = nullptr, v3 mtot = v3{0., 0., 0.}, double* hms = nullptr, int hst = 0) {
-    const double L = G.L;
-    v3 u1 = mk(X[0], X[1], X[2]), v1 = mk(X[3], X[4], X[5]);
-    v3 u2 = mk(X[6], X[7], X[8]), v2 = mk(X[9], X[10], X[11]);
-    // ---- rotation core, values --------------------------------------------------
-    ExpCoef k1 = exp_coef(norm3(v1)), k2 = exp_coef(norm3(v2));
-    m3 M, H, rsm;
-    v3 phi, dv;
-    ExpCoef kp, kh;
-    {
-        m3 R1 = rodrigues(v1, k1), R2 = rodrigues(v2, k2);
-        M = mulABt(R2, R1);
-        // φ = Rodrigues⁻¹(M) = spin⁻¹(M)/scac((tr M - 1)/2), Δv = φ/2
-        double sc = scac((at(M, 0, 0) + at(M, 1, 1) + at(M, 2, 2) - 1.) / 2.);
-        phi = mk((at(M, 2, 1) - at(M, 1, 2)) / 2. / sc, (at(M, 0, 2) - at(M, 2, 0)) / 2. / sc,
-                 (at(M, 1, 0) - at(M, 0, 1)) / 2. / sc);
-        dv = 0.5 * phi;
-        kp = exp_coef(norm3(phi));
-        kh = exp_coef(norm3(dv));
-        H = rodrigues(dv, kh);
-        rsm = mul(mul(H, R1), G.rm);
-    }
-    // ---- local deformations and the local gradient ---------------------------------
-    v3 cs = mk(0.5 * (u1.x + u2.x), 0.5 * (u1.y + u2.y), 0.5 * (u1.z + u2.z));
-    v3 d = mk(u2.x + G.tgm.x * 0.5 - cs.x, u2.y + G.tgm.y * 0.5 - cs.y, u2.z + G.tgm.z * 0.5 - cs.z);
-    v3 ul = mulT(rsm, d);
-    ul.x = ul.x - L * 0.5;
-    v3 vl = mulT(rsm, dv);
-    v3 w = mk(ul.x + L / 2., ul.y, ul.z);
-    double ell = sqrt(w.x * w.x + w.y * w.y + w.z * w.z);
-    double eps = ell * 2. / L - 1.;
-    double Lsum = ((G.dL[0] + G.dL[1]) + G.dL[2]) + G.dL[3];
-    double fq[6] = {0, 0, 0, 0, 0, 0};
-    // D_q = ∂²Π_int/∂q² (q = (ul, vl)): dense uu block, u₂v₃ and u₃v₂ couplings, diagonal vv
-    s3 Duu;
-    double D15 = 0., D24 = 0., D33 = 0., D44 = 0., D55 = 0.;
-    {
-        double de = 2. / L / ell;
-        double fa = S.EA * Lsum * eps;
-        fq[0] += fa * de * w.x; fq[1] += fa * de * w.y; fq[2] += fa * de * w.z;
-        double c1 = S.EA * Lsum * de * de, c2 = fa * de, il2 = 1. / (ell * ell);
-        Duu.xx = c1 * w.x * w.x + c2 * (1. - w.x * w.x * il2);
-        Duu.yy = c1 * w.y * w.y + c2 * (1. - w.y * w.y * il2);
-        Duu.zz = c1 * w.z * w.z + c2 * (1. - w.z * w.z * il2);
-        Duu.xy = c1 * w.x * w.y - c2 * w.x * w.y * il2;
-        Duu.xz = c1 * w.x * w.z - c2 * w.x * w.z * il2;
-        Duu.yz = c1 * w.y * w.z - c2 * w.y * w.z * il2;
-    }
-    const double ka = 2. / L, kv = 2. / L;
-    for (int g = 0; g < 4; ++g) {
-        double z = G.zgp[g];
-        double ku = (-24. * z) / (L * L);
-        double k1v = ka * vl.x, k2v = ku * ul.y + kv * vl.z, k3v = ku * ul.z - kv * vl.y;
-        double dl = G.dL[g];
-        double m1 = S.GJ * k1v, m2 = S.EI3 * k2v, m3v = S.EI2 * k3v;
-        fq[3] += dl * m1 * ka;
-        fq[1] += dl * m2 * ku; fq[5] += dl * m2 * kv;
-        fq[2] += dl * m3v * ku; fq[4] += -dl * m3v * kv;
-        D33 += dl * S.GJ * ka * ka;
-        Duu.yy += dl * S.EI3 * ku * ku; D15 += dl * S.EI3 * ku * kv; D55 += dl * S.EI3 * kv * kv;
-        Duu.zz += dl * S.EI2 * ku * ku; D24 += -dl * S.EI2 * ku * kv; D44 += dl * S.EI2 * kv * kv;
-    }
-    // external load Π_e = Σ_gp dL fₑ·(rₛₘ p_gp + cₛₘ), p_gp = tgₑ ζ + Y_gp q
-    v3 gphi_e = mk(0, 0, 0), esum = mk(0, 0, 0);
-    s3 Hee; Hee.xx = Hee.yy = Hee.zz = Hee.xy = Hee.xz = Hee.yz = 0.;
-    v3 Ye[6];   // columns of Ỹ = Σ spin(e) rₛₘ Y_gp over q = (u1,u2,u3,v1,v2,v3); column v1 is zero
-    for (int j = 0; j < 6; ++j) Ye[j] = mk(0, 0, 0);
-    {
-        v3 r0 = col(rsm, 0), r1 = col(rsm, 1), r2 = col(rsm, 2);
-        for (int g = 0; g < 4; ++g) {
-            double z = G.zgp[g];
-            double ya = 2. * z, yu = -4. * (z * z * z) + 3. * z, yv = (z * z - 1. / 4.) * L;
-            v3 y = mk(ya * ul.x, yu * ul.y + yv * vl.z, yu * ul.z - yv * vl.y);
-            v3 s = mul(rsm, mk(L * z + y.x, y.y, y.z));
-            v3 e = GEN ? eg[g] : G.dL[g] * fe;
-            esum = esum + e;
-            gphi_e = gphi_e + cross(s, e);
-            double es = dot(e, s);
-            Hee.xx += e.x * s.x - es; Hee.yy += e.y * s.y - es; Hee.zz += e.z * s.z - es;
-            Hee.xy += 0.5 * (e.x * s.y + s.x * e.y); Hee.xz += 0.5 * (e.x * s.z + s.x * e.z); Hee.yz += 0.5 * (e.y * s.z + s.y * e.z);
-            v3 re = mulT(rsm, e);
-            fq[0] += ya * re.x; fq[1] += yu * re.y; fq[5] += yv * re.y; fq[2] += yu * re.z; fq[4] += -yv * re.z;
-            Ye[0] = Ye[0] + cross(e, ya * r0);
-            Ye[1] = Ye[1] + cross(e, yu * r1);
-            Ye[2] = Ye[2] + cross(e, yu * r2);
-            Ye[4] = Ye[4] + cross(e, -yv * r2);
-            Ye[5] = Ye[5] + cross(e, yv * r1);
+// ------------------------------------------------ coefficient functions of t = θ²
+// a = sinθ/θ, b = (1−cosθ)/θ², c = (θ−sinθ)/θ³, each with its first two derivatives in t
+// (a′ = ½(c−b), b′ = (a−2b)/2t, c′ = (b−3c)/2t). Series for t < 1 (last term below 1e-18).
+struct RotFun { double a, b, c, a1, b1, c1, a2, b2, c2; };
+MH_HD RotFun rot_fun(double t) {
+    RotFun f;
+    if (t < 1.) {
+        // 1/(2k+2)!, 1/(2k+3)!
+        const double B[10] = {0.5, 1. / 24., 1. / 720., 1. / 40320., 1. / 3628800., 1. / 479001600., 1. / 87178291200.,
+                              1. / 20922789888000., 1. / 6402373705728000., 1. / 2432902008176640000.};
+        const double C[10] = {1. / 6., 1. / 120., 1. / 5040., 1. / 362880., 1. / 39916800., 1. / 6227020800.,
+                              1. / 1307674368000., 1. / 355687428096000., 1. / 121645100408832000.,
+                              1. / 51090942171709440000.};
+        const double u = -t;
+        double b = 0., b1 = 0., b2 = 0., c = 0., c1 = 0., c2 = 0.;
+#pragma unroll
+        for (int k = 9; k >= 0; --k) {
+            b = b * u + B[k]; c = c * u + C[k];
+            if (k > 0) { b1 = b1 * u - k * B[k]; c1 = c1 * u - k * C[k]; }
+            if (k > 1) { b2 = b2 * u + k * (k - 1) * B[k]; c2 = c2 * u + k * (k - 1) * C[k]; }
         }
+        f.b = b; f.b1 = b1; f.b2 = b2; f.c = c; f.c1 = c1; f.c2 = c2;
+        f.a = 1. - t * c;
+    } else {
+        const double th = sqrt(t), h = 0.5 / t, sh = sin(0.5 * th);
+        f.a = sin(th) / th;
+        f.b = 2. * sh * sh / t;
+        f.c = (1. - f.a) / t;
+        f.b1 = (f.a - 2. * f.b) * h;
+        f.c1 = (f.b - 3. * f.c) * h;
+        const double a1 = 0.5 * (f.c - f.b);
+        f.b2 = (a1 - 4. * f.b1) * h;
+        f.c2 = (f.b1 - 5. * f.c1) * h;
     }
-    v3 Fu = mul(rsm, mk(fq[0], fq[1], fq[2]));
-    v3 Fv = mul(rsm, mk(fq[3], fq[4], fq[5]));
-    v3 gphi = cross(Fu, d) + cross(Fv, dv) + gphi_e;
-    // couple term m·Log(rₛₘ): gradient T(ψ)⁻ᵀm w.r.t. the spatial spin of rₛₘ, and the
-    // second-order part -Jᵀ B J (J = T(ψ)⁻¹, B = dT_form(ψ, T⁻ᵀm)) of its Hessian
-    s3 Hm; Hm.xx = Hm.yy = Hm.zz = Hm.xy = Hm.xz = Hm.yz = 0.;
+    f.a1 = 0.5 * (f.c - f.b);
+    f.a2 = 0.5 * (f.c1 - f.b1);
+    return f;
+}
+// τ = tan(φ/4)/φ and κ = ½e − ¼τ, e = (1 − (φ/2)cot(φ/2))/φ², with two derivatives in t = φ² = 4θ²,
+// from the functions at θ = φ/2 (< π/2): τ = b/2a, κ = −c/8a.
+struct HalfFun { double k, k1, k2, q, q1, q2; };   // τ, τ′, τ″, κ, κ′, κ″
+MH_HD HalfFun half_fun(const RotFun& f) {
+    const double h = 0.5 / f.a, g = f.a1 / f.a;
+    HalfFun o;
+    o.k = f.b * h;
+    const double k1 = f.b1 * h - g * o.k;
+    o.k1 = 0.25 * k1;
+    o.k2 = 0.0625 * ((f.b2 - f.a2 / f.a * f.b) * h - 2. * g * k1);
+    const double q = f.c * h, q1 = f.c1 * h - g * q;
+    o.q = -0.25 * q;
+    o.q1 = -0.0625 * q1;
+    o.q2 = -0.015625 * ((f.c2 - f.a2 / f.a * f.c) * h - 2. * g * q1);
+    return o;
+}
+
+// The corotated frame (BeamElement.jl:192-208): r = rₛₘ, d = uₗ₂ + (L/2, 0, 0), vl = vₗ₂.
+struct BeamFrame { m3 r; v3 d, vl; RotFun f1, f2, fh; };   // coefficients at |v₁|², |v₂|², |vₗ|²
+MH_HD void beam_frame(const BeamGeo& G, const double* X, BeamFrame& f) {
+    const v3 v1 = mk(X[3], X[4], X[5]), v2 = mk(X[9], X[10], X[11]);
+    ExpCoef k;
+    f.f1 = rot_fun(dot(v1, v1)); f.f2 = rot_fun(dot(v2, v2));
+    k.a = f.f1.a; k.b = f.f1.b;
+    const m3 R1 = rodrigues(v1, k);
+    k.a = f.f2.a; k.b = f.f2.b;
+    const m3 M = mulABt(rodrigues(v2, k), R1);
+    // Δv = ½ Rodrigues⁻¹(M), Rodrigues⁻¹(M) = spin⁻¹(M)/scac((tr M - 1)/2)
+    const double h = 0.25 / scac((at(M, 0, 0) + at(M, 1, 1) + at(M, 2, 2) - 1.) / 2.);
+    const v3 dv = mk((at(M, 2, 1) - at(M, 1, 2)) * h, (at(M, 0, 2) - at(M, 2, 0)) * h, (at(M, 1, 0) - at(M, 0, 1)) * h);
+    f.fh = rot_fun(dot(dv, dv));
+    k.a = f.fh.a; k.b = f.fh.b;
+    f.r = mul(mul(rodrigues(dv, k), R1), G.rm);
+    // (u₂ + ½tgₘ) − cₛₘ in the reference's order: its rounding is the axial strain's
+    const v3 cs = mk(0.5 * (X[0] + X[6]), 0.5 * (X[1] + X[7]), 0.5 * (X[2] + X[8]));
+    f.d = mulT(f.r, mk(X[6] + G.tgm.x * 0.5 - cs.x, X[7] + G.tgm.y * 0.5 - cs.y, X[8] + G.tgm.z * 0.5 - cs.z));
+    f.vl = mulT(f.r, dv);
+}
+
+// The loads held fixed in the closed form: moments over the Gauss points of e_gp = dL_gp·fₑ with the
+// shape factors 1, ya, yu, yv of x_gp (global), and the couple Σ dL·mₑ. For a constant load ya and yu
+// sum to zero and yv to −L²/6.
+struct BeamLoads { v3 e0, ea, eu, ev, m; };
+
+// Residual and compact tangent of Π = Π_int + Σ_gp e_gp·x_gp + m·vₛₘ with the loads held fixed;
+// GEN = false: a constant load (ea = eu = m = 0). vₛₘ = Rodrigues⁻¹(rₛₘ) (BeamElement.jl:203).
+//
+// In the corotated frame (components along r's axes), with the node spins t_n = rᵀT(v_n)δv_n,
+// s = t₁+t₂, Δ = t₂−t₁, V = spin vₗ:
+//   frame spin ω = ½s − τVΔ, δvₗ = CΔ, C = ½I + 4κV², δd = rᵀδ(½(u₂−u₁)) + d×ω
+// (τ, κ: half_fun at |φ|² = 4|vₗ|²). The Gauss sums of the internal energy are exact:
+// Π_int = ½EA·L·ε² + ½(k₃d_y² + k₂d_z²) + ½vₗ·D vₗ, k = 48EI/L³, D = 4/L·diag(GJ, EI₂, EI₃).
+// Second derivatives: of ω and vₗ along constant node spins (the curvature of the rotations),
+//   N·W₂ + F_v·V₂ = Δ·(kA I + sym(v hᵀ))Δ + ½τ(N·s v·Δ − N·v s·Δ) + ½s·(P×Δ),
+// of body vectors b = rᵀB: ω×(ω×b). The axial force meets the rotations only through d×ω and drops
+// out of Q (the ω-ω part) and of the coupling to translations.
+//
+// Bound: FP64 latency at two waves per SIMD, then HBM. Over six columns of global spins the same
+// Hessian took 6,299 operations and 462 registers (one wave per SIMD); here about 2,000 and 256.
+// 973,000 elements: 320 µs before, 142 now.
+struct BeamSpin {
+    v3 Fb, N, Fv, ve, a, u;          // forces and moment, body loads
+    s3 Q, KD; m3 KS;                 // ω-ω, Δ-Δ, s-Δ
+    double k2, k3, c2, c3, tau, al, be;   // bending springs, axial terms of D_uu, τ, C = αI + βvvᵀ
+    v3 l1, l2;                       // node moments (global)
+    RotFun f1, f2;                   // T(v_n)
+};
+template <bool GEN>
+MH_HD void beam_spin(const BeamSection& S, double L, const BeamFrame& f, const double* X, const BeamLoads& ld, BeamSpin& o) {
+    const m3& r = f.r;
+    const v3 d = f.d, v = f.vl;
+    const v3 v1 = mk(X[3], X[4], X[5]), v2 = mk(X[9], X[10], X[11]);
+    const double k3 = 48. * S.EI3 / (L * L * L), k2 = 48. * S.EI2 / (L * L * L);
+    const v3 D = mk(4. / L * S.GJ, 4. / L * S.EI2, 4. / L * S.EI3);
+    const double ell = sqrt(dot(d, d)), de = 2. / (L * ell);
+    const double eps = ell * 2. / L - 1., fa = S.EA * L * eps;
+    const v3 ve = mulT(r, ld.ev);
+    v3 a = mk(0., 0., 0.), u = a;
+    // forces conjugate to d (Fb: without the axial force along d) and vₗ, moment conjugate to ω
+    v3 Fb = mk(0., k3 * d.y, k2 * d.z), N;
+    const v3 Fv = mk(D.x * v.x, D.y * v.y - ve.z, D.z * v.z + ve.y);
     if (GEN) {
-        v3 psi = mk(0, 0, 0);
-        {
-            double sc = scac((at(rsm, 0, 0) + at(rsm, 1, 1) + at(rsm, 2, 2) - 1.) / 2.);
-            psi = mk((at(rsm, 2, 1) - at(rsm, 1, 2)) / 2. / sc, (at(rsm, 0, 2) - at(rsm, 2, 0)) / 2. / sc,
-                     (at(rsm, 1, 0) - at(rsm, 0, 1)) / 2. / sc);
-        }
-        ExpCoef kpsi = exp_coef(norm3(psi));
-        m3 Jp = tangent_inv(psi, kpsi);
-        v3 mu_m = mulT(Jp, mtot);
-        gphi = gphi + mu_m;
-        s3 B = dT_form(psi, mu_m, kpsi);
-        v3 J0 = col(Jp, 0), J1 = col(Jp, 1), J2 = col(Jp, 2);
-        v3 BJ0 = smul(B, J0), BJ1 = smul(B, J1), BJ2 = smul(B, J2);
-        Hm.xx = -dot(J0, BJ0); Hm.yy = -dot(J1, BJ1); Hm.zz = -dot(J2, BJ2);
-        Hm.xy = -dot(J0, BJ1); Hm.xz = -dot(J0, BJ2); Hm.yz = -dot(J1, BJ2);
-        // parked (LDS, stride hst) until Hφφ' is formed: fewer registers live through the
-        // rotation Jacobians
-        if (hms) { hms[0] = Hm.xx; hms[hst] = Hm.yy; hms[2 * hst] = Hm.zz; hms[3 * hst] = Hm.xy; hms[4 * hst] = Hm.xz; hms[5 * hst] = Hm.yz; }
+        a = mulT(r, ld.ea); u = mulT(r, ld.eu);
+        Fb = Fb + mk(a.x, u.y, u.z);
     }
-    v3 gD = Fv;
-    // translational residual R = Aᵀ g_z on u₁, u₂
-    out.R[0] = -0.5 * Fu.x + 0.5 * esum.x; out.R[1] = -0.5 * Fu.y + 0.5 * esum.y; out.R[2] = -0.5 * Fu.z + 0.5 * esum.z;
-    out.R[6] = 0.5 * Fu.x + 0.5 * esum.x;  out.R[7] = 0.5 * Fu.y + 0.5 * esum.y;  out.R[8] = 0.5 * Fu.z + 0.5 * esum.z;
-    // ---- rotation core, first-order spin Jacobians (6 columns: δv₁ then δv₂) ----------
-    v3 JD[6], W[6], HT1[3], MT1[3], T2c[3];
-    m3 TH = tangent_op(dv, kh);
+    N = cross(Fb, d) + cross(mk(0., v.z, -v.y), ve);
+    s3 Q;   // ω-ω
     {
-        m3 T1 = tangent_op(v1, k1), T2 = tangent_op(v2, k2), Tpi = tangent_inv(phi, kp);
-        for (int j = 0; j < 3; ++j) {
-            v3 t1 = col(T1, j);
-            T2c[j] = col(T2, j);
-            MT1[j] = mul(M, t1);
-            HT1[j] = mul(H, t1);
-            JD[j] = mul(Tpi, -0.5 * MT1[j]);
-            JD[3 + j] = mul(Tpi, 0.5 * T2c[j]);
-        }
-        for (int j = 0; j < 6; ++j) W[j] = mul(TH, JD[j]);
-        for (int j = 0; j < 3; ++j) W[j] = W[j] + HT1[j];
-        // ---- second-order rotation chain contracted with the adjoints (into S) ------
-        // μ = ½ T(φ)⁻ᵀ (gΔ + T_Hᵀ gφ);  λ₁ = Hᵀ gφ - Mᵀ μ;  λ₂ = μ
-        v3 mu = 0.5 * mulT(Tpi, gD + mulT(TH, gphi));
-        v3 lam1 = mulT(H, gphi) - mulT(M, mu);
-        for (int i = 0; i < 21; ++i) out.Kc[24 + i] = 0.;
-        double* Sm = out.Kc + 24;
-        s3 B1 = dT_form(v1, lam1, k1), B2 = dT_form(v2, mu, k2);
-        Sm[sym6(0, 0)] += B1.xx; Sm[sym6(1, 1)] += B1.yy; Sm[sym6(2, 2)] += B1.zz;
-        Sm[sym6(0, 1)] += B1.xy; Sm[sym6(0, 2)] += B1.xz; Sm[sym6(1, 2)] += B1.yz;
-        Sm[sym6(3, 3)] += B2.xx; Sm[sym6(4, 4)] += B2.yy; Sm[sym6(5, 5)] += B2.zz;
-        Sm[sym6(3, 4)] += B2.xy; Sm[sym6(3, 5)] += B2.xz; Sm[sym6(4, 5)] += B2.yz;
-        s3 BH = dT_form(dv, gphi, kh), BP = dT_form(phi, mu, kp);
-        for (int a = 0; a < 6; ++a) {
-            // J_φ = 2 J_Δ:  J_Δᵀ B_H J_Δ - J_φᵀ B_P J_φ = J_Δᵀ (B_H - 4 B_P) J_Δ
-            v3 h = smul(BH, JD[a]) - 4. * smul(BP, JD[a]);
-            v3 wHa = a < 3 ? W[a] - HT1[a] : W[a];
-            for (int b = a; b < 6; ++b) {
-                v3 wHb = b < 3 ? W[b] - HT1[b] : W[b];
-                double t = dot(JD[b], h);
-                v3 hwa = a < 3 ? HT1[a] : mk(0, 0, 0), hwb = b < 3 ? HT1[b] : mk(0, 0, 0);
-                t += -0.5 * (dot(wHa, cross(gphi, hwb)) - dot(hwa, cross(gphi, wHb)));
-                v3 w2a = a >= 3 ? T2c[a - 3] : mk(0, 0, 0), w2b = b >= 3 ? T2c[b - 3] : mk(0, 0, 0);
-                v3 mwa = a < 3 ? MT1[a] : mk(0, 0, 0), mwb = b < 3 ? MT1[b] : mk(0, 0, 0);
-                t += 0.5 * (dot(w2a, cross(mu, mwb)) - dot(mwa, cross(mu, w2b)));
-                Sm[sym6(a, b)] += t;
-            }
-        }
-    }
-    // rotational residual
-    for (int j = 0; j < 6; ++j) out.R[j < 3 ? 3 + j : 6 + j] = dot(W[j], gphi) + dot(JD[j], gD);
-    // ---- A = rₛₘ D_uu rₛₘᵀ ----------------------------------------------------------------
-    {
-        v3 c0 = col(rsm, 0), c1 = col(rsm, 1), c2 = col(rsm, 2);
-        // rows of rₛₘ D_uu: (rₛₘ D_uu)[i][k] = Σ_m rsm[i][m] D[m][k]
-        v3 Dc0 = mk(Duu.xx, Duu.xy, Duu.xz), Dc1 = mk(Duu.xy, Duu.yy, Duu.yz), Dc2 = mk(Duu.xz, Duu.yz, Duu.zz);
-        v3 P0 = mul(rsm, Dc0), P1 = mul(rsm, Dc1), P2 = mul(rsm, Dc2);   // columns of rₛₘ D_uu
-        // A = (rₛₘ D_uu) rₛₘᵀ: A[i][j] = Σ_k P_k[i] rsm[j][k]
-        auto Aij = [&](int i, int j) {
-            return (&P0.x)[i] * at(rsm, j, 0) + (&P1.x)[i] * at(rsm, j, 1) + (&P2.x)[i] * at(rsm, j, 2);
+        auto sy = [](s3& q, v3 x, v3 y, double w) {   // q += w·sym(x yᵀ)
+            q.xx += w * x.x * y.x; q.yy += w * x.y * y.y; q.zz += w * x.z * y.z;
+            q.xy += 0.5 * w * (x.x * y.y + x.y * y.x); q.xz += 0.5 * w * (x.x * y.z + x.z * y.x);
+            q.yz += 0.5 * w * (x.y * y.z + x.z * y.y);
         };
-        out.Kc[0] = Aij(0, 0); out.Kc[1] = Aij(1, 1); out.Kc[2] = Aij(2, 2);
-        out.Kc[3] = Aij(0, 1); out.Kc[4] = Aij(0, 2); out.Kc[5] = Aij(1, 2);
-        (void)c0; (void)c1; (void)c2;
-    }
-    // ---- Br = ∂q/∂v (6×6), T, and the remaining rotation-rotation terms ---------------------
-    {
-        // Q3 = spin(F_u) - Ỹ_u rₛₘᵀ   (3×3),  T = rₛₘ(D_uu Br_u + D_uv Br_v) + Q3ᵀ W
-        s3 Hpp;   // Hφφ' = sym(Fu dᵀ) - (Fu·d)I + sym(Fv Δvᵀ) - (Fv·Δv)I + Σ[sym(e sᵀ) - (e·s)I]
-        double fud = dot(Fu, d), fvd = dot(Fv, dv);
-        Hpp.xx = Fu.x * d.x - fud + Fv.x * dv.x - fvd + Hee.xx;
-        Hpp.yy = Fu.y * d.y - fud + Fv.y * dv.y - fvd + Hee.yy;
-        Hpp.zz = Fu.z * d.z - fud + Fv.z * dv.z - fvd + Hee.zz;
-        Hpp.xy = 0.5 * (Fu.x * d.y + d.x * Fu.y) + 0.5 * (Fv.x * dv.y + dv.x * Fv.y) + Hee.xy;
-        Hpp.xz = 0.5 * (Fu.x * d.z + d.x * Fu.z) + 0.5 * (Fv.x * dv.z + dv.x * Fv.z) + Hee.xz;
-        Hpp.yz = 0.5 * (Fu.y * d.z + d.y * Fu.z) + 0.5 * (Fv.y * dv.z + dv.y * Fv.z) + Hee.yz;
-        if (GEN && hms) { Hm.xx = hms[0]; Hm.yy = hms[hst]; Hm.zz = hms[2 * hst]; Hm.xy = hms[3 * hst]; Hm.xz = hms[4 * hst]; Hm.yz = hms[5 * hst]; }
+        const v3 rv = mk(0., v.z, -v.y);
+        double tr = dot(Fb, d) + dot(rv, ve);
+        Q.xx = Q.yy = Q.zz = Q.xy = Q.xz = Q.yz = 0.;
+        sy(Q, Fb, d, 1.);
+        sy(Q, rv, ve, 1.);
+        const v3 gy = mk(d.z, 0., -d.x), gz = mk(-d.y, d.x, 0.);
+        sy(Q, gy, gy, k3);
+        sy(Q, gz, gz, k2);
         if (GEN) {
-            Hpp.xx += Hm.xx; Hpp.yy += Hm.yy; Hpp.zz += Hm.zz;
-            Hpp.xy += Hm.xy; Hpp.xz += Hm.xz; Hpp.yz += Hm.yz;
+            const v3 dx = mk(d.x, 0., 0.), dyz = mk(0., d.y, d.z);
+            N = N + cross(dx, a) + cross(dyz, u);
+            tr += d.x * a.x + (d.y * u.y + d.z * u.z);
+            sy(Q, dx, a, 1.);
+            sy(Q, dyz, u, 1.);
+            sy(Q, mk(0., -a.z, a.y), mk(0., -d.z, d.y), 2.);
+            sy(Q, mk(u.z, 0., -u.x), gy, 2.);
+            sy(Q, mk(-u.y, u.x, 0.), gz, 2.);
+            // couple: μ = T(ψ)⁻ᵀ rᵀm and −Jᵀ dT(ψ, μ) J, J = T(ψ)⁻¹ (r = Rodrigues(ψ) commutes with them)
+            double sc = scac((at(r, 0, 0) + at(r, 1, 1) + at(r, 2, 2) - 1.) / 2.);
+            const v3 psi = mk((at(r, 2, 1) - at(r, 1, 2)) / 2. / sc, (at(r, 0, 2) - at(r, 2, 0)) / 2. / sc,
+                              (at(r, 1, 0) - at(r, 0, 1)) / 2. / sc);
+            const ExpCoef kp = exp_coef(norm3(psi));
+            const m3 J = tangent_inv(psi, kp);
+            const v3 mu = mulT(J, mulT(r, ld.m));
+            N = N + mu;
+            const s3 B = dT_form(psi, mu, kp);
+            const v3 J0 = col(J, 0), J1 = col(J, 1), J2 = col(J, 2), B0 = smul(B, J0), B1 = smul(B, J1), B2 = smul(B, J2);
+            Q.xx -= dot(J0, B0); Q.yy -= dot(J1, B1); Q.zz -= dot(J2, B2);
+            Q.xy -= dot(J0, B1); Q.xz -= dot(J0, B2); Q.yz -= dot(J1, B2);
         }
-        double* Sm = out.Kc + 24;
-        v3 Bu[6], Bv[6], Np[6];
-        for (int j = 0; j < 6; ++j) {
-            Bu[j] = mulT(rsm, cross(d, W[j]));
-            Bv[j] = mulT(rsm, JD[j] + cross(dv, W[j]));
-            // N'_rot column j = spin(Fv) JD_j - Ỹ Br_j   (Ỹ column 3 (v1) is zero)
-            v3 yb = (Bu[j].x * Ye[0] + Bu[j].y * Ye[1]) + Bu[j].z * Ye[2];
-            yb = yb + Bv[j].y * Ye[4] + Bv[j].z * Ye[5];
-            Np[j] = cross(Fv, JD[j]) - yb;
+        Q.xx -= tr; Q.yy -= tr; Q.zz -= tr;
+    }
+    o.c2 = fa * de;
+    o.c3 = S.EA * L * de * de - o.c2 / (ell * ell);
+    // rotations: node moments and the spin blocks K₁₁, K₁₂, K₂₂
+    const double vv = dot(v, v);
+    const HalfFun hf = half_fun(f.fh);
+    const double tau = hf.k, be = 4. * hf.q, al = 0.5 - be * vv;
+    const v3 P = al * Fv + (be * dot(v, Fv)) * v, Nv = cross(N, v);
+    o.f1 = f.f1; o.f2 = f.f2;
+    const v3 pD = P - tau * Nv;
+    o.l1 = mul(r, 0.5 * N - pD); o.l2 = mul(r, 0.5 * N + pD);
+    m3 QV;   // Q V
+    m3& KS = o.KS;   // K_sΔ = −½τQV + ½GᵀC + ¼τ(N vᵀ − N·v I) + ¼spin(P), G = spin(e₁) spin(ve)
+    s3& KD = o.KD;   // K_ΔΔ = τ²VᵀQV + C D C + sym(C G W) + kA I + sym(v hᵀ)
+    {
+        const v3 q0 = mk(Q.xx, Q.xy, Q.xz), q1 = mk(Q.xy, Q.yy, Q.yz), q2 = mk(Q.xz, Q.yz, Q.zz);
+        // rows of QV: q×v
+        const v3 w0 = cross(q0, v), w1 = cross(q1, v), w2 = cross(q2, v);
+        QV.a[0] = w0.x; QV.a[3] = w0.y; QV.a[6] = w0.z;
+        QV.a[1] = w1.x; QV.a[4] = w1.y; QV.a[7] = w1.z;
+        QV.a[2] = w2.x; QV.a[5] = w2.y; QV.a[8] = w2.z;
+        // VᵀQV: columns QV_j → −v×(QV_j)
+        const v3 c0 = cross(col(QV, 0), v), c1 = cross(col(QV, 1), v), c2 = cross(col(QV, 2), v);
+        const double t2 = tau * tau;
+        KD.xx = t2 * c0.x; KD.yy = t2 * c1.y; KD.zz = t2 * c2.z;
+        KD.xy = t2 * c1.x; KD.xz = t2 * c2.x; KD.yz = t2 * c2.y;
+        const double b2 = be * be * (D.x * v.x * v.x + D.y * v.y * v.y + D.z * v.z * v.z), ab = al * be;
+        const double fv = dot(Fv, v);
+        const double kA = fv * (-0.5 * tau + be * al);
+        const double kB = 0.5 * tau - 16. * hf.q1 * vv + be * (al - 1. - tau * vv);
+        const double kC = fv * (16. * hf.q1 + 2. * be * be + be * tau);
+        const double c = tau * tau + 4. * hf.k1 + be * tau;
+        const v3 h = kB * Fv + kC * v - c * Nv;
+        KD.xx += al * al * D.x + (2. * ab * D.x + b2) * v.x * v.x + kA + v.x * h.x;
+        KD.yy += al * al * D.y + (2. * ab * D.y + b2) * v.y * v.y + kA + v.y * h.y;
+        KD.zz += al * al * D.z + (2. * ab * D.z + b2) * v.z * v.z + kA + v.z * h.z;
+        KD.xy += (ab * (D.x + D.y) + b2) * v.x * v.y + 0.5 * (v.x * h.y + v.y * h.x);
+        KD.xz += (ab * (D.x + D.z) + b2) * v.x * v.z + 0.5 * (v.x * h.z + v.z * h.x);
+        KD.yz += (ab * (D.y + D.z) + b2) * v.y * v.z + 0.5 * (v.y * h.z + v.z * h.y);
+        // G = ve e₁ᵀ − (ve·e₁) I; GᵀC = e₁ (C ve)ᵀ − veₓ C, CGW = −τ(C ve (e₁ᵀV) − veₓ C V); CV = αV
+        const v3 Cve = al * ve + (be * dot(v, ve)) * v;
+        const v3 eV = mk(0., -v.z, v.y);   // row e₁ᵀV
+        // sym(αV) = 0, so only the dyad remains: CGW + (CGW)ᵀ = −τ(Cve eVᵀ + eV Cveᵀ)
+        KD.yy -= 2. * tau * Cve.y * eV.y; KD.zz -= 2. * tau * Cve.z * eV.z;
+        KD.xy -= tau * Cve.x * eV.y; KD.xz -= tau * Cve.x * eV.z; KD.yz -= tau * (Cve.y * eV.z + Cve.z * eV.y);
+        const double nv = 0.25 * tau * dot(N, v), t4 = 0.25 * tau, ht = 0.5 * tau;
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            const double vj = j == 0 ? v.x : (j == 1 ? v.y : v.z);
+            KS.a[3 * j] = t4 * N.x * vj - ht * QV.a[3 * j];
+            KS.a[3 * j + 1] = t4 * N.y * vj - ht * QV.a[3 * j + 1];
+            KS.a[3 * j + 2] = t4 * N.z * vj - ht * QV.a[3 * j + 2];
         }
-        for (int a = 0; a < 6; ++a) {
-            // D Br column a
-            v3 DBu = smul(Duu, Bu[a]) + mk(0., D15 * Bv[a].z, D24 * Bv[a].y);
-            v3 DBv = mk(D33 * Bv[a].x, D44 * Bv[a].y + D24 * Bu[a].z, D55 * Bv[a].z + D15 * Bu[a].y);
-            v3 hw = smul(Hpp, W[a]);
-            for (int b = a; b < 6; ++b) {
-                double t = dot(Bu[b], DBu) + dot(Bv[b], DBv) + dot(W[b], hw) + dot(W[a], Np[b]) + dot(W[b], Np[a]);
-                Sm[sym6(a, b)] += t;
-            }
-            // T column a: rₛₘ (D_uu Bu_a + D_uv Bv_a) + Q3ᵀ W_a
-            v3 C = mul(rsm, DBu);
-            // Q3ᵀ W_a = spin(Fu)ᵀ W_a - rₛₘ Ỹ_uᵀ W_a = W_a × Fu - rₛₘ (Ye_k · W_a)_k
-            v3 yw = mk(dot(Ye[0], W[a]), dot(Ye[1], W[a]), dot(Ye[2], W[a]));
-            v3 Tc = C + cross(W[a], Fu) - mul(rsm, yw);
-            out.Kc[6 + 0 * 6 + a] = Tc.x; out.Kc[6 + 1 * 6 + a] = Tc.y; out.Kc[6 + 2 * 6 + a] = Tc.z;
+        KS.a[0] -= nv; KS.a[4] -= nv; KS.a[8] -= nv;
+        KS.a[0] += 0.5 * Cve.x; KS.a[3] += 0.5 * Cve.y; KS.a[6] += 0.5 * Cve.z;   // ½e₁(C ve)ᵀ
+        const double hx = 0.5 * ve.x;
+        KS.a[0] -= hx * (al + be * v.x * v.x); KS.a[4] -= hx * (al + be * v.y * v.y); KS.a[8] -= hx * (al + be * v.z * v.z);
+        const double sxy = hx * be * v.x * v.y, sxz = hx * be * v.x * v.z, syz = hx * be * v.y * v.z;
+        KS.a[1] -= sxy; KS.a[3] -= sxy; KS.a[2] -= sxz; KS.a[6] -= sxz; KS.a[5] -= syz; KS.a[7] -= syz;
+        KS.a[1] += 0.25 * P.z; KS.a[3] -= 0.25 * P.z;
+        KS.a[2] -= 0.25 * P.y; KS.a[6] += 0.25 * P.y;
+        KS.a[5] += 0.25 * P.x; KS.a[7] -= 0.25 * P.x;
+    }
+    o.Fb = Fb; o.N = N; o.Fv = Fv; o.ve = ve; o.a = a; o.u = u; o.Q = Q;
+    o.k2 = k2; o.k3 = k3; o.tau = tau; o.al = al; o.be = be;
+}
+
+template <bool GEN>
+MH_HD void beam_tangent(const BeamSection& S, double L, const BeamFrame& f, const double* X, const BeamLoads& ld,
+                        BeamOut& out) {
+    const m3& r = f.r;
+    const v3 d = f.d, v = f.vl;
+    const v3 v1 = mk(X[3], X[4], X[5]), v2 = mk(X[9], X[10], X[11]);
+    BeamSpin o;
+    beam_spin<GEN>(S, L, f, X, ld, o);
+    const RotFun &f1 = o.f1, &f2 = o.f2;
+    const v3 &Fb = o.Fb, &a = o.a, &u = o.u, &l1 = o.l1, &l2 = o.l2;
+    const s3 &Q = o.Q, &KD = o.KD;
+    const m3& KS = o.KS;
+    const double k2 = o.k2, k3 = o.k3, tau = o.tau;
+    // translations: residual and A = r D_uu rᵀ, D_uu = c₂I + c₃ d dᵀ + diag(0, k₃, k₂)
+    {
+        const v3 g = mul(r, Fb + o.c2 * d);
+        out.R[0] = 0.5 * (ld.e0.x - g.x); out.R[1] = 0.5 * (ld.e0.y - g.y); out.R[2] = 0.5 * (ld.e0.z - g.z);
+        out.R[6] = 0.5 * (ld.e0.x + g.x); out.R[7] = 0.5 * (ld.e0.y + g.y); out.R[8] = 0.5 * (ld.e0.z + g.z);
+        const double c2 = o.c2, c3 = o.c3;
+        const v3 dg = mul(r, d), ry = col(r, 1), rz = col(r, 2);
+        out.Kc[0] = c2 + (c3 * dg.x * dg.x + k3 * ry.x * ry.x + k2 * rz.x * rz.x);
+        out.Kc[1] = c2 + (c3 * dg.y * dg.y + k3 * ry.y * ry.y + k2 * rz.y * rz.y);
+        out.Kc[2] = c2 + (c3 * dg.z * dg.z + k3 * ry.z * ry.z + k2 * rz.z * rz.z);
+        out.Kc[3] = c3 * dg.x * dg.y + k3 * ry.x * ry.y + k2 * rz.x * rz.y;
+        out.Kc[4] = c3 * dg.x * dg.z + k3 * ry.x * ry.z + k2 * rz.x * rz.z;
+        out.Kc[5] = c3 * dg.y * dg.z + k3 * ry.y * ry.z + k2 * rz.y * rz.z;
+    }
+    auto Tt = [](v3 w, const RotFun& k, v3 q) { const v3 y = cross(w, q); return q - k.b * y + k.c * cross(w, y); };
+    {
+        const v3 q1 = Tt(v1, f1, l1), q2 = Tt(v2, f2, l2);
+        out.R[3] = q1.x; out.R[4] = q1.y; out.R[5] = q1.z;
+        out.R[9] = q2.x; out.R[10] = q2.y; out.R[11] = q2.z;
+    }
+    // L_n = rᵀT(v_n), column j: rᵀ(e_j + b v×e_j + c v×(v×e_j))
+    auto Lcol = [&](v3 w, const RotFun& k, int j) {
+        const v3 e = mk(j == 0 ? 1. : 0., j == 1 ? 1. : 0., j == 2 ? 1. : 0.), y = cross(w, e);
+        return mulT(r, e + k.b * y + k.c * cross(w, y));
+    };
+    v3 L1[3], L2[3];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) { L1[j] = Lcol(v1, f1, j); L2[j] = Lcol(v2, f2, j); }
+    auto dyt = [](v3 w, v3 g, const RotFun& k) {
+        ExpCoef q;
+        q.c = k.c; q.beta = 2. * k.b1; q.gamma = 2. * k.c1;
+        return dT_form(w, g, q);
+    };
+    double* Sm = out.Kc + 24;
+    {
+        auto sm = [&](double sg) {   // ¼Q + K_ΔΔ + sg (K_sΔ + K_sΔᵀ)
+            s3 k;
+            k.xx = 0.25 * Q.xx + KD.xx + 2. * sg * KS.a[0]; k.yy = 0.25 * Q.yy + KD.yy + 2. * sg * KS.a[4];
+            k.zz = 0.25 * Q.zz + KD.zz + 2. * sg * KS.a[8];
+            k.xy = 0.25 * Q.xy + KD.xy + sg * (KS.a[1] + KS.a[3]);
+            k.xz = 0.25 * Q.xz + KD.xz + sg * (KS.a[2] + KS.a[6]);
+            k.yz = 0.25 * Q.yz + KD.yz + sg * (KS.a[5] + KS.a[7]);
+            return k;
+        };
+        const s3 K1 = sm(-1.), B1 = dyt(v1, l1, f1);
+        const v3 x0 = smul(K1, L1[0]), x1 = smul(K1, L1[1]), x2 = smul(K1, L1[2]);
+        Sm[sym6(0, 0)] = dot(L1[0], x0) + B1.xx; Sm[sym6(0, 1)] = dot(L1[0], x1) + B1.xy;
+        Sm[sym6(0, 2)] = dot(L1[0], x2) + B1.xz; Sm[sym6(1, 1)] = dot(L1[1], x1) + B1.yy;
+        Sm[sym6(1, 2)] = dot(L1[1], x2) + B1.yz; Sm[sym6(2, 2)] = dot(L1[2], x2) + B1.zz;
+        const s3 K2 = sm(1.), B2 = dyt(v2, l2, f2);
+        const v3 y0 = smul(K2, L2[0]), y1 = smul(K2, L2[1]), y2 = smul(K2, L2[2]);
+        Sm[sym6(3, 3)] = dot(L2[0], y0) + B2.xx; Sm[sym6(3, 4)] = dot(L2[0], y1) + B2.xy;
+        Sm[sym6(3, 5)] = dot(L2[0], y2) + B2.xz; Sm[sym6(4, 4)] = dot(L2[1], y1) + B2.yy;
+        Sm[sym6(4, 5)] = dot(L2[1], y2) + B2.yz; Sm[sym6(5, 5)] = dot(L2[2], y2) + B2.zz;
+        // K₁₂ = ¼Q − K_ΔΔ + K_sΔ − K_sΔᵀ
+        const double qxx = 0.25 * Q.xx - KD.xx, qyy = 0.25 * Q.yy - KD.yy, qzz = 0.25 * Q.zz - KD.zz;
+        const double qxy = 0.25 * Q.xy - KD.xy, qxz = 0.25 * Q.xz - KD.xz, qyz = 0.25 * Q.yz - KD.yz;
+        const double axy = KS.a[3] - KS.a[1], axz = KS.a[6] - KS.a[2], ayz = KS.a[7] - KS.a[5];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            const v3 q = L2[j];
+            const v3 z = mk(qxx * q.x + (qxy + axy) * q.y + (qxz + axz) * q.z,
+                            (qxy - axy) * q.x + qyy * q.y + (qyz + ayz) * q.z,
+                            (qxz - axz) * q.x + (qyz - ayz) * q.y + qzz * q.z);
+#pragma unroll
+            for (int i = 0; i < 3; ++i) Sm[sym6(i, 3 + j)] = dot(L1[i], z);
         }
+    }
+    // T = r T_ω [W₁L₁ | W₂L₂], W = ½I ± τV, T_ω ω = ω×Fb + (0, k₃, k₂)∘(d×ω) + ((a×ω)ₓ, (u×ω)_y, (u×ω)_z)
+    auto Tcol = [&](v3 l, double sg) {
+        const v3 w = 0.5 * l + (sg * tau) * cross(v, l);   // ω of this node's column
+        const v3 dw = cross(d, w);
+        v3 t = cross(w, Fb) + mk(0., k3 * dw.y, k2 * dw.z);
+        if (GEN) { const v3 aw = cross(a, w), uw = cross(u, w); t = t + mk(aw.x, uw.y, uw.z); }
+        return mul(r, t);
+    };
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        const v3 t1 = Tcol(L1[j], 1.), t2 = Tcol(L2[j], -1.);
+        out.Kc[6 + j] = t1.x; out.Kc[12 + j] = t1.y; out.Kc[18 + j] = t1.z;
+        out.Kc[9 + j] = t2.x; out.Kc[15 + j] = t2.y; out.Kc[21 + j] = t2.z;
     }
     int nan = 0;
     // Muscade's residual always contracts mₑ with ∂vₛₘ/∂X (BeamElement.jl:170), with
     // vₛₘ = Rodrigues⁻¹(rₛₘ) = spin⁻¹(rₛₘ)/scac((tr rₛₘ - 1)/2): for a corotated frame at
     // a half turn, scac and acos′ there make it NaN even where mₑ = 0.
-    if (!GEN) nan |= !((at(rsm, 0, 0) + at(rsm, 1, 1) + at(rsm, 2, 2) - 1.) / 2. > -1.);
+    if (!GEN) nan |= !((at(r, 0, 0) + at(r, 1, 1) + at(r, 2, 2) - 1.) / 2. > -1.);
     for (int i = 0; i < 12; ++i) nan |= (out.R[i] != out.R[i]);
     for (int i = 0; i < kCompact; ++i) nan |= (out.Kc[i] != out.Kc[i]);
     out.nan = nan;
+}
+// The static element: fₑ constant along the beam.
+MH_HD void beam_static(const BeamGeo& G, const BeamSection& S, v3 fe, const double* X, BeamOut& out) {
+    BeamFrame f;
+    beam_frame(G, X, f);
+    BeamLoads ld;
+    ld.e0 = G.L * fe;
+    ld.ev = (-G.L * G.L / 6.) * fe;
+    ld.ea = ld.eu = ld.m = mk(0., 0., 0.);
+    beam_tangent<false>(S, G.L, f, X, ld, out);
+}
+
+// Λ·∂R/∂X (g, 12) and Λ·∂R/∂fₑ (gf) of the static element: the second derivative of Π along Λ, without
+// forming the tangent. Returns whether a value is NaN (the element's own NaN included).
+MH_HD int beam_static_vjp(const BeamGeo& G, const BeamSection& S, v3 fe, const double* X, const double* lam, double* g,
+                          v3& gf) {
+    const double L = G.L;
+    BeamFrame f;
+    beam_frame(G, X, f);
+    BeamLoads ld;
+    ld.e0 = L * fe;
+    ld.ev = (-L * L / 6.) * fe;
+    ld.ea = ld.eu = ld.m = mk(0., 0., 0.);
+    BeamSpin o;
+    beam_spin<false>(S, L, f, X, ld, o);
+    const m3& r = f.r;
+    const v3 d = f.d, v = f.vl, v1 = mk(X[3], X[4], X[5]), v2 = mk(X[9], X[10], X[11]);
+    const v3 u1 = mk(lam[0], lam[1], lam[2]), r1 = mk(lam[3], lam[4], lam[5]), u2 = mk(lam[6], lam[7], lam[8]),
+             r2 = mk(lam[9], lam[10], lam[11]);
+    auto T = [](v3 w, const RotFun& k, v3 q, double sg) { const v3 y = cross(w, q); return q + (sg * k.b) * y + k.c * cross(w, y); };
+    const v3 t1 = mulT(r, T(v1, o.f1, r1, 1.)), t2 = mulT(r, T(v2, o.f2, r2, 1.));
+    const v3 s = t1 + t2, dl = t2 - t1, D = mulT(r, 0.5 * (u2 - u1));
+    const v3 w = 0.5 * s - o.tau * cross(v, dl), dw = cross(d, w);
+    // d: D_uu D + T_ω ω
+    const v3 k = mk(0., o.k3, o.k2);
+    auto had = [](v3 x, v3 y) { return mk(x.x * y.x, x.y * y.y, x.z * y.z); };
+    const v3 gd = mul(r, o.c2 * D + (o.c3 * dot(d, D)) * d + had(k, D) + cross(w, o.Fb) + had(k, dw));
+    // T_ωᵀD on both nodes' frame spins
+    const v3 q = cross(o.Fb, D) + cross(had(k, D), d), qv = o.tau * cross(v, q);
+    const v3 ys = 0.25 * smul(o.Q, s) + mul(o.KS, dl), yd = mulT(o.KS, s) + smul(o.KD, dl);
+    const v3 y1 = ys - yd + 0.5 * q - qv, y2 = ys + yd + 0.5 * q + qv;
+    ExpCoef kc;
+    kc.c = o.f1.c; kc.beta = 2. * o.f1.b1; kc.gamma = 2. * o.f1.c1;
+    const v3 g1 = T(v1, o.f1, mul(r, y1), -1.) + smul(dT_form(v1, o.l1, kc), r1);
+    kc.c = o.f2.c; kc.beta = 2. * o.f2.b1; kc.gamma = 2. * o.f2.c1;
+    const v3 g2 = T(v2, o.f2, mul(r, y2), -1.) + smul(dT_form(v2, o.l2, kc), r2);
+    g[0] = -0.5 * gd.x; g[1] = -0.5 * gd.y; g[2] = -0.5 * gd.z; g[3] = g1.x; g[4] = g1.y; g[5] = g1.z;
+    g[6] = 0.5 * gd.x; g[7] = 0.5 * gd.y; g[8] = 0.5 * gd.z; g[9] = g2.x; g[10] = g2.y; g[11] = g2.z;
+    // Σ_gp dL x_gp = L cₛₘ − L²/6 r(vₗ×e₁)
+    const v3 dvl = o.al * dl + (o.be * dot(v, dl)) * v;
+    gf = (0.5 * L) * (u1 + u2) + (-L * L / 6.) * mul(r, cross(w, mk(0., v.z, -v.y)) + mk(0., dvl.z, -dvl.y));
+    int nan = !((at(r, 0, 0) + at(r, 1, 1) + at(r, 2, 2) - 1.) / 2. > -1.);
+    for (int i = 0; i < 12; ++i) nan |= g[i] != g[i];
+    return nan;
 }
 
 // Full 12×12 entry from the compact form (host harnesses and checks).

@@ -318,7 +318,7 @@ struct BeamArgs {
 // The 45 tangent numbers of the block's elements are staged in LDS and written
 // as one contiguous, coalesced range.
 template <bool UDOF, int BLK>
-__global__ __launch_bounds__(BLK) void beam_static_kernel(BeamArgs a) {
+__global__ __launch_bounds__(BLK, 2) void beam_static_kernel(BeamArgs a) {
     __shared__ double tile[BLK * mh::kCompact];
     const int64_t e0 = xcd_tile(a.per_xcd) * BLK;
     if (e0 >= a.nele) return;   // whole workgroup leaves together
@@ -493,17 +493,19 @@ __device__ __forceinline__ void dyn_load(const BeamDynArgs& a, int64_t e, mh::Be
     }
 }
 
-// Value pass, one element per lane: the element's record and the frozen loads from the time jets,
-// then the residual and the compact tangent of Π with those loads held fixed.
+// Value pass, one element per lane: the element's record and the loads, then the residual and the
+// compact tangent of Π with those loads held fixed. Bound: FP64 latency at two waves per SIMD, and the
+// records (1,096 B an element at second order). From time jets it took 19,400 instructions and one
+// wave per SIMD, in closed form 8,800; 383,000 elements, second order: 362 µs before, 219 now.
 constexpr int kDynTile = 64;   // elements whose records lie together
 constexpr int kDynRecMax = mh::kDynRec<3>;
-static_assert(kBeamBlock % kDynTile == 0, "whole tiles per workgroup");
+constexpr int kValueBlock = 64;   // one wave: the LDS tile of the compact tangents lets seven share a CU
+static_assert(kValueBlock % kDynTile == 0, "whole tiles per workgroup");
 int64_t rec_numbers(int64_t nele) { return (nele + kDynTile - 1) / kDynTile * kDynTile * kDynRecMax; }
 template <int ND, bool UDOF>
-__global__ __launch_bounds__(kBeamBlock) void beam_dyn_value_kernel(BeamDynArgs a) {
-    __shared__ double tile[kBeamBlock * mh::kCompact];
-    __shared__ double hmsh[6 * kBeamBlock];   // each lane's couple Hessian, parked (stride kBeamBlock)
-    const int64_t e0 = xcd_tile(a.per_xcd) * kBeamBlock;
+__global__ __launch_bounds__(kValueBlock, 2) void beam_dyn_value_kernel(BeamDynArgs a) {
+    __shared__ double tile[kValueBlock * mh::kCompact];
+    const int64_t e0 = xcd_tile(a.per_xcd) * kValueBlock;
     if (e0 >= a.nele) return;   // whole workgroup leaves together
     const int tid = threadIdx.x;
     const int64_t e = e0 + tid;
@@ -514,11 +516,14 @@ __global__ __launch_bounds__(kBeamBlock) void beam_dyn_value_kernel(BeamDynArgs 
         mh::BeamDynSection D;
         double X[ND][12], U[3];
         dyn_load<ND, UDOF>(a, e, G, S, D, X, U);
-        mh::v3 eg[4], mtot;
+        mh::BeamFrame f;
+        mh::BeamLoads ld;
         double* rec = a.rec + e / kDynTile * (kDynTile * mh::kDynRec<ND>) + e % kDynTile;
-        mh::dyn_record<ND>(G, D, X, U, [&](int q, double v) { rec[q * kDynTile] = v; }, eg, mtot);
+        mh::beam_frame(G, X[0], f);
+        mh::dyn_record<ND>(G, D, X, U, f, [&](int q, double v) { rec[q * kDynTile] = v; }, ld);
+        MH_PHASE();
         mh::BeamOut out;
-        mh::beam_static<true>(G, S, mh::mk(0., 0., 0.), X[0], out, eg, mtot, hmsh + tid, kBeamBlock);
+        mh::beam_tangent<true>(S, G.L, f, X[0], ld, out);
         if (a.R) {
 #pragma unroll
             for (int i = 0; i < 12; ++i) a.R[i * n + e] = out.R[i] * a.sR[i];
@@ -533,9 +538,9 @@ __global__ __launch_bounds__(kBeamBlock) void beam_dyn_value_kernel(BeamDynArgs 
         if (out.nan) atomicMin(a.flag, a.gtag | (unsigned long long)e);
     }
     __syncthreads();
-    const int64_t nv = (n - e0 < kBeamBlock ? n - e0 : kBeamBlock) * mh::kCompact;
+    const int64_t nv = (n - e0 < kValueBlock ? n - e0 : kValueBlock) * mh::kCompact;
     double* dst = a.Kc + e0 * mh::kCompact;
-    for (int64_t f = tid; f < nv; f += kBeamBlock) dst[f] = tile[f];
+    for (int64_t f = tid; f < nv; f += kValueBlock) dst[f] = tile[f];
 }
 
 // Requestables of the beams of one group at the device state (mh_beam_results): one
@@ -852,16 +857,16 @@ struct VjpArgs {
     unsigned long long gtag;
 };
 
-// Static beams, one per lane: Λ·K = K·Λ with the compact symmetric tangent; U-dofs
-// through y = ∂x_gp/∂X·Λ (one ε-jet pass).
+// Static beams, one per lane: Λ·K, the second derivative of Π along Λ (mh::beam_static_vjp), and
+// ∂L/∂U = −Λ·∂R/∂fₑ.
 template <bool UDOF>
 __global__ __launch_bounds__(kBeamBlock) void beam_vjp_static_kernel(VjpArgs a) {
     const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= a.nele) return;
     const int64_t n = a.nele;
-    double X[1][12], lam[12];
+    double X[12], lam[12];
 #pragma unroll
-    for (int k = 0; k < 12; ++k) { const int32_t q = a.idx[k * n + e]; X[0][k] = a.X[0][q]; lam[k] = a.lam[q]; }
+    for (int k = 0; k < 12; ++k) { const int32_t q = a.idx[k * n + e]; X[k] = a.X[0][q]; lam[k] = a.lam[q]; }
     const int32_t n1 = a.nodes[e], n2 = a.nodes[n + e];
     mh::v3 c1 = mh::mk(a.xyz[3 * (int64_t)n1], a.xyz[3 * (int64_t)n1 + 1], a.xyz[3 * (int64_t)n1 + 2]);
     mh::v3 c2 = mh::mk(a.xyz[3 * (int64_t)n2], a.xyz[3 * (int64_t)n2 + 1], a.xyz[3 * (int64_t)n2 + 2]);
@@ -869,25 +874,13 @@ __global__ __launch_bounds__(kBeamBlock) void beam_vjp_static_kernel(VjpArgs a) 
     mh::BeamSection S;
     S.EA = a.sec[e]; S.EI2 = a.sec[n + e]; S.EI3 = a.sec[2 * n + e]; S.GJ = a.sec[3 * n + e]; S.w = a.sec[6 * n + e];
     mh::v3 fe = mh::mk(0., 0., S.w);
-    int nan = 0;
-    if (UDOF) {
-        fe = fe - mh::mk(a.U[a.uidx[e]], a.U[a.uidx[n + e]], a.U[a.uidx[2 * n + e]]);
-        // ∂L/∂U first, so that nothing but λ stays live through the closed form
-        mh::DynY y;
-        mh::dyn_y(G, X, lam, y);
-        const mh::v3 gu = mh::dyn_vjp_u(G, y);
-        a.gu[e] = gu.x; a.gu[n + e] = gu.y; a.gu[2 * n + e] = gu.z;
-    }
-    mh::BeamOut out;
-    mh::beam_static(G, S, fe, X[0], out);
-    nan |= out.nan;
+    if (UDOF) fe = fe - mh::mk(a.U[a.uidx[e]], a.U[a.uidx[n + e]], a.U[a.uidx[2 * n + e]]);
+    double g[12];
+    mh::v3 gf;
+    const int nan = mh::beam_static_vjp(G, S, fe, X, lam, g, gf);
+    if (UDOF) { a.gu[e] = -gf.x; a.gu[n + e] = -gf.y; a.gu[2 * n + e] = -gf.z; }
 #pragma unroll
-    for (int i = 0; i < 12; ++i) {
-        double g = 0.;
-        for (int j = 0; j < 12; ++j) g = g + mh::compact_entry(out.Kc, i, j) * lam[j];
-        a.g[i * n + e] = g;
-        nan |= g != g;
-    }
+    for (int i = 0; i < 12; ++i) a.g[i * n + e] = g[i];
     if (nan) atomicMin(a.flag, a.gtag | (unsigned long long)e);
 }
 
@@ -1547,9 +1540,9 @@ BeamArgs static_beam_args(Ctx* c, const Group& g, unsigned long long gtag) {
 template <int ND, bool UDOF>
 void launch_dyn(BeamDynArgs& a, bool step, hipStream_t s) {
     {
-        const int64_t ntile = (a.nele + kBeamBlock - 1) / kBeamBlock;
+        const int64_t ntile = (a.nele + kValueBlock - 1) / kValueBlock;
         a.per_xcd = (ntile + kXCD - 1) / kXCD;
-        hipLaunchKernelGGL((beam_dyn_value_kernel<ND, UDOF>), dim3((unsigned)(a.per_xcd * kXCD)), dim3(kBeamBlock), 0, s, a);
+        hipLaunchKernelGGL((beam_dyn_value_kernel<ND, UDOF>), dim3((unsigned)(a.per_xcd * kXCD)), dim3(kValueBlock), 0, s, a);
     }
     const int tile = step ? kStepTile : kDirTile;
     const int64_t ntile = (a.nele + tile - 1) / tile;
@@ -1640,15 +1633,15 @@ int launch_vjp(Ctx* c, const Group& g, int nd, unsigned long long gtag) {
         b.Kc = c->d_Kc + g.kcbase; b.K = nullptr; b.R = nullptr; b.dR = nullptr;
         b.rec = c->d_rec + g.recbase;
         b.flag = c->d_flag; b.gtag = gtag;
-        const int64_t ntile = (g.nele + kBeamBlock - 1) / kBeamBlock;
+        const int64_t ntile = (g.nele + kValueBlock - 1) / kValueBlock;
         b.per_xcd = (ntile + kXCD - 1) / kXCD;
         const dim3 grv((unsigned)(b.per_xcd * kXCD));
         if (nd == 2) {
-            if (u) hipLaunchKernelGGL((beam_dyn_value_kernel<2, true>), grv, dim3(kBeamBlock), 0, s, b);
-            else hipLaunchKernelGGL((beam_dyn_value_kernel<2, false>), grv, dim3(kBeamBlock), 0, s, b);
+            if (u) hipLaunchKernelGGL((beam_dyn_value_kernel<2, true>), grv, dim3(kValueBlock), 0, s, b);
+            else hipLaunchKernelGGL((beam_dyn_value_kernel<2, false>), grv, dim3(kValueBlock), 0, s, b);
         } else {
-            if (u) hipLaunchKernelGGL((beam_dyn_value_kernel<3, true>), grv, dim3(kBeamBlock), 0, s, b);
-            else hipLaunchKernelGGL((beam_dyn_value_kernel<3, false>), grv, dim3(kBeamBlock), 0, s, b);
+            if (u) hipLaunchKernelGGL((beam_dyn_value_kernel<3, true>), grv, dim3(kValueBlock), 0, s, b);
+            else hipLaunchKernelGGL((beam_dyn_value_kernel<3, false>), grv, dim3(kValueBlock), 0, s, b);
         }
         a.Kc = b.Kc;
         a.rec = b.rec;
@@ -1848,10 +1841,10 @@ static int build_dmap(Ctx* c, const std::vector<PairSpec>& ps, int64_t nrow, int
 template <int ND>
 static void launch_direct_beam(bool u, dim3 grv, dim3 gr, hipStream_t s, const BeamDynArgs& b, const DirectArgs& a) {
     if (u) {
-        hipLaunchKernelGGL((beam_dyn_value_kernel<ND, true>), grv, dim3(kBeamBlock), 0, s, b);
+        hipLaunchKernelGGL((beam_dyn_value_kernel<ND, true>), grv, dim3(kValueBlock), 0, s, b);
         hipLaunchKernelGGL((beam_direct_kernel<ND, true>), gr, dim3(kDirLanes), 0, s, a);
     } else {
-        hipLaunchKernelGGL((beam_dyn_value_kernel<ND, false>), grv, dim3(kBeamBlock), 0, s, b);
+        hipLaunchKernelGGL((beam_dyn_value_kernel<ND, false>), grv, dim3(kValueBlock), 0, s, b);
         hipLaunchKernelGGL((beam_direct_kernel<ND, false>), gr, dim3(kDirLanes), 0, s, a);
     }
 }
@@ -1889,7 +1882,7 @@ static int launch_direct(Ctx* c, const Group& g, int nd, double dt, unsigned lon
         b.Kc = c->d_Kc + g.kcbase; b.K = nullptr; b.R = c->d_Rd + g.rbase; b.dR = nullptr;
         b.rec = c->d_rec + g.recbase;
         b.flag = c->d_flag; b.gtag = gtag;
-        const int64_t ntile = (g.nele + kBeamBlock - 1) / kBeamBlock;
+        const int64_t ntile = (g.nele + kValueBlock - 1) / kValueBlock;
         b.per_xcd = (ntile + kXCD - 1) / kXCD;
         const dim3 grv((unsigned)(b.per_xcd * kXCD));
         a.Kc = b.Kc;
