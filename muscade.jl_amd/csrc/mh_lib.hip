@@ -80,6 +80,16 @@ struct DMap {
     uint32_t* srcT = nullptr;
 };
 
+// The nz scatter's map of nodes whose six dof columns hold whole 6×6 blocks of beam contributions
+// (build_node_map). Per block: the nz of its first entry, the column length | sources << 16, where its
+// sources start in src, and the first of them. rest: every other nz.
+struct NodeMap {
+    int64_t nblock = 0, nrest = 0;
+    int4* blk = nullptr;
+    int32_t* rest = nullptr;
+    uint32_t* src = nullptr;
+};
+
 struct Ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -145,6 +155,8 @@ struct Ctx {
     double* d_dL1 = nullptr;     // 2·nX: L1[Λ][1], L1[X][1]
     double* d_dL2 = nullptr;     // 2(OX+1)·nnz(XX) + 2·nnz(XU): L2[Λ,X][1,d], L2[X,Λ][d,1], L2[Λ,U][1,1], L2[U,Λ][1,1]
     int scatter_variant = 0;     // nz scatter shape picked at prepare (launch_scatter)
+    NodeMap nmap;                // the nz scatter by nodes, used while use_nodes
+    bool use_nodes = false;
     int beam_variant = 1;        // static beam kernel shape picked by tune_beams (launch_beam_static)
     float beam_ms[3] = {0.f, 0.f, 0.f};
     bool beam_tuned = false;
@@ -259,6 +271,8 @@ void free_prepared(Ctx* c) {
     free_big(c);
     dfree(c->d_Kbuf); dfree(c->d_Rbuf); dfree(c->d_dRbuf); dfree(c->d_nzval); dfree(c->d_rhs); dfree(c->d_Kc); dfree(c->d_rec);
     dfree(c->d_colptr); dfree(c->d_rowval); dfree(c->d_kseg); dfree(c->d_ksrc); dfree(c->d_rseg); dfree(c->d_rsrc);
+    dfree(c->nmap.blk); dfree(c->nmap.rest); dfree(c->nmap.src);
+    c->nmap = NodeMap(); c->use_nodes = false;
     dfree(c->d_useg); dfree(c->d_usrc); dfree(c->d_gbuf); dfree(c->d_gX); dfree(c->d_gubuf); dfree(c->d_gU);
     dfree(c->d_aseg); dfree(c->d_asrc); dfree(c->d_gabuf); dfree(c->d_gA); dfree(c->d_crhs);
     dfree(c->d_spi); dfree(c->d_spv); c->sp_cap = 0;
@@ -1244,6 +1258,9 @@ __global__ __launch_bounds__(kBlock) void point_direct_kernel(DirectArgs a, int 
 
 // Contribution source: (code << 29) | index; the code selects an exact multiplier.
 constexpr uint32_t kIdxMask = (1u << 29) - 1;
+__host__ __device__ inline uint32_t multiplier_code(double m) {
+    return m == 1. ? 0u : m == -1. ? 1u : m == 0.5 ? 2u : m == -0.5 ? 3u : m == 0.25 ? 4u : 5u;
+}
 __device__ __forceinline__ double contrib(const double* __restrict__ buf, uint32_t s) {
     const double v = buf[s & kIdxMask];
     switch (s >> 29) {
@@ -1363,6 +1380,160 @@ void launch_scatter(int variant, hipStream_t s, int64_t nseg, const int32_t* seg
     else launch_scatter_shape<CODED, false>(variant, s, nseg, seg, src, buf, out, nullptr);
 }
 
+// ---- the nz scatter by nodes -------------------------------------------------
+// The six columns of a node whose elements are beams hold whole 6×6 blocks: one per neighbour and
+// the node's own. A block's 36 entries come from the same elements, 6×6 of their 12×12 each, so one index
+// per element and block stands for 36 sources and 36 segment starts. Blocks are numbered in the order
+// of their nz. A wave takes ten: lane 6b + r owns row r of block b and walks the six columns. Each nz is
+// summed in the same element order as in scatter_kernel. The nz of all other columns (Holds, loads,
+// nodes of other kinds) follow in the same launch, a lane each.
+// Bound: HBM. The index traffic falls from 8 B a nz to 16 B a block; stores go through L2, where the
+// rows of a line meet (written past it they cost 244 µs instead of 180). 383,000 beams in chains: 237 µs
+// for the best segmented shape, 180 here.
+constexpr int kNodeWaves = 4, kWaveBlocks = 10;
+constexpr int kNodeUnits = 4;   // tens of blocks a wave takes one after another
+struct NodeArgs {
+    NodeMap m;
+    int64_t per_xcd, ntile;   // ntile: tiles of blocks; tiles of `rest` follow
+    int units;
+    const int32_t* seg;
+    const uint32_t* src;
+    const double* K;
+    double* out;
+    const int32_t* dst;
+};
+template <bool IDX>
+__global__ __launch_bounds__(64 * kNodeWaves) void node_scatter_kernel(NodeArgs a) {
+    const int64_t tile = xcd_tile(a.per_xcd);
+    const int t = threadIdx.x;
+    auto put = [&](int64_t k, double v) {
+        const int64_t o = IDX ? (int64_t)__builtin_nontemporal_load(a.dst + k) : k;
+        a.out[o] = v;
+    };
+    if (tile >= a.ntile) {
+        const int64_t q = (tile - a.ntile) * (64 * kNodeWaves) + t;
+        if (q >= a.m.nrest) return;
+        const int64_t k = a.m.rest[q];
+        double v = 0.;
+        for (int32_t p = a.seg[k], e = a.seg[k + 1]; p < e; ++p) v += a.K[a.src[p]];
+        put(k, v);
+        return;
+    }
+    const int l = t & 63, w = t >> 6, r = l % 6;
+    if (l >= 6 * kWaveBlocks) return;   // no barrier below
+    for (int u = 0; u < a.units; ++u) {
+        const int64_t b = ((tile * kNodeWaves + w) * a.units + u) * kWaveBlocks + l / 6;
+        if (b >= a.m.nblock) return;
+        const int4 h = a.m.blk[b];
+        const int n = h.y >> 16;
+        double v[6];
+#pragma unroll
+        for (int c = 0; c < 6; ++c) v[c] = 0.;
+        for (int j = 0; j < n; ++j) {
+            const double* k = a.K + (uint32_t)(j == 0 ? h.w : (int)a.m.src[h.z + j]) + r;
+#pragma unroll
+            for (int c = 0; c < 6; ++c) v[c] += k[12 * c];
+        }
+#pragma unroll
+        for (int c = 0; c < 6; ++c) put((int64_t)h.x + r + c * (h.y & 0xffff), v[c]);
+    }
+}
+void launch_node_scatter(const NodeMap& m, hipStream_t s, const int32_t* seg, const uint32_t* src, const double* K,
+                         double* out, const int32_t* dst) {
+    NodeArgs a;
+    a.m = m; a.seg = seg; a.src = src; a.K = K; a.out = out; a.dst = dst;
+    a.units = m.nblock >= (int64_t)2048 * kNodeWaves * kNodeUnits * kWaveBlocks ? kNodeUnits : 1;   // two workgroups a SIMD stay
+    const int64_t per = (int64_t)kNodeWaves * a.units * kWaveBlocks;
+    a.ntile = (m.nblock + per - 1) / per;
+    const int64_t nt = a.ntile + (m.nrest + 64 * kNodeWaves - 1) / (64 * kNodeWaves);
+    a.per_xcd = (nt + kXCD - 1) / kXCD;
+    const dim3 gr((unsigned)(a.per_xcd * kXCD)), bl(64 * kNodeWaves);
+    if (dst) hipLaunchKernelGGL((node_scatter_kernel<true>), gr, bl, 0, s, a);
+    else hipLaunchKernelGGL((node_scatter_kernel<false>), gr, bl, 0, s, a);
+}
+
+// Prepare: bit 0 of f[J] where J is the first of a beam node's six dofs, bit 1 where a beam's dofs are
+// not consecutive.
+__global__ __launch_bounds__(kBlock) void node_base_kernel(int64_t nele, const int32_t* __restrict__ idx, int32_t* __restrict__ f) {
+    const int64_t e = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (e >= nele) return;
+    for (int h = 0; h < 2; ++h) {
+        const int32_t J = idx[(int64_t)6 * h * nele + e];
+        bool ok = true;
+        for (int k = 1; k < 6; ++k) ok = ok && idx[(int64_t)(6 * h + k) * nele + e] == J + k;
+        atomicOr(f + J, 1);
+        if (!ok)
+            for (int k = 0; k < 6; ++k) atomicOr(f + idx[(int64_t)(6 * h + k) * nele + e], 2);
+    }
+}
+// Whether J is the base of a node whose columns are whole blocks, every source where block_source
+// says; its blocks and sources counted. dp: the block of rows J.
+__device__ inline bool node_check(int64_t J, int64_t nX, const int32_t* __restrict__ f, const int32_t* __restrict__ colptr,
+                                  const int32_t* __restrict__ rowval, const int32_t* __restrict__ seg,
+                                  const uint32_t* __restrict__ src, int& m, int& ns, int& dp) {
+    if (J + 6 > nX || f[J] != 1) return false;
+    for (int k = 1; k < 6; ++k) if (f[J + k] != 0) return false;
+    const int32_t k0 = colptr[J], len = colptr[J + 1] - k0;
+    if (len % 6 != 0 || len == 0 || len > 6 * 64) return false;
+    m = len / 6; ns = 0; dp = -1;
+    for (int c = 1; c < 6; ++c) if (colptr[J + c + 1] - colptr[J + c] != len) return false;
+    for (int b = 0; b < m; ++b) {
+        const int32_t I = rowval[k0 + 6 * b], k00 = k0 + 6 * b;
+        if (I == J) dp = b;
+        const int nc = seg[k00 + 1] - seg[k00];
+        if (nc < 1 || nc > 0x7fff) return false;
+        ns += nc;
+        for (int c = 0; c < 6; ++c)
+            for (int r = 0; r < 6; ++r) {
+                const int32_t k = k00 + c * len + r;
+                if (rowval[k] != I + r || seg[k + 1] - seg[k] != nc) return false;
+            }
+        for (int j = 0; j < nc; ++j)   // element j's entries at their places in its 12×12
+            for (int c = 0; c < 6; ++c)
+                for (int r = 0; r < 6; ++r)
+                    if (src[seg[k00 + c * len + r] + j] != src[seg[k00] + j] + (uint32_t)(r + 12 * c)) return false;
+    }
+    return dp >= 0;
+}
+// cnt: 4 × (nX + 1): node, blocks, sources, other nz of each column.
+__global__ __launch_bounds__(kBlock) void node_count_kernel(int64_t nX, const int32_t* __restrict__ f, const int32_t* __restrict__ colptr,
+                                                            const int32_t* __restrict__ rowval, const int32_t* __restrict__ seg,
+                                                            const uint32_t* __restrict__ src, int32_t* __restrict__ cnt) {
+    const int64_t J = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (J > nX) return;
+    int m = 0, ns = 0, dp = 0;
+    const bool ok = J < nX && node_check(J, nX, f, colptr, rowval, seg, src, m, ns, dp);
+    const int64_t n1 = nX + 1;
+    cnt[J] = ok; cnt[n1 + J] = ok ? m : 0; cnt[2 * n1 + J] = ok ? ns : 0;
+}
+__global__ __launch_bounds__(kBlock) void node_rest_kernel(int64_t nX, const int32_t* __restrict__ ok, const int32_t* __restrict__ colptr,
+                                                           int32_t* __restrict__ rest) {
+    const int64_t J = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (J > nX) return;
+    bool in = J == nX;
+    for (int k = 0; k < 6; ++k) in = in || (J >= k && ok[J - k]);
+    rest[J] = in ? 0 : colptr[J + 1] - colptr[J];
+}
+// pos: the exclusive sums of cnt.
+__global__ __launch_bounds__(kBlock) void node_fill_kernel(int64_t nX, const int32_t* __restrict__ cnt, const int32_t* __restrict__ pos,
+                                                           const int32_t* __restrict__ colptr, const int32_t* __restrict__ rowval,
+                                                           const int32_t* __restrict__ seg, const uint32_t* __restrict__ src, NodeMap o) {
+    const int64_t J = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (J > nX) return;
+    const int64_t n1 = nX + 1;
+    if (J == nX) return;
+    if (cnt[J]) {
+        const int32_t b0 = pos[n1 + J], k0 = colptr[J], len = colptr[J + 1] - k0;
+        int32_t p = pos[2 * n1 + J];
+        for (int b = 0; b < len / 6; ++b) {
+            const int32_t k00 = k0 + 6 * b, nc = seg[k00 + 1] - seg[k00];
+            o.blk[b0 + b] = make_int4(k00, len | nc << 16, p, (int)src[seg[k00]]);
+            for (int j = 0; j < nc; ++j) o.src[p++] = src[seg[k00] + j];
+        }
+    }
+    for (int32_t i = 0; i < cnt[3 * n1 + J]; ++i) o.rest[pos[3 * n1 + J] + i] = colptr[J] + i;
+}
+
 // Long segments (many elements share a dof, e.g. a U-node loading a whole stretch of
 // beams): one workgroup per segment. Lane t sums a contiguous sub-range sequentially, then
 // lane 0 adds the kTile partials in lane order — a fixed, deterministic order.
@@ -1426,8 +1597,7 @@ __global__ __launch_bounds__(kBlock) void gen_pairs_kernel(int64_t nele, int nX,
     if (compact) {
         double m;
         const int slot = mh::compact_slot(i, j, &m);
-        const uint32_t code = m == 1. ? 0u : m == -1. ? 1u : m == 0.5 ? 2u : m == -0.5 ? 3u : m == 0.25 ? 4u : 5u;
-        vals[q] = (code << 29) | (uint32_t)(kbase + e * mh::kCompact + slot);
+        vals[q] = (multiplier_code(m) << 29) | (uint32_t)(kbase + e * mh::kCompact + slot);
     } else {
         vals[q] = (uint32_t)(kbase + e * per + i + (int64_t)nX * j);
     }
@@ -1726,6 +1896,47 @@ static int upload_soa(Ctx* c, T** dst, const T* src, int n, int64_t nele) {
 
 // The rhs map (asm[1] for the X dofs): contributions of every element dof into Lλ, in
 // traversal order, stably sorted by dof (Assemble.jl:340-357 with add_value!'s order).
+// The node map of the prepared nz maps (nmap.nblock = 0 when no beam node has whole-block columns).
+static int build_node_map(Ctx* c) {
+    hipStream_t s = c->stream;
+    const int64_t nX = c->nX, n1 = nX + 1;
+    NodeMap& m = c->nmap;
+    int32_t *f = nullptr, *cnt = nullptr, *pos = nullptr;
+    HIPCHK(c, hipMalloc(&f, sizeof(int32_t) * n1));
+    HIPCHK(c, hipMalloc(&cnt, sizeof(int32_t) * 4 * n1));
+    HIPCHK(c, hipMalloc(&pos, sizeof(int32_t) * 4 * n1));
+    HIPCHK(c, hipMemsetAsync(f, 0, sizeof(int32_t) * n1, s));
+    for (auto& g : c->groups)
+        if ((g.kind == MH_KIND_BEAM || g.kind == MH_KIND_BEAM_U) && g.nele)
+            hipLaunchKernelGGL(node_base_kernel, dim3(grid(g.nele)), dim3(kBlock), 0, s, g.nele, g.d_idx, f);
+    hipLaunchKernelGGL(node_count_kernel, dim3(grid(n1)), dim3(kBlock), 0, s, nX, f, c->d_colptr, c->d_rowval,
+                       c->d_kseg, c->d_ksrc, cnt);
+    hipLaunchKernelGGL(node_rest_kernel, dim3(grid(n1)), dim3(kBlock), 0, s, nX, cnt, c->d_colptr, cnt + 3 * n1);
+    size_t tb = 0;
+    void* tmp = nullptr;
+    HIPCHK(c, hipcub::DeviceScan::ExclusiveSum(nullptr, tb, cnt, pos, (int)n1, s));
+    HIPCHK(c, hipMalloc(&tmp, std::max<size_t>(tb, 1)));
+    int32_t tot[4];
+    for (int k = 0; k < 4; ++k) {
+        HIPCHK(c, hipcub::DeviceScan::ExclusiveSum(tmp, tb, cnt + k * n1, pos + k * n1, (int)n1, s));
+        HIPCHK(c, hipMemcpyAsync(&tot[k], pos + k * n1 + nX, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+    }
+    HIPCHK(c, hipStreamSynchronize(s));
+    dfree(tmp);
+    if (tot[0] > 0) {
+        m.nblock = tot[1]; m.nrest = tot[3];
+        HIPCHK(c, hipMalloc(&m.blk, sizeof(int4) * tot[1]));
+        HIPCHK(c, hipMalloc(&m.src, sizeof(uint32_t) * std::max(tot[2], 1)));
+        HIPCHK(c, hipMalloc(&m.rest, sizeof(int32_t) * std::max(tot[3], 1)));
+        hipLaunchKernelGGL(node_fill_kernel, dim3(grid(n1)), dim3(kBlock), 0, s, nX, cnt, pos, c->d_colptr, c->d_rowval,
+                           c->d_kseg, c->d_ksrc, m);
+    }
+    if (int r = check_launch(c, "node map")) return r;
+    HIPCHK(c, hipStreamSynchronize(s));
+    dfree(f); dfree(cnt); dfree(pos);
+    return MH_OK;
+}
+
 static int build_rmap(Ctx* c) {
     hipStream_t s = c->stream;
     const int64_t nR = c->nR, nX = c->nX;
@@ -2276,6 +2487,14 @@ int mh_prepare_sweepx(mh_ctx* c, int OX, int64_t* nnz_out) {
             if (tmin < best) { best = tmin; c->scatter_variant = v; }
         }
     }
+    // The scatter by nodes, where it covers at least half of the nz (its other nz are searched one by one)
+    // and the elements' matrices are whole: 180 µs against 237 for the best segmented shape (383,000
+    // beams in chains). From compact matrices it is the slower one (553 µs against 513, 973,000 beams
+    // of a lattice): a row's entries lie in 18 places of 360 B.
+    if (nnz > 0 && !coded) {
+        if (int r = build_node_map(c)) return r;
+        c->use_nodes = c->nmap.nblock > 0 && 2 * c->nmap.nrest <= nnz;
+    }
     c->beam_tuned = false;
     c->prepared = true;
     if (nnz_out) *nnz_out = nnz;
@@ -2439,7 +2658,9 @@ static int enqueue_sweepx(Ctx* c, int OX, bool step, const double* c6, bool time
             out = c->d_cbuf;
             dst = c->d_cslot;
         }
-        if (c->coded) launch_scatter<true>(c->scatter_variant, s, c->nnz, c->d_kseg, c->d_ksrc, c->d_Kbuf, out, dst);
+        if (c->use_nodes) {
+            launch_node_scatter(c->nmap, s, c->d_kseg, c->d_ksrc, c->d_Kbuf, out, dst);
+        } else if (c->coded) launch_scatter<true>(c->scatter_variant, s, c->nnz, c->d_kseg, c->d_ksrc, c->d_Kbuf, out, dst);
         else launch_scatter<false>(c->scatter_variant, s, c->nnz, c->d_kseg, c->d_ksrc, c->d_Kbuf, out, dst);
     }
     if (timed) HIPCHK(c, hipEventRecord(c->ev[2], s));
@@ -2741,6 +2962,7 @@ int mh_calib_copy(mh_ctx* c, int64_t n, double* ms) {
 int mh_set_scatter_variant(mh_ctx* c, int variant) {
     if (!c || !c->prepared || variant < 0 || variant >= kScatterVariants) return MH_ERR_ARG;
     c->scatter_variant = variant;
+    c->use_nodes = false;   // the shape asked for, not the scatter by nodes
     ++c->gen;   // a captured graph holds the old launch
     return MH_OK;
 }
