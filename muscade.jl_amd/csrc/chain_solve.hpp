@@ -64,17 +64,6 @@ __global__ __launch_bounds__(kCB) void fill_i32(int64_t n, int32_t* __restrict__
     if (i < n) p[i] = v;
 }
 
-// Identity rows of padding positions (their slots are uncovered, so zeroed before).
-template <int B>
-__global__ __launch_bounds__(kCB) void dummy_kernel(int64_t n, const int32_t* __restrict__ dpos, double* __restrict__ D,
-                                                    double* __restrict__ b) {
-    const int64_t q = (int64_t)blockIdx.x * kCB + threadIdx.x;
-    if (q >= n) return;
-    const int64_t p = dpos[q], blk = p / B, i = p - blk * B;
-    D[blk * B * B + i * B + i] = 1.0;
-    b[p] = 0.0;
-}
-
 // Prepare: one thread per column c of the CSC pattern. slot[k] of each nz k: ≥ 0, its index
 // in D|L|U; −(4p + w + 1), coupling w (0: cL, row λ col h; 1: cU, row h col λ; 2: the λ
 // diagonal) of λ pair p. unc[q] is cleared for every slot q that an nz covers.
@@ -162,15 +151,24 @@ __global__ __launch_bounds__(kCB) void pack_rhs_kernel(int64_t nX, const int32_t
     else pc[4 * (int64_t)(-p - 1) + 3] = rhs[d];
 }
 
-// One thread per λ pair: save row h (L | D | U parts and r_h), replace it by x_h = r_λ/cL.
+// One thread per λ pair: save row h (L | D | U parts and r_h), replace it by x_h = r_λ/cL. Then one
+// per padding position: its identity row (its slots are uncovered, so zeroed before).
 template <int B>
 __global__ __launch_bounds__(kCB) void pair_kernel(int64_t np, const int32_t* __restrict__ hpos,
                                                    const double* __restrict__ pc, double* __restrict__ D,
                                                    double* __restrict__ L, double* __restrict__ U,
                                                    double* __restrict__ b, double* __restrict__ saved,
-                                                   unsigned* __restrict__ flag) {
+                                                   unsigned* __restrict__ flag, int64_t ndum,
+                                                   const int32_t* __restrict__ dpos) {
     const int64_t p = (int64_t)blockIdx.x * kCB + threadIdx.x;
-    if (p >= np) return;
+    if (p >= np) {
+        if (p - np < ndum) {
+            const int64_t q = dpos[p - np], blk = q / B, i = q - blk * B;
+            D[blk * B * B + i * B + i] = 1.0;
+            b[q] = 0.0;
+        }
+        return;
+    }
     const double cL = pc[4 * p], cU = pc[4 * p + 1], dg = pc[4 * p + 2], rl = pc[4 * p + 3];
     if (dg != 0.0 || cL == 0.0 || cU == 0.0) {
         atomicOr(flag, kBadPair);
@@ -491,35 +489,41 @@ __global__ __launch_bounds__(kChunk* B) void back_kernel(System x, const double*
     if (i < cnt) x.b[(k0 + i) * B + r] = xs[i * B + r];
 }
 
-// Δx in dof order: x at the dof's position, or λ from the saved row of its held dof.
+// Δx of dof c: x at the dof's position, or λ from the saved row of its held dof.
+struct Unpack {
+    int64_t nb = 0;
+    const int32_t *pos = nullptr, *hpos = nullptr;
+    const double *pc = nullptr, *saved = nullptr, *x = nullptr;
+};
 template <int B>
-__global__ __launch_bounds__(kCB) void unpack_kernel(int64_t nX, int64_t nb, const int32_t* __restrict__ pos,
-                                                     const int32_t* __restrict__ hpos, const double* __restrict__ pc,
-                                                     const double* __restrict__ saved, const double* __restrict__ x,
-                                                     double* __restrict__ dx) {
-    const int64_t c = (int64_t)blockIdx.x * kCB + threadIdx.x;
-    if (c >= nX) return;
-    const int32_t pc_ = pos[c];
-    if (pc_ >= 0) { dx[c] = x[pc_]; return; }
+__device__ inline double unpack_dof(const Unpack& u, int64_t c) {
+    const int32_t pc_ = u.pos[c];
+    if (pc_ >= 0) return u.x[pc_];
     const int64_t p = -pc_ - 1;
-    const int64_t h = hpos[p], blk = h / B;
-    const double* sv = saved + p * (3 * B + 1);
+    const int64_t h = u.hpos[p], blk = h / B;
+    const double* sv = u.saved + p * (3 * B + 1);
     double r = sv[3 * B];
     if (blk > 0)
-        for (int k = 0; k < B; ++k) r -= sv[k] * x[(blk - 1) * B + k];
-    for (int k = 0; k < B; ++k) r -= sv[B + k] * x[blk * B + k];
-    if (blk + 1 < nb)
-        for (int k = 0; k < B; ++k) r -= sv[2 * B + k] * x[(blk + 1) * B + k];
-    dx[c] = r / pc[4 * p + 1];
+        for (int k = 0; k < B; ++k) r -= sv[k] * u.x[(blk - 1) * B + k];
+    for (int k = 0; k < B; ++k) r -= sv[B + k] * u.x[blk * B + k];
+    if (blk + 1 < u.nb)
+        for (int k = 0; k < B; ++k) r -= sv[2 * B + k] * u.x[(blk + 1) * B + k];
+    return r / u.pc[4 * p + 1];
+}
+template <int B>
+__global__ __launch_bounds__(kCB) void unpack_kernel(int64_t nX, Unpack u, double* __restrict__ dx) {
+    const int64_t c = (int64_t)blockIdx.x * kCB + threadIdx.x;
+    if (c < nX) dx[c] = unpack_dof<B>(u, c);
 }
 
 // Newmarkβdecrement!{OX} (src/SweepX.jl:98-132) over all X dofs, in the host's operation
 // order and without contraction, so that a given Δx decrements the state bitwise as the
 // host loop does; per-block partial sums of Δx² and Lλ².
 // k: the Newmark coefficients (a₁,a₂,a₃,b₁,b₂,b₃) in device memory, so that a captured graph
-// replays with the current ones.
+// replays with the current ones. B > 0: Δx is taken from the solve's blocks (and kept in dx).
+template <int B>
 __global__ __launch_bounds__(kCB) void newmark_kernel(int64_t nX, int OX, int first, const double* __restrict__ k,
-                                                      const double* __restrict__ dx, const double* __restrict__ rhs,
+                                                      Unpack u, double* __restrict__ dx, const double* __restrict__ rhs,
                                                       const double* __restrict__ scale, double* __restrict__ X0,
                                                       double* __restrict__ X1, double* __restrict__ X2,
                                                       double* __restrict__ part) {
@@ -529,7 +533,10 @@ __global__ __launch_bounds__(kCB) void newmark_kernel(int64_t nX, int OX, int fi
     const int64_t c = (int64_t)blockIdx.x * kCB + threadIdx.x;
     double q1 = 0.0, q2 = 0.0;
     if (c < nX) {
-        const double d = dx[c], sc = scale[c], r = rhs[c];
+        double d;
+        if constexpr (B > 0) dx[c] = d = unpack_dof<B>(u, c);
+        else d = dx[c];
+        const double sc = scale[c], r = rhs[c];
         q1 = d * d;
         q2 = r * r;
         if (OX == 2) {
@@ -569,9 +576,11 @@ __global__ __launch_bounds__(kCB) void newmark_kernel(int64_t nX, int OX, int fi
     }
     if (threadIdx.x == 0) { part[2 * blockIdx.x] = s1[0]; part[2 * blockIdx.x + 1] = s2[0]; }
 }
-// One workgroup: the partial sums in a fixed order (deterministic).
+// One workgroup: the partial sums in a fixed order (deterministic), and the solve's status words; both
+// to pinned host memory.
 __global__ __launch_bounds__(kCB) void norm_kernel(int64_t npart, const double* __restrict__ part,
-                                                   double* __restrict__ out) {
+                                                   double* __restrict__ out, const unsigned* __restrict__ status,
+                                                   unsigned* __restrict__ hstatus) {
     __shared__ double s1[kCB], s2[kCB];
     double q1 = 0.0, q2 = 0.0;
     for (int64_t k = threadIdx.x; k < npart; k += kCB) { q1 += part[2 * k]; q2 += part[2 * k + 1]; }
@@ -583,6 +592,7 @@ __global__ __launch_bounds__(kCB) void norm_kernel(int64_t npart, const double* 
         __syncthreads();
     }
     if (threadIdx.x == 0) { out[0] = s1[0]; out[1] = s2[0]; }
+    if (threadIdx.x < kStatusBytes / 4) hstatus[threadIdx.x] = status[threadIdx.x];
 }
 
 }  // namespace chain

@@ -90,6 +90,11 @@ struct NodeMap {
     uint32_t* src = nullptr;
 };
 
+// flag: the first NaN element; cflag, where: the chain solve's status words (chain::kStatusBytes).
+struct CallWords { double c6[6]; unsigned long long flag; unsigned cflag[2]; unsigned long long where[2]; };
+struct CallResults { unsigned long long flag; unsigned cflag[2]; unsigned long long where[2]; double norm[2]; };
+static_assert(sizeof(CallWords) == 80 && chain::kStatusBytes == 24, "status words follow the flag");
+
 struct Ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -108,8 +113,12 @@ struct Ctx {
     int64_t nK = 0, nP = 0, nR = 0, nnz = 0;
     double* d_Kc = nullptr;      // dynamic beams: scaled compact static part, 45 per element
     double* d_rec = nullptr;     // dynamic beams: the elements' records (mh::DynRec), in tiles of kDynTile
-    double* d_c6 = nullptr;      // SweepX: the Newmark coefficients of the current call (6)
-    double* h_c6 = nullptr;      // pinned staging of d_c6
+    // words of one call: uploaded in one copy ahead of its kernels (upload_call), and the results its
+    // last kernels leave in pinned host memory
+    CallWords* d_call = nullptr;
+    CallWords* h_call = nullptr;       // pinned staging
+    CallResults* h_res = nullptr;      // pinned
+    double* d_c6 = nullptr;            // d_call->c6
     double* d_Kbuf = nullptr;
     double* d_Rbuf = nullptr;
     double* d_dRbuf = nullptr;
@@ -121,8 +130,8 @@ struct Ctx {
     uint32_t* d_ksrc = nullptr;
     int32_t* d_rseg = nullptr;
     uint32_t* d_rsrc = nullptr;
-    unsigned long long* d_flag = nullptr;
-    unsigned long long* h_flag = nullptr;   // pinned host copy of d_flag (copied on the stream)
+    unsigned long long* d_flag = nullptr;   // d_call->flag
+    unsigned long long* h_flag = nullptr;   // h_res->flag
     void* d_scratch = nullptr;   // this device's address of the fixed `scratch` array (set at create)
     // adjoint (VJP) of the residual Lagrangian
     int64_t nRU = 0;             // per-element ∂L/∂U entries
@@ -190,12 +199,11 @@ struct Ctx {
     double* d_cred = nullptr;    // the block systems of the later phases of the reduction
     std::vector<chain::System> csys;   // one per phase; the first is d_cbuf
     double* d_dx = nullptr;      // nX: Δx of the last solve
-    unsigned* d_cflag = nullptr;
-    unsigned* h_cflag = nullptr; // pinned
+    unsigned* d_cflag = nullptr; // d_call->cflag
+    unsigned* h_cflag = nullptr; // h_res->cflag
     double* d_scaleX = nullptr;  // nX: dof scales (mh_newton_prepare)
     double* d_part = nullptr;    // 2 × workgroups of newmark_kernel
-    double* d_norm = nullptr;
-    double* h_norm = nullptr;    // pinned: Σ Δx², Σ Lλ²
+    double* h_norm = nullptr;    // h_res->norm: Σ Δx², Σ Lλ²
     hipEvent_t cev[4] = {nullptr, nullptr, nullptr, nullptr};
     // DirectXUA's all-steps system assembled on the device (mh_big_prepare / mh_big_assemble)
     int64_t bnv = 0, bnp = 0, bnnz = 0, bnhost = 0, bndev = 0;
@@ -248,8 +256,6 @@ void free_graph(Ctx* c) { for (int k = 0; k < 4; ++k) free_graph(c, k); }
 void free_chain(Ctx* c) {
     dfree(c->d_cpos); dfree(c->d_chpos); dfree(c->d_cdum); dfree(c->d_cbuf); dfree(c->d_csaved); dfree(c->d_dx);
     dfree(c->d_cslot); dfree(c->d_cunc); dfree(c->d_cred); c->csys.clear(); c->cnu = 0;
-    dfree(c->d_cflag);
-    if (c->h_cflag) { (void)hipHostFree(c->h_cflag); c->h_cflag = nullptr; }
     for (auto& e : c->cev) if (e) { (void)hipEventDestroy(e); e = nullptr; }
     c->cB = 0; c->cnb = c->cnp = c->cnd = 0;
 }
@@ -296,8 +302,7 @@ void free_model(Ctx* c) {
     dfree(c->d_xyz);
     for (auto& x : c->d_X) dfree(x);
     dfree(c->d_U); dfree(c->d_A); dfree(c->d_lam);
-    dfree(c->d_scaleX); dfree(c->d_part); dfree(c->d_norm);
-    if (c->h_norm) { (void)hipHostFree(c->h_norm); c->h_norm = nullptr; }
+    dfree(c->d_scaleX); dfree(c->d_part);
 }
 
 // ------------------------------------------------------------------ kernels
@@ -446,14 +451,22 @@ __device__ __forceinline__ void point_element(const PointArgs& a, int64_t e) {
 // Up to kPointBatch point groups in one launch (they are small; one launch each would
 // cost more than their work). Thread q runs element q - start[g] of group g.
 constexpr int kPointBatch = 12;
+// Clears ahead of an assembly into the chain solve's blocks: the λ couplings and the slots no nz covers.
+struct ChainClear { int64_t npc = 0, nslot = 0; double* pc = nullptr; const int32_t* slot = nullptr; double* D = nullptr; };
 struct PointBatch {
     int ngroup;
     int64_t start[kPointBatch + 1];
     PointArgs g[kPointBatch];
+    ChainClear clear;   // after the elements, a thread each
 };
 __global__ __launch_bounds__(kBlock) void point_kernel(PointBatch b) {
     const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= b.start[b.ngroup]) return;
+    if (q >= b.start[b.ngroup]) {
+        const int64_t z = q - b.start[b.ngroup];
+        if (z < b.clear.npc) b.clear.pc[z] = 0.0;
+        else if (z - b.clear.npc < b.clear.nslot) b.clear.D[b.clear.slot[z - b.clear.npc]] = 0.0;
+        return;
+    }
     int gi = 0;
     while (q >= b.start[gi + 1]) ++gi;
     point_element(b.g[gi], q - b.start[gi]);
@@ -1278,8 +1291,6 @@ __device__ __forceinline__ double contrib(const double* __restrict__ buf, uint32
 // the whole workgroup loads them (coalesced indices, every lane gathering) into LDS in
 // chunks, then each lane sums its own segment sequentially from LDS. Lanes of long and
 // short segments therefore share the memory work evenly.
-// STEP (rhs of the :step mission): each contribution adds R then subtracts ∂R/∂δr
-// (add_value! then add_∂!{1,:minus}, src/SweepX.jl:56-57).
 constexpr int kTile = 256;
 constexpr int kChunk = 1024;
 // CODED: src carries multiplier codes (compact static beams); otherwise src is the
@@ -1288,13 +1299,12 @@ constexpr int kChunk = 1024;
 // prepare-time tuner picks (scatter_variant).
 // IDX: segment k is written to out[dst[k]] instead of out[k] (the nz straight into the
 // chain solve's blocks).
-template <bool STEP, bool CODED, int SPL = 1, int CH = kChunk, bool NTM = false, bool IDX = false>
+template <bool CODED, int SPL = 1, int CH = kChunk, bool NTM = false, bool IDX = false>
 __global__ __launch_bounds__(kTile) void scatter_kernel(int64_t nseg, int64_t per_xcd, const int32_t* __restrict__ seg,
                                                         const uint32_t* __restrict__ src, const double* __restrict__ buf,
-                                                        const double* __restrict__ dbuf, double* __restrict__ out,
+                                                        double* __restrict__ out,
                                                         const int32_t* __restrict__ dst = nullptr) {
     __shared__ double vals[CH];
-    __shared__ double dvals[STEP ? CH : 1];
     constexpr int kSeg = kTile * SPL;
     const int64_t k0 = xcd_tile(per_xcd) * kSeg;
     if (k0 >= nseg) return;   // the whole workgroup leaves together
@@ -1318,16 +1328,12 @@ __global__ __launch_bounds__(kTile) void scatter_kernel(int64_t nseg, int64_t pe
         for (int32_t q = c + t; q < cend; q += kTile) {
             const uint32_t sq = NTM ? __builtin_nontemporal_load(src + q) : src[q];
             vals[q - c] = CODED ? contrib(buf, sq) : buf[sq];
-            if (STEP) dvals[q - c] = dbuf[CODED ? (sq & kIdxMask) : sq];
         }
         __syncthreads();
 #pragma unroll
         for (int j = 0; j < SPL; ++j) {
             const int32_t a = p0[j] > c ? p0[j] : c, b = p1[j] < cend ? p1[j] : cend;
-            for (int32_t q = a; q < b; ++q) {
-                acc[j] += vals[q - c];
-                if (STEP) acc[j] -= dvals[q - c];
-            }
+            for (int32_t q = a; q < b; ++q) acc[j] += vals[q - c];
         }
         __syncthreads();
     }
@@ -1352,24 +1358,23 @@ void launch_scatter_shape(int variant, hipStream_t s, int64_t nseg, const int32_
     const int spl = kScatterSPL[variant];
     const int64_t per = ((nseg + kTile * spl - 1) / (kTile * spl) + kXCD - 1) / kXCD;
     const dim3 gr((unsigned)(per * kXCD));
-    const double* nul = nullptr;
     switch (variant) {
-    case 0: hipLaunchKernelGGL((scatter_kernel<false, CODED, 1, 1024, false, IDX>), gr, dim3(kTile), 0, s, nseg, per, seg, src, buf, nul, out, dst); break;
-    case 1: hipLaunchKernelGGL((scatter_kernel<false, CODED, 2, 1024, false, IDX>), gr, dim3(kTile), 0, s, nseg, per, seg, src, buf, nul, out, dst); break;
-    case 2: hipLaunchKernelGGL((scatter_kernel<false, CODED, 2, 2048, false, IDX>), gr, dim3(kTile), 0, s, nseg, per, seg, src, buf, nul, out, dst); break;
-    case 3: hipLaunchKernelGGL((scatter_kernel<false, CODED, 3, 2048, false, IDX>), gr, dim3(kTile), 0, s, nseg, per, seg, src, buf, nul, out, dst); break;
-    case 4: hipLaunchKernelGGL((scatter_kernel<false, CODED, 4, 1024, false, IDX>), gr, dim3(kTile), 0, s, nseg, per, seg, src, buf, nul, out, dst); break;
-    case 5: hipLaunchKernelGGL((scatter_kernel<false, CODED, 4, 2048, false, IDX>), gr, dim3(kTile), 0, s, nseg, per, seg, src, buf, nul, out, dst); break;
-    case 6: hipLaunchKernelGGL((scatter_kernel<false, CODED, 6, 2048, false, IDX>), gr, dim3(kTile), 0, s, nseg, per, seg, src, buf, nul, out, dst); break;
-    case 7: hipLaunchKernelGGL((scatter_kernel<false, CODED, 8, 2048, false, IDX>), gr, dim3(kTile), 0, s, nseg, per, seg, src, buf, nul, out, dst); break;
-    case 8: hipLaunchKernelGGL((scatter_kernel<false, CODED, 1, 1024, true, IDX>), gr, dim3(kTile), 0, s, nseg, per, seg, src, buf, nul, out, dst); break;
-    case 9: hipLaunchKernelGGL((scatter_kernel<false, CODED, 2, 1024, true, IDX>), gr, dim3(kTile), 0, s, nseg, per, seg, src, buf, nul, out, dst); break;
-    case 10: hipLaunchKernelGGL((scatter_kernel<false, CODED, 2, 2048, true, IDX>), gr, dim3(kTile), 0, s, nseg, per, seg, src, buf, nul, out, dst); break;
-    case 11: hipLaunchKernelGGL((scatter_kernel<false, CODED, 3, 2048, true, IDX>), gr, dim3(kTile), 0, s, nseg, per, seg, src, buf, nul, out, dst); break;
-    case 12: hipLaunchKernelGGL((scatter_kernel<false, CODED, 4, 1024, true, IDX>), gr, dim3(kTile), 0, s, nseg, per, seg, src, buf, nul, out, dst); break;
-    case 13: hipLaunchKernelGGL((scatter_kernel<false, CODED, 4, 2048, true, IDX>), gr, dim3(kTile), 0, s, nseg, per, seg, src, buf, nul, out, dst); break;
-    case 14: hipLaunchKernelGGL((scatter_kernel<false, CODED, 6, 2048, true, IDX>), gr, dim3(kTile), 0, s, nseg, per, seg, src, buf, nul, out, dst); break;
-    default: hipLaunchKernelGGL((scatter_kernel<false, CODED, 8, 2048, true, IDX>), gr, dim3(kTile), 0, s, nseg, per, seg, src, buf, nul, out, dst); break;
+    case 0: hipLaunchKernelGGL((scatter_kernel<CODED, 1, 1024, false, IDX>), gr, dim3(kTile), 0, s, nseg, per, seg, src, buf, out, dst); break;
+    case 1: hipLaunchKernelGGL((scatter_kernel<CODED, 2, 1024, false, IDX>), gr, dim3(kTile), 0, s, nseg, per, seg, src, buf, out, dst); break;
+    case 2: hipLaunchKernelGGL((scatter_kernel<CODED, 2, 2048, false, IDX>), gr, dim3(kTile), 0, s, nseg, per, seg, src, buf, out, dst); break;
+    case 3: hipLaunchKernelGGL((scatter_kernel<CODED, 3, 2048, false, IDX>), gr, dim3(kTile), 0, s, nseg, per, seg, src, buf, out, dst); break;
+    case 4: hipLaunchKernelGGL((scatter_kernel<CODED, 4, 1024, false, IDX>), gr, dim3(kTile), 0, s, nseg, per, seg, src, buf, out, dst); break;
+    case 5: hipLaunchKernelGGL((scatter_kernel<CODED, 4, 2048, false, IDX>), gr, dim3(kTile), 0, s, nseg, per, seg, src, buf, out, dst); break;
+    case 6: hipLaunchKernelGGL((scatter_kernel<CODED, 6, 2048, false, IDX>), gr, dim3(kTile), 0, s, nseg, per, seg, src, buf, out, dst); break;
+    case 7: hipLaunchKernelGGL((scatter_kernel<CODED, 8, 2048, false, IDX>), gr, dim3(kTile), 0, s, nseg, per, seg, src, buf, out, dst); break;
+    case 8: hipLaunchKernelGGL((scatter_kernel<CODED, 1, 1024, true, IDX>), gr, dim3(kTile), 0, s, nseg, per, seg, src, buf, out, dst); break;
+    case 9: hipLaunchKernelGGL((scatter_kernel<CODED, 2, 1024, true, IDX>), gr, dim3(kTile), 0, s, nseg, per, seg, src, buf, out, dst); break;
+    case 10: hipLaunchKernelGGL((scatter_kernel<CODED, 2, 2048, true, IDX>), gr, dim3(kTile), 0, s, nseg, per, seg, src, buf, out, dst); break;
+    case 11: hipLaunchKernelGGL((scatter_kernel<CODED, 3, 2048, true, IDX>), gr, dim3(kTile), 0, s, nseg, per, seg, src, buf, out, dst); break;
+    case 12: hipLaunchKernelGGL((scatter_kernel<CODED, 4, 1024, true, IDX>), gr, dim3(kTile), 0, s, nseg, per, seg, src, buf, out, dst); break;
+    case 13: hipLaunchKernelGGL((scatter_kernel<CODED, 4, 2048, true, IDX>), gr, dim3(kTile), 0, s, nseg, per, seg, src, buf, out, dst); break;
+    case 14: hipLaunchKernelGGL((scatter_kernel<CODED, 6, 2048, true, IDX>), gr, dim3(kTile), 0, s, nseg, per, seg, src, buf, out, dst); break;
+    default: hipLaunchKernelGGL((scatter_kernel<CODED, 8, 2048, true, IDX>), gr, dim3(kTile), 0, s, nseg, per, seg, src, buf, out, dst); break;
     }
 }
 // Launch one of the tuned shapes of the nz scatter; dst (optional): write segment k to out[dst[k]].
@@ -1379,6 +1384,40 @@ void launch_scatter(int variant, hipStream_t s, int64_t nseg, const int32_t* seg
     if (dst) launch_scatter_shape<CODED, true>(variant, s, nseg, seg, src, buf, out, dst);
     else launch_scatter_shape<CODED, false>(variant, s, nseg, seg, src, buf, out, nullptr);
 }
+
+// The rhs: out[d] = Σ R[src[p]] (− dR[src[p]] after each, on :step: add_value! then
+// add_∂!{1,:minus}, src/SweepX.jl:56-57), a lane per dof in the order of
+// scatter_kernel, and, for the chain solve (pos), also into its right-hand side b or its λ pairs. The
+// first lane hands the NaN flag (the element kernels are done) to the host.
+struct RhsArgs {
+    int64_t n = 0;
+    const int32_t* seg = nullptr;
+    const uint32_t* src = nullptr;
+    const double* R = nullptr;
+    const double* dR = nullptr;
+    double* out = nullptr;
+    const int32_t* pos = nullptr;
+    double *b = nullptr, *pc = nullptr;
+    const unsigned long long* flag = nullptr;
+    unsigned long long* hflag = nullptr;
+};
+__device__ __forceinline__ void rhs_dof(const RhsArgs& a, int64_t d) {
+    if (d == 0 && a.hflag) *a.hflag = *a.flag;
+    if (d >= a.n) return;
+    double v = 0.;
+    for (int32_t p = a.seg[d], e = a.seg[d + 1]; p < e; ++p) {
+        const uint32_t q = a.src[p];
+        v += a.R[q];
+        if (a.dR) v -= a.dR[q];
+    }
+    a.out[d] = v;
+    if (a.pos) {
+        const int32_t p = a.pos[d];
+        if (p >= 0) a.b[p] = v;
+        else a.pc[4 * (int64_t)(-p - 1) + 3] = v;
+    }
+}
+__global__ __launch_bounds__(kBlock) void rhs_kernel(RhsArgs a) { rhs_dof(a, (int64_t)blockIdx.x * kBlock + threadIdx.x); }
 
 // ---- the nz scatter by nodes -------------------------------------------------
 // The six columns of a node whose elements are beams hold whole 6×6 blocks: one per neighbour and
@@ -1394,8 +1433,9 @@ constexpr int kNodeWaves = 4, kWaveBlocks = 10;
 constexpr int kNodeUnits = 4;   // tens of blocks a wave takes one after another
 struct NodeArgs {
     NodeMap m;
-    int64_t per_xcd, ntile;   // ntile: tiles of blocks; tiles of `rest` follow
+    int64_t per_xcd, ntile, nrest;   // tiles of blocks, then of `rest`, then of the rhs
     int units;
+    RhsArgs rhs;
     const int32_t* seg;
     const uint32_t* src;
     const double* K;
@@ -1410,6 +1450,10 @@ __global__ __launch_bounds__(64 * kNodeWaves) void node_scatter_kernel(NodeArgs 
         const int64_t o = IDX ? (int64_t)__builtin_nontemporal_load(a.dst + k) : k;
         a.out[o] = v;
     };
+    if (tile >= a.ntile + a.nrest) {
+        if (a.rhs.seg) rhs_dof(a.rhs, (tile - a.ntile - a.nrest) * (64 * kNodeWaves) + t);
+        return;
+    }
     if (tile >= a.ntile) {
         const int64_t q = (tile - a.ntile) * (64 * kNodeWaves) + t;
         if (q >= a.m.nrest) return;
@@ -1439,13 +1483,14 @@ __global__ __launch_bounds__(64 * kNodeWaves) void node_scatter_kernel(NodeArgs 
     }
 }
 void launch_node_scatter(const NodeMap& m, hipStream_t s, const int32_t* seg, const uint32_t* src, const double* K,
-                         double* out, const int32_t* dst) {
+                         double* out, const int32_t* dst, const RhsArgs& rhs = RhsArgs()) {
     NodeArgs a;
-    a.m = m; a.seg = seg; a.src = src; a.K = K; a.out = out; a.dst = dst;
+    a.m = m; a.seg = seg; a.src = src; a.K = K; a.out = out; a.dst = dst; a.rhs = rhs;
     a.units = m.nblock >= (int64_t)2048 * kNodeWaves * kNodeUnits * kWaveBlocks ? kNodeUnits : 1;   // two workgroups a SIMD stay
     const int64_t per = (int64_t)kNodeWaves * a.units * kWaveBlocks;
     a.ntile = (m.nblock + per - 1) / per;
-    const int64_t nt = a.ntile + (m.nrest + 64 * kNodeWaves - 1) / (64 * kNodeWaves);
+    a.nrest = (m.nrest + 64 * kNodeWaves - 1) / (64 * kNodeWaves);
+    const int64_t nt = a.ntile + a.nrest + (rhs.n + 64 * kNodeWaves - 1) / (64 * kNodeWaves);
     a.per_xcd = (nt + kXCD - 1) / kXCD;
     const dim3 gr((unsigned)(a.per_xcd * kXCD)), bl(64 * kNodeWaves);
     if (dst) hipLaunchKernelGGL((node_scatter_kernel<true>), gr, bl, 0, s, a);
@@ -2181,17 +2226,17 @@ int mh_ctx_create(int device, mh_ctx** out) {
         delete c; return MH_ERR_HIP;
     }
     for (auto& e : c->ev) if (hipEventCreate(&e) != hipSuccess) { delete c; return MH_ERR_HIP; }
-    if (hipMalloc(&c->d_flag, sizeof(unsigned long long)) != hipSuccess) { delete c; return MH_ERR_HIP; }
-    if (hipHostMalloc((void**)&c->h_flag, sizeof(unsigned long long), hipHostMallocDefault) != hipSuccess) {
-        (void)hipFree(c->d_flag); delete c; return MH_ERR_HIP;
-    }
-    if (hipMalloc(&c->d_c6, sizeof(double) * 6) != hipSuccess ||
-        hipHostMalloc((void**)&c->h_c6, sizeof(double) * 6, hipHostMallocDefault) != hipSuccess ||
+    if (hipMalloc(&c->d_call, sizeof(CallWords)) != hipSuccess ||
+        hipHostMalloc((void**)&c->h_call, sizeof(CallWords), hipHostMallocDefault) != hipSuccess ||
+        hipHostMalloc((void**)&c->h_res, sizeof(CallResults), hipHostMallocDefault) != hipSuccess ||
         scratch_address(device, &c->d_scratch) != MH_OK) {
-        if (c->h_c6) (void)hipHostFree(c->h_c6);
-        if (c->d_c6) (void)hipFree(c->d_c6);
-        (void)hipHostFree(c->h_flag); (void)hipFree(c->d_flag); delete c; return MH_ERR_HIP;
+        if (c->h_res) (void)hipHostFree(c->h_res);
+        if (c->h_call) (void)hipHostFree(c->h_call);
+        if (c->d_call) (void)hipFree(c->d_call);
+        delete c; return MH_ERR_HIP;
     }
+    c->d_c6 = c->d_call->c6; c->d_flag = &c->d_call->flag; c->d_cflag = c->d_call->cflag;
+    c->h_flag = &c->h_res->flag; c->h_cflag = c->h_res->cflag; c->h_norm = c->h_res->norm;
     *out = c;
     return MH_OK;
 }
@@ -2201,10 +2246,9 @@ int mh_ctx_destroy(mh_ctx* c) {
     (void)hipSetDevice(c->device);
     (void)hipStreamSynchronize(c->stream);
     free_model(c);
-    dfree(c->d_flag);
-    if (c->h_flag) (void)hipHostFree(c->h_flag);
-    dfree(c->d_c6);
-    if (c->h_c6) (void)hipHostFree(c->h_c6);
+    dfree(c->d_call);
+    if (c->h_call) (void)hipHostFree(c->h_call);
+    if (c->h_res) (void)hipHostFree(c->h_res);
     for (auto& e : c->ev) if (e) (void)hipEventDestroy(e);
     if (c->blas) (void)rocblas_destroy_handle(c->blas);
     if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -2572,7 +2616,7 @@ int mh_set_time(mh_ctx* c, double t) {
 
 }  // extern "C"
 
-// Every launch of one assemble!{mission} of AssemblySweepX{OX}: the NaN-flag reset, the
+// Every launch of one assemble!{mission} of AssemblySweepX{OX} (after upload_call): the
 // element kernels of all groups, the nz scatter and the rhs scatter, on the context's
 // stream. With timed, HIP events bracket the three phases (not inside a graph capture).
 // The tuner of the static beam kernel's LDS tile (elements per workgroup), run once per
@@ -2613,15 +2657,16 @@ static int tune_beams(Ctx* c) {
 // cleared first) instead of nzval, for a device Newton iteration that solves right after.
 static int enqueue_sweepx(Ctx* c, int OX, bool step, const double* c6, bool timed, bool fused = false) {
     hipStream_t s = c->stream;
-    hipLaunchKernelGGL(fill_u64, dim3(1), dim3(1), 0, s, c->d_flag, ~0ull);
     if (timed) HIPCHK(c, hipEventRecord(c->ev[0], s));
     PointBatch pb;
     pb.ngroup = 0;
     pb.start[0] = 0;
     auto flush_points = [&]() {
-        if (pb.ngroup == 0) return;
-        hipLaunchKernelGGL(point_kernel, dim3(grid(pb.start[pb.ngroup])), dim3(kBlock), 0, s, pb);
+        const int64_t n = pb.start[pb.ngroup] + pb.clear.npc + pb.clear.nslot;
+        if (n == 0) return;
+        hipLaunchKernelGGL(point_kernel, dim3(grid(n)), dim3(kBlock), 0, s, pb);
         pb.ngroup = 0;
+        pb.clear = ChainClear();
     };
     for (size_t gi = 0; gi < c->groups.size(); ++gi) {
         Group& g = c->groups[gi];
@@ -2644,38 +2689,34 @@ static int enqueue_sweepx(Ctx* c, int OX, bool step, const double* c6, bool time
             if (++pb.ngroup == kPointBatch) flush_points();
         }
     }
+    double* const pc = c->d_cbuf ? c->d_cbuf + 3 * c->cnb * c->cB * c->cB + c->cnb * c->cB : nullptr;
+    if (fused) {
+        pb.clear.npc = 4 * c->cnp; pb.clear.pc = pc;
+        pb.clear.nslot = c->cnu; pb.clear.slot = c->d_cunc; pb.clear.D = c->d_cbuf;
+    }
     flush_points();
     if (int r = check_launch(c, "element kernels")) return r;
     if (timed) HIPCHK(c, hipEventRecord(c->ev[1], s));
+    RhsArgs rh;
+    rh.n = c->nX; rh.seg = c->d_rseg; rh.src = c->d_rsrc; rh.R = c->d_Rbuf; rh.dR = step ? c->d_dRbuf : nullptr; rh.out = c->d_rhs;
+    rh.flag = c->d_flag; rh.hflag = c->h_flag;
+    if (fused) { rh.pos = c->d_cpos; rh.b = c->d_cbuf + 3 * c->cnb * c->cB * c->cB; rh.pc = pc; }
+    double* out = fused ? c->d_cbuf : c->d_nzval;
+    const int32_t* dst = fused ? c->d_cslot : nullptr;
+    // One launch for both sums where the nz go by nodes and both are small: at 94,000 dofs a pass takes
+    // 120 µs joined and 125 apart, at 290,000 it makes no difference, at 2.3 million 1023 and 919. Apart
+    // when they are timed apart.
+    const bool joined = c->use_nodes && c->nnz && !timed && c->nX <= 1 << 17;
     if (c->nnz) {
-        double* out = c->d_nzval;
-        const int32_t* dst = nullptr;
-        if (fused) {
-            const int64_t pcbase = 3 * c->cnb * c->cB * c->cB + c->cnb * c->cB;
-            if (c->cnp)
-                hipLaunchKernelGGL(chain::fill_f64, dim3((unsigned)((4 * c->cnp + chain::kCB - 1) / chain::kCB)),
-                                   dim3(chain::kCB), 0, s, 4 * c->cnp, c->d_cbuf + pcbase, 0.0);
-            out = c->d_cbuf;
-            dst = c->d_cslot;
-        }
         if (c->use_nodes) {
-            launch_node_scatter(c->nmap, s, c->d_kseg, c->d_ksrc, c->d_Kbuf, out, dst);
+            const RhsArgs none;
+            launch_node_scatter(c->nmap, s, c->d_kseg, c->d_ksrc, c->d_Kbuf, out, dst, joined ? rh : none);
         } else if (c->coded) launch_scatter<true>(c->scatter_variant, s, c->nnz, c->d_kseg, c->d_ksrc, c->d_Kbuf, out, dst);
         else launch_scatter<false>(c->scatter_variant, s, c->nnz, c->d_kseg, c->d_ksrc, c->d_Kbuf, out, dst);
     }
     if (timed) HIPCHK(c, hipEventRecord(c->ev[2], s));
-    if (c->nX) {
-        const int64_t per = ((c->nX + kTile - 1) / kTile + kXCD - 1) / kXCD;
-        if (step)
-            hipLaunchKernelGGL((scatter_kernel<true, false>), dim3((unsigned)(per * kXCD)), dim3(kTile), 0, s, c->nX, per,
-                               c->d_rseg, c->d_rsrc, c->d_Rbuf, (const double*)c->d_dRbuf, c->d_rhs);
-        else
-            hipLaunchKernelGGL((scatter_kernel<false, false>), dim3((unsigned)(per * kXCD)), dim3(kTile), 0, s, c->nX, per,
-                               c->d_rseg, c->d_rsrc, c->d_Rbuf, (const double*)nullptr, c->d_rhs);
-    }
+    if (!joined) hipLaunchKernelGGL(rhs_kernel, dim3(std::max(grid(c->nX), 1u)), dim3(kBlock), 0, s, rh);
     if (timed) HIPCHK(c, hipEventRecord(c->ev[3], s));
-    // the NaN flag goes to pinned host memory on the stream (a node of a captured graph)
-    HIPCHK(c, hipMemcpyAsync(c->h_flag, c->d_flag, sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
     return check_launch(c, "scatter kernels");
 }
 
@@ -2701,11 +2742,16 @@ static int finish_sweepx(Ctx* c, mh_err* err) {
     return MH_OK;
 }
 
-// The Newmark coefficients of this call into d_c6, ahead of the kernels on the stream: kernels
-// (eager or replayed from a graph) read them there, so a graph outlives a change of Δt.
-static int upload_c6(Ctx* c, int OX, const double* c6) {
-    for (int i = 0; i < 6; ++i) c->h_c6[i] = (OX > 0 && c6) ? c6[i] : 0.;
-    HIPCHK(c, hipMemcpyAsync(c->d_c6, c->h_c6, sizeof(double) * 6, hipMemcpyHostToDevice, c->stream));
+// The Newmark coefficients of this call, with the NaN flag and the chain solve's status words reset, in
+// one copy ahead of the kernels on the stream: kernels (eager or replayed from a graph) read them
+// there, so a graph outlives a change of Δt and holds no nodes that clear flags.
+static int upload_call(Ctx* c, int OX, const double* c6) {
+    CallWords& h = *c->h_call;
+    for (int i = 0; i < 6; ++i) h.c6[i] = (OX > 0 && c6) ? c6[i] : 0.;
+    h.flag = ~0ull;
+    h.cflag[0] = h.cflag[1] = 0u;
+    h.where[0] = h.where[1] = ~0ull;
+    HIPCHK(c, hipMemcpyAsync(c->d_call, c->h_call, sizeof(CallWords), hipMemcpyHostToDevice, c->stream));
     return MH_OK;
 }
 
@@ -2727,7 +2773,7 @@ int mh_assemble_sweepx(mh_ctx* c, int OX, int mission, const double* c6, mh_err*
     if (!c->beam_tuned)
         if (int r = tune_beams(c)) return r;
     const bool step = (mission == 0) && OX > 0;
-    if (int r = upload_c6(c, OX, c6)) return r;
+    if (int r = upload_call(c, OX, c6)) return r;
     if (int r = enqueue_sweepx(c, OX, step, c6, true)) return r;
     c->timed = true;
     c->graph_timed = false;
@@ -2742,7 +2788,7 @@ int mh_assemble_sweepx_graph(mh_ctx* c, int OX, int mission, const double* c6, m
         ++c->gen;
     }
     const bool step = (mission == 0) && OX > 0;
-    if (int r = upload_c6(c, OX, c6)) return r;
+    if (int r = upload_call(c, OX, c6)) return r;
     const double key[9] = {0, 0, 0, 0, 0, 0, 0, 0, reads_time(c) ? c->t : 0.};
     const int sl = step ? 1 : 0;
     bool same = c->gexec[sl] && c->gOX[sl] == OX && c->ggen[sl] == c->gen;
@@ -2827,8 +2873,8 @@ int mh_vjp_lagrangian(mh_ctx* c, int OX, mh_err* err) {
     if (c->nX) {
         const int64_t per = ((c->nX + kTile - 1) / kTile + kXCD - 1) / kXCD;
         for (int d = 0; d < nd; ++d)
-            hipLaunchKernelGGL((scatter_kernel<false, false>), dim3((unsigned)(per * kXCD)), dim3(kTile), 0, s, c->nX, per,
-                               c->d_rseg, c->d_rsrc, c->d_gbuf + d * c->nR, (const double*)nullptr, c->d_gX + d * c->nX);
+            hipLaunchKernelGGL((scatter_kernel<false>), dim3((unsigned)(per * kXCD)), dim3(kTile), 0, s, c->nX, per,
+                               c->d_rseg, c->d_rsrc, c->d_gbuf + d * c->nR, c->d_gX + d * c->nX);
     }
     HIPCHK(c, hipEventRecord(c->ev[2], s));
     if (c->nU) {
@@ -2837,8 +2883,8 @@ int mh_vjp_lagrangian(mh_ctx* c, int OX, mh_err* err) {
                                c->d_gubuf, c->d_gU);
         } else if (c->nRU) {
             const int64_t per = ((c->nU + kTile - 1) / kTile + kXCD - 1) / kXCD;
-            hipLaunchKernelGGL((scatter_kernel<false, false>), dim3((unsigned)(per * kXCD)), dim3(kTile), 0, s, c->nU, per,
-                               c->d_useg, c->d_usrc, c->d_gubuf, (const double*)nullptr, c->d_gU);
+            hipLaunchKernelGGL((scatter_kernel<false>), dim3((unsigned)(per * kXCD)), dim3(kTile), 0, s, c->nU, per,
+                               c->d_useg, c->d_usrc, c->d_gubuf, c->d_gU);
         } else {
             HIPCHK(c, hipMemsetAsync(c->d_gU, 0, sizeof(double) * c->nU, s));
         }
@@ -3078,13 +3124,12 @@ int mh_assemble_direct(mh_ctx* c, int mission, double dt, mh_err* err) {
         if (int r = launch_direct(c, g, nd, dt, (unsigned long long)gi << 40)) return r;
     }
     HIPCHK(c, hipEventRecord(c->ev[1], s));
-    const double* nul = nullptr;
     if (c->nX) {
         const int64_t per = ((c->nX + kTile - 1) / kTile + kXCD - 1) / kXCD;
-        hipLaunchKernelGGL((scatter_kernel<false, false>), dim3((unsigned)(per * kXCD)), dim3(kTile), 0, s, c->nX, per,
-                           c->d_rseg, c->d_rsrc, c->d_Rd, nul, c->d_dL1);
-        hipLaunchKernelGGL((scatter_kernel<false, false>), dim3((unsigned)(per * kXCD)), dim3(kTile), 0, s, c->nX, per,
-                           c->d_rseg, c->d_rsrc, c->d_L1x, nul, c->d_dL1 + c->nX);
+        hipLaunchKernelGGL((scatter_kernel<false>), dim3((unsigned)(per * kXCD)), dim3(kTile), 0, s, c->nX, per,
+                           c->d_rseg, c->d_rsrc, c->d_Rd, c->d_dL1);
+        hipLaunchKernelGGL((scatter_kernel<false>), dim3((unsigned)(per * kXCD)), dim3(kTile), 0, s, c->nX, per,
+                           c->d_rseg, c->d_rsrc, c->d_L1x, c->d_dL1 + c->nX);
     }
     HIPCHK(c, hipEventRecord(c->ev[2], s));
     if (mission == 1) {
@@ -3164,8 +3209,13 @@ namespace {
 
 int64_t cgrid(int64_t n) { return (n + chain::kCB - 1) / chain::kCB; }
 
-// fused: the assembly already scattered Lλx into the blocks (enqueue_sweepx with fused),
-// after clearing pc; the pack is skipped.
+template <int B>
+chain::Unpack unpack_args(Ctx* c) {
+    double* b = c->d_cbuf + 3 * c->cnb * B * B;
+    return chain::Unpack{c->cnb, c->d_cpos, c->d_chpos, b + c->cnb * B, c->d_csaved, b};
+}
+// fused: the assembly already scattered Lλx and Lλ into the blocks (enqueue_sweepx with fused), after
+// the clears; the pack is skipped, and the unpack left to the Newton update.
 template <int B>
 int enqueue_chain_solve(Ctx* c, const double* rhs, bool timed = true, bool fused = false) {
     using namespace chain;
@@ -3177,15 +3227,15 @@ int enqueue_chain_solve(Ctx* c, const double* rhs, bool timed = true, bool fused
     double* b = U + nb * BB;
     double* pc = b + nb * B;
     if (timed) HIPCHK(c, hipEventRecord(c->cev[0], s));
-    hipLaunchKernelGGL(clear_flag, dim3(1), dim3(1), 0, s, c->d_cflag);
+    if (!fused) hipLaunchKernelGGL(clear_flag, dim3(1), dim3(1), 0, s, c->d_cflag);
     if (c->cnp && !fused) hipLaunchKernelGGL(fill_f64, dim3(cgrid(4 * c->cnp)), dim3(kCB), 0, s, 4 * c->cnp, pc, 0.0);
-    if (c->cnu) hipLaunchKernelGGL(zero_slots_kernel, dim3(cgrid(c->cnu)), dim3(kCB), 0, s, c->cnu, c->d_cunc, D);
-    if (c->cnd) hipLaunchKernelGGL(dummy_kernel<B>, dim3(cgrid(c->cnd)), dim3(kCB), 0, s, c->cnd, c->d_cdum, D, b);
+    if (c->cnu && !fused) hipLaunchKernelGGL(zero_slots_kernel, dim3(cgrid(c->cnu)), dim3(kCB), 0, s, c->cnu, c->d_cunc, D);
     if (c->nnz && !fused)
         hipLaunchKernelGGL(pack_kernel, dim3(cgrid(c->nnz)), dim3(kCB), 0, s, c->nnz, c->d_cslot, c->d_nzval, c->d_cbuf);
-    hipLaunchKernelGGL(pack_rhs_kernel, dim3(cgrid(c->nX)), dim3(kCB), 0, s, c->nX, c->d_cpos, rhs, b, pc);
-    if (c->cnp) hipLaunchKernelGGL(pair_kernel<B>, dim3(cgrid(c->cnp)), dim3(kCB), 0, s, c->cnp, c->d_chpos, pc, D, L,
-                                   U, b, c->d_csaved, c->d_cflag);
+    if (!fused) hipLaunchKernelGGL(pack_rhs_kernel, dim3(cgrid(c->nX)), dim3(kCB), 0, s, c->nX, c->d_cpos, rhs, b, pc);
+    if (c->cnp + c->cnd)
+        hipLaunchKernelGGL(pair_kernel<B>, dim3(cgrid(c->cnp + c->cnd)), dim3(kCB), 0, s, c->cnp, c->d_chpos, pc, D, L, U, b,
+                           c->d_csaved, c->d_cflag, c->cnd, c->d_cdum);
     if (timed) HIPCHK(c, hipEventRecord(c->cev[1], s));
     const auto& sy = c->csys;
     const size_t np = sy.size();
@@ -3196,8 +3246,8 @@ int enqueue_chain_solve(Ctx* c, const double* rhs, bool timed = true, bool fused
     if (timed) HIPCHK(c, hipEventRecord(c->cev[2], s));
     for (size_t p = np - 1; p-- > 0;)
         hipLaunchKernelGGL(back_kernel<B>, chunks(sy[p]), dim3(chain::kChunk * B), 0, s, sy[p], (const double*)sy[p + 1].b);
-    hipLaunchKernelGGL(unpack_kernel<B>, dim3(cgrid(c->nX)), dim3(kCB), 0, s, c->nX, nb, c->d_cpos, c->d_chpos, pc,
-                       c->d_csaved, b, c->d_dx);
+    if (!fused)
+        hipLaunchKernelGGL(unpack_kernel<B>, dim3(cgrid(c->nX)), dim3(kCB), 0, s, c->nX, unpack_args<B>(c), c->d_dx);
     if (timed) HIPCHK(c, hipEventRecord(c->cev[3], s));
     HIPCHK(c, hipGetLastError());
     return MH_OK;
@@ -3285,8 +3335,6 @@ int mh_chain_prepare(mh_ctx* c, int B, int64_t nblock, const int64_t* pos, int64
     HIPCHK(c, hipMalloc(&c->d_cbuf, sizeof(double) * ntot));
     HIPCHK(c, hipMalloc(&c->d_csaved, sizeof(double) * std::max<int64_t>(npair * (3 * B + 1), 1)));
     HIPCHK(c, hipMalloc(&c->d_dx, sizeof(double) * std::max<int64_t>(c->nX, 1)));
-    HIPCHK(c, hipMalloc(&c->d_cflag, chain::kStatusBytes));
-    HIPCHK(c, hipHostMalloc((void**)&c->h_cflag, chain::kStatusBytes, hipHostMallocDefault));
     for (auto& e : c->cev) HIPCHK(c, hipEventCreate(&e));
     {   // the phases of the reduction: each leaves the first block of every chunk to the next
         chain::System x;
@@ -3432,29 +3480,30 @@ int mh_newton_prepare(mh_ctx* c, const double* scaleX) {
     if (!c || (c->nX && !scaleX)) return MH_ERR_ARG;
     HIPCHK(c, hipSetDevice(c->device));
     HIPCHK(c, hipStreamSynchronize(c->stream));
-    dfree(c->d_scaleX); dfree(c->d_part); dfree(c->d_norm);
-    if (c->h_norm) { (void)hipHostFree(c->h_norm); c->h_norm = nullptr; }
+    dfree(c->d_scaleX); dfree(c->d_part);
     const int64_t n = std::max<int64_t>(c->nX, 1);
     HIPCHK(c, hipMalloc(&c->d_scaleX, sizeof(double) * n));
     HIPCHK(c, hipMalloc(&c->d_part, sizeof(double) * 2 * cgrid(n)));
-    HIPCHK(c, hipMalloc(&c->d_norm, sizeof(double) * 2));
-    HIPCHK(c, hipHostMalloc((void**)&c->h_norm, sizeof(double) * 2, hipHostMallocDefault));
     if (c->nX) HIPCHK(c, copy_sync(c, c->d_scaleX, scaleX, sizeof(double) * c->nX, hipMemcpyHostToDevice));
     ++c->gen;   // a captured Newton iteration holds the old buffers
     return MH_OK;
 }
 
-// Newmarkβdecrement!{OX} of the device X with the last Δx, and the norms into pinned memory
-// (kernels and a copy on the stream: also nodes of a captured Newton iteration).
-// The coefficients are read from d_c6 (upload_c6 first).
-static int enqueue_newton_update(Ctx* c, int OX, int first) {
+// Newmarkβdecrement!{OX} of the device X with the last Δx (fused: taken from the solve's blocks in the
+// same kernel), and the norms and the solve's status words into pinned memory.
+// The coefficients are read from d_c6 (upload_call first).
+static int enqueue_newton_update(Ctx* c, int OX, int first, bool fused = false) {
     hipStream_t s = c->stream;
     const int64_t ng = cgrid(std::max<int64_t>(c->nX, 1));
-    hipLaunchKernelGGL(chain::newmark_kernel, dim3(ng), dim3(chain::kCB), 0, s, c->nX, OX, first, c->d_c6, c->d_dx,
-                       c->d_rhs, c->d_scaleX, c->d_X[0], c->d_X[1], c->d_X[2], c->d_part);
-    hipLaunchKernelGGL(chain::norm_kernel, dim3(1), dim3(chain::kCB), 0, s, ng, c->d_part, c->d_norm);
+    auto run = [&](auto kernel, const chain::Unpack& u) {
+        hipLaunchKernelGGL(kernel, dim3(ng), dim3(chain::kCB), 0, s, c->nX, OX, first, c->d_c6, u, c->d_dx, c->d_rhs,
+                           c->d_scaleX, c->d_X[0], c->d_X[1], c->d_X[2], c->d_part);
+    };
+    if (!fused) run(chain::newmark_kernel<0>, chain::Unpack());
+    else if (c->cB == 6) run(chain::newmark_kernel<6>, unpack_args<6>(c));
+    else run(chain::newmark_kernel<3>, unpack_args<3>(c));
+    hipLaunchKernelGGL(chain::norm_kernel, dim3(1), dim3(chain::kCB), 0, s, ng, c->d_part, c->h_norm, c->d_cflag, c->h_cflag);
     HIPCHK(c, hipGetLastError());
-    HIPCHK(c, hipMemcpyAsync(c->h_norm, c->d_norm, sizeof(double) * 2, hipMemcpyDeviceToHost, s));
     return MH_OK;
 }
 static int check_newton_args(Ctx* c, int OX, const double* c6, const double* norms) {
@@ -3466,7 +3515,7 @@ static int check_newton_args(Ctx* c, int OX, const double* c6, const double* nor
 int mh_newton_update(mh_ctx* c, int OX, int first, const double* c6, double* norms) {
     if (int r = check_newton_args(c, OX, c6, norms)) return r;
     HIPCHK(c, hipSetDevice(c->device));
-    if (int r = upload_c6(c, OX, c6)) return r;
+    if (int r = upload_call(c, OX, c6)) return r;
     if (int r = enqueue_newton_update(c, OX, first)) return r;
     HIPCHK(c, hipStreamSynchronize(c->stream));
     norms[0] = c->h_norm[0];
@@ -3483,7 +3532,7 @@ int mh_newton_iteration_graph(mh_ctx* c, int OX, int first, const double* c6, do
         ++c->gen;
     }
     const bool step = first && OX > 0;
-    if (int r = upload_c6(c, OX, c6)) return r;
+    if (int r = upload_call(c, OX, c6)) return r;
     const double key[9] = {0, 0, 0, 0, 0, 0, 0, 0, reads_time(c) ? c->t : 0.};
     const int sl = first ? 3 : 2;
     bool same = c->gexec[sl] && c->gOX[sl] == OX && c->ggen[sl] == c->gen;
@@ -3495,11 +3544,7 @@ int mh_newton_iteration_graph(mh_ctx* c, int OX, int first, const double* c6, do
         int r = enqueue_sweepx(c, OX, step, c6, false, true);
         if (r == MH_OK)
             r = c->cB == 6 ? enqueue_chain_solve<6>(c, c->d_rhs, false, true) : enqueue_chain_solve<3>(c, c->d_rhs, false, true);
-        if (r == MH_OK) {
-            const hipError_t e = hipMemcpyAsync(c->h_cflag, c->d_cflag, chain::kStatusBytes, hipMemcpyDeviceToHost, s);
-            if (e != hipSuccess) { c->err = std::string("capture: ") + hipGetErrorString(e); r = MH_ERR_HIP; }
-        }
-        if (r == MH_OK) r = enqueue_newton_update(c, OX, first);
+        if (r == MH_OK) r = enqueue_newton_update(c, OX, first, true);
         hipGraph_t g = nullptr;
         const hipError_t ec = hipStreamEndCapture(s, &g);
         if (r != MH_OK || ec != hipSuccess) {
