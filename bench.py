@@ -31,12 +31,12 @@ FP64_PEAK = 78.6e12        # MI355X FP64 vector, FLOP/s
 # FP64 operations per beam of the static kernel (add/sub/mul/div/sqrt = 1, fma = 2),
 # from the SQ_INSTS_VALU_{ADD,MUL,FMA,TRANS}_F64 counters of one assembly of this
 # workload divided by the number of beams (profiles/space_frame_100x100x33_pmc.md).
-F_ELEM = 6299
+F_ELEM = 2794
 # The same for the dynamic beam of the catenary chains (OX = 2): value pass + direction pass
 # per beam, and their HBM bytes per assembly from FETCH_SIZE/WRITE_SIZE
 # (profiles/catenary_chains_256_kernels.md), by mission.
-F_DYN = {"iter": 10890 + 75981, "step": 10890 + 84845}
-DYN_TRAFFIC = {"iter": 9.17e9 + 13.77e9, "step": 9.17e9 + 14.39e9}
+F_DYN = {"iter": 5902 + 19572, "step": 5902 + 26212}
+DYN_TRAFFIC = {"iter": 15.41e9 + 23.47e9, "step": 15.41e9 + 28.69e9}
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "space_frame_100x100x33_traffic.json")
 
 
