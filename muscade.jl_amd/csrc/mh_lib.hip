@@ -246,6 +246,11 @@ struct Ctx {
     } while (0)
 
 template <class T> void dfree(T*& p) { if (p) { (void)hipFree(p); p = nullptr; } }
+// Room for n values (at least one) at p, unless a call before left it there. Every buffer by itself: the
+// first of several says nothing about the others where an allocation failed.
+template <class T> hipError_t dneed(T*& p, int64_t n) {
+    return p ? hipSuccess : hipMalloc(&p, sizeof(T) * std::max<int64_t>(n, 1));
+}
 
 void free_graph(Ctx* c, int slot) {
     if (c->gexec[slot]) { (void)hipGraphExecDestroy(c->gexec[slot]); c->gexec[slot] = nullptr; }
@@ -2834,7 +2839,7 @@ int mh_graph_captures(mh_ctx* c, int64_t* n) {
 int mh_set_lambda(mh_ctx* c, const double* lam) {
     if (!c || !lam || !(c->prepared || c->direct)) return MH_ERR_ARG;
     HIPCHK(c, hipSetDevice(c->device));
-    if (!c->d_lam) HIPCHK(c, hipMalloc(&c->d_lam, sizeof(double) * std::max<int64_t>(c->nX, 1)));
+    HIPCHK(c, dneed(c->d_lam, c->nX));
     if (c->nX) HIPCHK(c, hipMemcpyAsync(c->d_lam, lam, sizeof(double) * c->nX, hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     return MH_OK;
@@ -2848,25 +2853,23 @@ int mh_vjp_lagrangian(mh_ctx* c, int OX, mh_err* err) {
     HIPCHK(c, hipSetDevice(c->device));
     hipStream_t s = c->stream;
     const int nd = OX + 1;
-    if (!c->d_gbuf) {
-        HIPCHK(c, hipMalloc(&c->d_gbuf, sizeof(double) * std::max<int64_t>(3 * c->nR, 1)));
-        HIPCHK(c, hipMalloc(&c->d_gX, sizeof(double) * std::max<int64_t>(3 * c->nX, 1)));
-        HIPCHK(c, hipMalloc(&c->d_gubuf, sizeof(double) * std::max<int64_t>(c->nRU, 1)));
-        HIPCHK(c, hipMalloc(&c->d_gU, sizeof(double) * std::max<int64_t>(c->nU, 1)));
-        if (c->nRA) {
-            HIPCHK(c, hipMalloc(&c->d_gabuf, sizeof(double) * c->nRA));
-            HIPCHK(c, hipMalloc(&c->d_gA, sizeof(double) * std::max<int64_t>(c->nA, 1)));
-        }
+    HIPCHK(c, dneed(c->d_gbuf, 3 * c->nR));
+    HIPCHK(c, dneed(c->d_gX, 3 * c->nX));
+    HIPCHK(c, dneed(c->d_gubuf, c->nRU));
+    HIPCHK(c, dneed(c->d_gU, c->nU));
+    if (c->nRA) {
+        HIPCHK(c, dneed(c->d_gabuf, c->nRA));
+        HIPCHK(c, dneed(c->d_gA, c->nA));
     }
-    if (OX > 0 && !c->d_Kc) {
+    if (OX > 0) {
         int64_t nKc = 0, nRec = 0;
         for (auto& g : c->groups)
             if (g.kind == MH_KIND_BEAM || g.kind == MH_KIND_BEAM_U) {
                 g.kcbase = nKc; nKc += g.nele * mh::kCompact;
                 g.recbase = nRec; nRec += rec_numbers(g.nele);
             }
-        if (nKc) HIPCHK(c, hipMalloc(&c->d_Kc, sizeof(double) * nKc));
-        if (nRec) HIPCHK(c, hipMalloc(&c->d_rec, sizeof(double) * nRec));
+        if (nKc) HIPCHK(c, dneed(c->d_Kc, nKc));
+        if (nRec) HIPCHK(c, dneed(c->d_rec, nRec));
     }
     hipLaunchKernelGGL(fill_u64, dim3(1), dim3(1), 0, s, c->d_flag, ~0ull);
     HIPCHK(c, hipEventRecord(c->ev[0], s));
@@ -3416,9 +3419,8 @@ static int adjoint_solve_tail(Ctx* c, double alpha) {
     return chain_status(c);
 }
 static int adjoint_buffers(Ctx* c) {
-    const int64_t n = std::max<int64_t>(c->nX, 1);
-    if (!c->d_crhs) HIPCHK(c, hipMalloc(&c->d_crhs, sizeof(double) * n));
-    if (!c->d_lam) HIPCHK(c, hipMalloc(&c->d_lam, sizeof(double) * n));
+    HIPCHK(c, dneed(c->d_crhs, c->nX));
+    HIPCHK(c, dneed(c->d_lam, c->nX));
     return MH_OK;
 }
 
@@ -3450,9 +3452,11 @@ int mh_adjoint_solve_sparse(mh_ctx* c, int64_t n, const int64_t* idx, const doub
     if (int r = adjoint_buffers(c)) return r;
     if (m > c->sp_cap) {
         dfree(c->d_spi); dfree(c->d_spv);
-        c->sp_cap = std::max<int64_t>(m, 256);
-        HIPCHK(c, hipMalloc(&c->d_spi, sizeof(int64_t) * c->sp_cap));
-        HIPCHK(c, hipMalloc(&c->d_spv, sizeof(double) * c->sp_cap));
+        c->sp_cap = 0;
+        const int64_t cap = std::max<int64_t>(m, 256);
+        HIPCHK(c, dneed(c->d_spi, cap));
+        HIPCHK(c, dneed(c->d_spv, cap));
+        c->sp_cap = cap;
     }
     hipStream_t s = c->stream;
     const int64_t nx = std::max<int64_t>(c->nX, 1);
@@ -3487,10 +3491,12 @@ int mh_newton_prepare(mh_ctx* c, const double* scaleX) {
     HIPCHK(c, hipSetDevice(c->device));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     dfree(c->d_scaleX); dfree(c->d_part);
-    const int64_t n = std::max<int64_t>(c->nX, 1);
-    HIPCHK(c, hipMalloc(&c->d_scaleX, sizeof(double) * n));
-    HIPCHK(c, hipMalloc(&c->d_part, sizeof(double) * 2 * cgrid(n)));
-    if (c->nX) HIPCHK(c, copy_sync(c, c->d_scaleX, scaleX, sizeof(double) * c->nX, hipMemcpyHostToDevice));
+    // d_scaleX last: its being there is what the calls that use both look at
+    HIPCHK(c, dneed(c->d_part, 2 * cgrid(std::max<int64_t>(c->nX, 1))));
+    HIPCHK(c, dneed(c->d_scaleX, c->nX));
+    const hipError_t e = c->nX ? copy_sync(c, c->d_scaleX, scaleX, sizeof(double) * c->nX, hipMemcpyHostToDevice) : hipSuccess;
+    if (e != hipSuccess) dfree(c->d_scaleX);
+    HIPCHK(c, e);
     ++c->gen;   // a captured Newton iteration holds the old buffers
     return MH_OK;
 }
