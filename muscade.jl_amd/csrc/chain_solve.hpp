@@ -43,11 +43,18 @@ enum : unsigned {
 };
 
 // The status words of a solve: flag (the k* bits) at word 0, then, as 64-bit values at
-// byte 8 and 16, a block found with a bad pivot (of the earliest phase; a block i = s + 2s·t of
-// level s, or 0 for the last remaining block) and the first bad λ pair
-// (all ones: none).
+// byte 8 and 16, the bad pivot's place (singular_block) and the first bad λ pair (all ones: none).
 constexpr int kStatusBytes = 24;
 __device__ inline unsigned long long* status_where(unsigned* f) { return reinterpret_cast<unsigned long long*>(f + 2); }
+// A diagonal block's place in the order of elimination: its level (block i = s + 2s·t leaves at level
+// s, block 0 is the last one), then the block. The least one is kept: a zero pivot makes later levels'
+// blocks of other workgroups bad too, whenever those run.
+constexpr int kPlaceShift = 48;
+__device__ inline void singular_block(unsigned* f, unsigned long long block) {
+    atomicOr(f, kSingular);
+    const unsigned long long level = block ? (unsigned long long)__builtin_ctzll(block) : 63ull;
+    atomicMin(status_where(f), level << kPlaceShift | block);
+}
 __global__ void clear_flag(unsigned* f) {
     f[0] = 0u;
     status_where(f)[0] = ~0ull;
@@ -172,7 +179,7 @@ __global__ __launch_bounds__(kCB) void pair_kernel(int64_t np, const int32_t* __
     const double cL = pc[4 * p], cU = pc[4 * p + 1], dg = pc[4 * p + 2], rl = pc[4 * p + 3];
     if (dg != 0.0 || cL == 0.0 || cU == 0.0) {
         atomicOr(flag, kBadPair);
-        atomicCAS(status_where(flag) + 1, ~0ull, (unsigned long long)p);
+        atomicMin(status_where(flag) + 1, (unsigned long long)p);
     }
     const int64_t h = hpos[p], blk = h / B, i = h - blk * B;
     double* sv = saved + p * (3 * B + 1);
@@ -286,10 +293,7 @@ __device__ inline void reduce_levels(double* __restrict__ M, int m, int E, int l
             if (live) load_col<B>(col, v);
             const bool ok = gauss_jordan<B>(v, base);
             if (live) {
-                if (!ok && q == 0) {
-                    atomicOr(flag, kSingular);
-                    atomicCAS(status_where(flag), ~0ull, (unsigned long long)((block0 + i) * stride));
-                }
+                if (!ok && q == 0) singular_block(flag, (unsigned long long)((block0 + i) * stride));
                 if (q < B || q >= 2 * B) {
 #pragma unroll
                     for (int r = 0; r < B; ++r) col[r] = v[r];
@@ -410,10 +414,7 @@ __global__ __launch_bounds__(kTopThreads) void top_kernel(System x, unsigned* __
         for (int r = 0; r < B; ++r) v[r] = 0.0;
         if (q < NC) load_col<B>(M + q * B, v);
         const bool ok = gauss_jordan<B>(v, 0);
-        if (q == 0 && !ok) {
-            atomicOr(flag, kSingular);
-            atomicCAS(status_where(flag), ~0ull, 0ull);
-        }
+        if (q == 0 && !ok) singular_block(flag, 0ull);
         if (q == 3 * B) {
 #pragma unroll
             for (int r = 0; r < B; ++r) M[3 * BB + r] = v[r];

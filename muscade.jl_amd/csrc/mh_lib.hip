@@ -3393,7 +3393,7 @@ static int chain_status_read(Ctx* c) {
         return MH_ERR_SOLVE;
     }
     if (f & chain::kSingular) {
-        const unsigned long long b = where[0];
+        const unsigned long long b = where[0] & ((1ull << chain::kPlaceShift) - 1);
         c->err = "zero or non-finite pivot in diagonal block " + std::to_string(b) + " (0-based, chain order; " +
                  (b ? "reduction level " + std::to_string(b & (~b + 1)) : std::string("the last block")) + ")";
         return MH_ERR_SOLVE;
