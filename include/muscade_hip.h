@@ -330,6 +330,10 @@ int mh_calib_copy(mh_ctx* ctx, int64_t n, double* ms);
  * launch_scatter) and each shape's measured time in ms (16).
  * A measurement utility; no counterpart in the reference. */
 int mh_get_tuning(mh_ctx* ctx, int* variant, float* ms);
+/* How the prepared assembly launches its sums: info[0] 1 where the nz of beam nodes go by 6×6 blocks,
+ * info[1] the blocks and info[2] the nz outside them, info[3] the tens of blocks a wave takes, info[4] 1
+ * where a graph sums the rhs in the same launch. A testing utility; no counterpart in the reference. */
+int mh_get_scatter(mh_ctx* ctx, int64_t* info);
 /* The static beam kernel's LDS tile (elements per workgroup: 64, 128 or 256; every tile gives
  * the same numbers), picked by a tuner at the context's first SweepX assembly on its state, and
  * each tile's measured time in ms (3); MH_ERR_ARG before that assembly. A measurement utility;

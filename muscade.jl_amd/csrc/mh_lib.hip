@@ -1493,11 +1493,15 @@ __global__ __launch_bounds__(64 * kNodeWaves) void node_scatter_kernel(NodeArgs 
         for (int c = 0; c < 6; ++c) put((int64_t)h.x + r + c * (h.y & 0xffff), v[c]);
     }
 }
+// Four tens a wave where two workgroups a SIMD stay.
+int node_units(const NodeMap& m) {
+    return m.nblock >= (int64_t)2048 * kNodeWaves * kNodeUnits * kWaveBlocks ? kNodeUnits : 1;
+}
 void launch_node_scatter(const NodeMap& m, hipStream_t s, const int32_t* seg, const uint32_t* src, const double* K,
                          double* out, const int32_t* dst, const RhsArgs& rhs = RhsArgs()) {
     NodeArgs a;
     a.m = m; a.seg = seg; a.src = src; a.K = K; a.out = out; a.dst = dst; a.rhs = rhs;
-    a.units = m.nblock >= (int64_t)2048 * kNodeWaves * kNodeUnits * kWaveBlocks ? kNodeUnits : 1;   // two workgroups a SIMD stay
+    a.units = node_units(m);
     const int64_t per = (int64_t)kNodeWaves * a.units * kWaveBlocks;
     a.ntile = (m.nblock + per - 1) / per;
     a.nrest = (m.nrest + 64 * kNodeWaves - 1) / (64 * kNodeWaves);
@@ -2664,6 +2668,10 @@ static int tune_beams(Ctx* c) {
     return MH_OK;
 }
 
+// One launch for both sums where the nz go by nodes and both are small: at 94,000 dofs a pass takes
+// 120 µs joined and 125 apart, at 290,000 it makes no difference, at 2.3 million 1023 and 919.
+static bool joins_rhs(const Ctx* c) { return c->use_nodes && c->nnz && c->nX <= 1 << 17; }
+
 // fused: Lλx goes straight into the chain solve's blocks (each nz to its slot; the pc part
 // cleared first) instead of nzval, for a device Newton iteration that solves right after.
 static int enqueue_sweepx(Ctx* c, int OX, bool step, const double* c6, bool timed, bool fused = false) {
@@ -2714,10 +2722,7 @@ static int enqueue_sweepx(Ctx* c, int OX, bool step, const double* c6, bool time
     if (fused) { rh.pos = c->d_cpos; rh.b = c->d_cbuf + 3 * c->cnb * c->cB * c->cB; rh.pc = pc; }
     double* out = fused ? c->d_cbuf : c->d_nzval;
     const int32_t* dst = fused ? c->d_cslot : nullptr;
-    // One launch for both sums where the nz go by nodes and both are small: at 94,000 dofs a pass takes
-    // 120 µs joined and 125 apart, at 290,000 it makes no difference, at 2.3 million 1023 and 919. Apart
-    // when they are timed apart.
-    const bool joined = c->use_nodes && c->nnz && !timed && c->nX <= 1 << 17;
+    const bool joined = joins_rhs(c) && !timed;   // apart when they are timed apart
     if (c->nnz) {
         if (c->use_nodes) {
             const RhsArgs none;
@@ -3026,6 +3031,16 @@ int mh_get_tuning(mh_ctx* c, int* variant, float* ms) {
     if (!c || !c->prepared) return MH_ERR_ARG;
     if (variant) *variant = c->scatter_variant;
     if (ms) for (int v = 0; v < kScatterVariants; ++v) ms[v] = c->scatter_ms[v];
+    return MH_OK;
+}
+
+int mh_get_scatter(mh_ctx* c, int64_t* info) {
+    if (!c || !c->prepared || !info) return MH_ERR_ARG;
+    info[0] = c->use_nodes;
+    info[1] = c->nmap.nblock;
+    info[2] = c->nmap.nrest;
+    info[3] = c->use_nodes ? node_units(c->nmap) : 0;
+    info[4] = joins_rhs(c);
     return MH_OK;
 }
 
