@@ -325,9 +325,10 @@ int mh_last_timings(mh_ctx* ctx, double* ms);
  * that HBM byte counters (FETCH_SIZE, WRITE_SIZE) are calibrated against. */
 int mh_calib_copy(mh_ctx* ctx, int64_t n, double* ms);
 /* Shape of the segmented nz scatter (assemblies whose beam matrices are whole scatter the nz of beam
- * nodes by 6×6 blocks instead, with the same sums) picked by the prepare-time tuner (0..15: segments per lane ×
+ * nodes by 6×6 blocks instead, with the same sums) picked by a tuner (0..15: segments per lane ×
  * LDS chunk, with or without nontemporal index loads and stores; see mh_lib.hip
- * launch_scatter) and each shape's measured time in ms (16).
+ * launch_scatter) and each shape's measured time in ms (16). It runs at prepare, or where the nz go by
+ * nodes in this call, beside the assembled values.
  * A measurement utility; no counterpart in the reference. */
 int mh_get_tuning(mh_ctx* ctx, int* variant, float* ms);
 /* How the prepared assembly launches its sums: info[0] 1 where the nz of beam nodes go by 6×6 blocks,

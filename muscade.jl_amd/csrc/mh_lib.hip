@@ -163,7 +163,8 @@ struct Ctx {
     double* d_L1x = nullptr;     // nR: per-element L1[X][1] entries (Lagrangian-path elements)
     double* d_dL1 = nullptr;     // 2·nX: L1[Λ][1], L1[X][1]
     double* d_dL2 = nullptr;     // 2(OX+1)·nnz(XX) + 2·nnz(XU): L2[Λ,X][1,d], L2[X,Λ][d,1], L2[Λ,U][1,1], L2[U,Λ][1,1]
-    int scatter_variant = 0;     // nz scatter shape picked at prepare (launch_scatter)
+    int scatter_variant = 0;     // shape of the segmented nz scatter (launch_scatter): the tuner's, or set
+    bool scatter_tuned = false;
     NodeMap nmap;                // the nz scatter by nodes, used while use_nodes
     bool use_nodes = false;
     int beam_variant = 1;        // static beam kernel shape picked by tune_beams (launch_beam_static)
@@ -1954,8 +1955,41 @@ static int upload_soa(Ctx* c, T** dst, const T* src, int n, int64_t nele) {
 }
 
 
-// The rhs map (asm[1] for the X dofs): contributions of every element dof into Lλ, in
-// traversal order, stably sorted by dof (Assemble.jl:340-357 with add_value!'s order).
+// Tuner: time each shape of the segmented nz scatter on the prepared maps, into out, and keep (pick) the
+// fastest. The sums are identical for every shape (each segment is summed in the same order).
+static int tune_scatter(Ctx* c, double* out, bool pick) {
+    if (c->nnz > 0) {
+        hipStream_t s = c->stream;
+        hipEvent_t ev[2] = {nullptr, nullptr};
+        auto run = [&]() -> int {
+            for (auto& e : ev) HIPCHK(c, hipEventCreate(&e));
+            float best = 1e30f;
+            for (int v = 0; v < kScatterVariants; ++v) {
+                float tmin = 1e30f;
+                for (int rep = 0; rep < 3; ++rep) {
+                    HIPCHK(c, hipEventRecord(ev[0], s));
+                    if (c->coded) launch_scatter<true>(v, s, c->nnz, c->d_kseg, c->d_ksrc, c->d_Kbuf, out);
+                    else launch_scatter<false>(v, s, c->nnz, c->d_kseg, c->d_ksrc, c->d_Kbuf, out);
+                    HIPCHK(c, hipEventRecord(ev[1], s));
+                    HIPCHK(c, hipEventSynchronize(ev[1]));
+                    float ms = 0.f;
+                    HIPCHK(c, hipEventElapsedTime(&ms, ev[0], ev[1]));
+                    if (rep > 0 && ms < tmin) tmin = ms;
+                }
+                if (int r = check_launch(c, "scatter tuning")) return r;
+                c->scatter_ms[v] = tmin;
+                if (tmin < best) { best = tmin; if (pick) c->scatter_variant = v; }
+            }
+            return MH_OK;
+        };
+        const int r = run();
+        for (auto& e : ev) if (e) (void)hipEventDestroy(e);
+        if (r) return r;
+    }
+    c->scatter_tuned = true;
+    return MH_OK;
+}
+
 // The node map of the prepared nz maps (nmap.nblock = 0 when no beam node has whole-block columns).
 static int build_node_map(Ctx* c) {
     hipStream_t s = c->stream;
@@ -1997,6 +2031,8 @@ static int build_node_map(Ctx* c) {
     return MH_OK;
 }
 
+// The rhs map (asm[1] for the X dofs): contributions of every element dof into Lλ, in
+// traversal order, stably sorted by dof (Assemble.jl:340-357 with add_value!'s order).
 static int build_rmap(Ctx* c) {
     hipStream_t s = c->stream;
     const int64_t nR = c->nR, nX = c->nX;
@@ -2525,35 +2561,20 @@ int mh_prepare_sweepx(mh_ctx* c, int OX, int64_t* nnz_out) {
         HIPCHK(c, hipStreamSynchronize(s));
         dfree(rkin); dfree(rkout); dfree(rvin);
     }
-    // ---- tuner: time each shape of the nz scatter on these maps and keep the fastest.
-    // The sums are identical for every shape (each segment is summed in the same order).
-    if (nnz > 0) {
-        float best = 1e30f;
-        for (int v = 0; v < kScatterVariants; ++v) {
-            float tmin = 1e30f;
-            for (int rep = 0; rep < 3; ++rep) {
-                HIPCHK(c, hipEventRecord(c->ev[0], s));
-                if (coded) launch_scatter<true>(v, s, nnz, c->d_kseg, c->d_ksrc, c->d_Kbuf, c->d_nzval);
-                else launch_scatter<false>(v, s, nnz, c->d_kseg, c->d_ksrc, c->d_Kbuf, c->d_nzval);
-                HIPCHK(c, hipEventRecord(c->ev[1], s));
-                HIPCHK(c, hipEventSynchronize(c->ev[1]));
-                float ms = 0.f;
-                HIPCHK(c, hipEventElapsedTime(&ms, c->ev[0], c->ev[1]));
-                if (rep > 0 && ms < tmin) tmin = ms;
-            }
-            if (int r = check_launch(c, "scatter tuning")) return r;
-            c->scatter_ms[v] = tmin;
-            if (tmin < best) { best = tmin; c->scatter_variant = v; }
-        }
-    }
     // The scatter by nodes, where it covers at least half of the nz (its other nz are searched one by one)
     // and the elements' matrices are whole: 180 µs against 237 for the best segmented shape (383,000
     // beams in chains). From compact matrices it is the slower one (553 µs against 513, 973,000 beams
-    // of a lattice): a row's entries lie in 18 places of 360 B.
+    // of a lattice): a row's entries lie in 18 places of 360 B. The segmented scatter's shapes are timed
+    // only where it runs: 48 launches and waits, 0.9 of the 1.8 ms of preparing a chain of 101 beams, 14 of 158 at
+    // 383,000.
     if (nnz > 0 && !coded) {
         if (int r = build_node_map(c)) return r;
         c->use_nodes = c->nmap.nblock > 0 && 2 * c->nmap.nrest <= nnz;
     }
+    c->scatter_tuned = false;
+    c->scatter_variant = 0;
+    if (!c->use_nodes)
+        if (int r = tune_scatter(c, c->d_nzval, true)) return r;
     c->beam_tuned = false;
     c->prepared = true;
     if (nnz_out) *nnz_out = nnz;
@@ -3029,6 +3050,14 @@ int mh_set_scatter_variant(mh_ctx* c, int variant) {
 
 int mh_get_tuning(mh_ctx* c, int* variant, float* ms) {
     if (!c || !c->prepared) return MH_ERR_ARG;
+    if (!c->scatter_tuned) {   // an assembly by nodes: timed on request, beside the assembled values
+        HIPCHK(c, hipSetDevice(c->device));
+        double* out = nullptr;
+        HIPCHK(c, dneed(out, c->nnz));
+        const int r = tune_scatter(c, out, c->use_nodes);   // a shape that was set stays
+        dfree(out);
+        if (r) return r;
+    }
     if (variant) *variant = c->scatter_variant;
     if (ms) for (int v = 0; v < kScatterVariants; ++v) ms[v] = c->scatter_ms[v];
     return MH_OK;

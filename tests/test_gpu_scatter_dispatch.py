@@ -112,3 +112,23 @@ def test_newton_iteration_into_the_blocks(mc, n):
     assert states[0][0] == states[1][0]
     for a, b in zip(states[0][1], states[1][1]):
         assert np.array_equal(bits(a), bits(b))
+
+
+def test_tuning_on_request(mc):
+    """Where the nz go by nodes the segmented shapes are timed when they are asked for, beside the
+    assembled values and the times of the last assembly; a shape that was set stays."""
+    import ctypes
+    model, st = chain(mc, 400)
+    out = mc.AssemblySweepX(2, model, st.dis)
+    out.c = mc.Newmarkβcoefficients(2, 0.05)
+    out.assemble(st, "iter")
+    before, times = out.nzval.copy(), out.timings()
+    for variant in (None, 5):
+        if variant is not None:
+            out.ctx.check(mc.lib.mh_set_scatter_variant(out.ctx.h, variant), "variant")
+        v, ms = ctypes.c_int(), (ctypes.c_float * 16)()
+        out.ctx.check(mc.lib.mh_get_tuning(out.ctx.h, ctypes.byref(v), ms), "tuning")
+        assert 0 <= v.value < 16 and all(x > 0 for x in ms) and variant in (None, v.value)
+        out.ctx.check(mc.lib.mh_get_nzval(out.ctx.h, mc._lib.dptr(out.nzval)), "nzval")
+        assert np.array_equal(bits(out.nzval), bits(before)) and np.array_equal(out.timings(), times)
+        assert info(mc, out)["nodes"] == (variant is None)
