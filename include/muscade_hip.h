@@ -333,7 +333,8 @@ int mh_calib_copy(mh_ctx* ctx, int64_t n, double* ms);
 int mh_get_tuning(mh_ctx* ctx, int* variant, float* ms);
 /* How the prepared assembly launches its sums: info[0] 1 where the nz of beam nodes go by 6×6 blocks,
  * info[1] the blocks and info[2] the nz outside them, info[3] the tens of blocks a wave takes, info[4] 1
- * where a graph sums the rhs in the same launch. A testing utility; no counterpart in the reference. */
+ * where a graph sums the rhs in the same launch, info[5] and info[6] the nz outside blocks and the dofs of
+ * the rhs that are long sums, a wave each. A testing utility; no counterpart in the reference. */
 int mh_get_scatter(mh_ctx* ctx, int64_t* info);
 /* The static beam kernel's LDS tile (elements per workgroup: 64, 128 or 256; every tile gives
  * the same numbers), picked by a tuner at the context's first SweepX assembly on its state, and

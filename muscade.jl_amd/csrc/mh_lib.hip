@@ -82,11 +82,11 @@ struct DMap {
 
 // The nz scatter's map of nodes whose six dof columns hold whole 6×6 blocks of beam contributions
 // (build_node_map). Per block: the nz of its first entry, the column length | sources << 16, where its
-// sources start in src, and the first of them. rest: every other nz.
+// sources start in src, and the first of them. rest: every other nz; longs: those of them with long segments.
 struct NodeMap {
-    int64_t nblock = 0, nrest = 0;
+    int64_t nblock = 0, nrest = 0, nlong = 0;
     int4* blk = nullptr;
-    int32_t* rest = nullptr;
+    int32_t *rest = nullptr, *longs = nullptr;
     uint32_t* src = nullptr;
 };
 
@@ -130,6 +130,8 @@ struct Ctx {
     uint32_t* d_ksrc = nullptr;
     int32_t* d_rseg = nullptr;
     uint32_t* d_rsrc = nullptr;
+    int64_t nrlong = 0;          // X dofs with long segments
+    int32_t* d_rlong = nullptr;
     unsigned long long* d_flag = nullptr;   // d_call->flag
     unsigned long long* h_flag = nullptr;   // h_res->flag
     void* d_scratch = nullptr;   // this device's address of the fixed `scratch` array (set at create)
@@ -283,7 +285,7 @@ void free_prepared(Ctx* c) {
     free_big(c);
     dfree(c->d_Kbuf); dfree(c->d_Rbuf); dfree(c->d_dRbuf); dfree(c->d_nzval); dfree(c->d_rhs); dfree(c->d_Kc); dfree(c->d_rec);
     dfree(c->d_colptr); dfree(c->d_rowval); dfree(c->d_kseg); dfree(c->d_ksrc); dfree(c->d_rseg); dfree(c->d_rsrc);
-    dfree(c->nmap.blk); dfree(c->nmap.rest); dfree(c->nmap.src);
+    dfree(c->nmap.blk); dfree(c->nmap.rest); dfree(c->nmap.src); dfree(c->nmap.longs); dfree(c->d_rlong); c->nrlong = 0;
     c->nmap = NodeMap(); c->use_nodes = false;
     dfree(c->d_useg); dfree(c->d_usrc); dfree(c->d_gbuf); dfree(c->d_gX); dfree(c->d_gubuf); dfree(c->d_gU);
     dfree(c->d_aseg); dfree(c->d_asrc); dfree(c->d_gabuf); dfree(c->d_gA); dfree(c->d_crhs);
@@ -1397,13 +1399,94 @@ void launch_scatter(int variant, hipStream_t s, int64_t nseg, const int32_t* seg
     else launch_scatter_shape<CODED, false>(variant, s, nseg, seg, src, buf, out, nullptr);
 }
 
+// A segment Σ A[src[p]] (− D[src[p]] after each, with D), p = b..e−1, by one lane: four gathers at a time, for
+// their latency, added in order (60,000 beams twelve between two nodes, :step: 17.4 µs one by one, 11.1 so).
+__device__ __forceinline__ double lane_sum(int32_t b, int32_t e, const uint32_t* __restrict__ src, const double* __restrict__ A,
+                                           const double* __restrict__ D) {
+    double v = 0.;
+    int32_t p = b;
+    for (; p + 4 <= e; p += 4) {
+        const uint32_t q0 = src[p], q1 = src[p + 1], q2 = src[p + 2], q3 = src[p + 3];
+        const double x0 = A[q0], x1 = A[q1], x2 = A[q2], x3 = A[q3];
+        if (D) {
+            const double y0 = D[q0], y1 = D[q1], y2 = D[q2], y3 = D[q3];
+            v += x0; v -= y0; v += x1; v -= y1; v += x2; v -= y2; v += x3; v -= y3;
+        } else {
+            v += x0; v += x1; v += x2; v += x3;
+        }
+    }
+    for (; p < e; ++p) {
+        const uint32_t q = src[p];
+        v += A[q];
+        if (D) v -= D[q];
+    }
+    return v;
+}
+// The same by a whole wave, for a segment of more than kLongSeg contributions (a dof or nz of a node that
+// joins many elements): 64 gathered at a time, the next on their way while one lane's value after the other is
+// added (two v_readlane and an add each). Every lane has the sum. A hub of 63 beams takes 9.6 µs by lanes and
+// 6.7 by waves (:step), of 1,000 253 (one by one) and 51; where every dof has many a wave each is no gain: 60,000
+// beams, 18 contributions a dof 10.4 and 21.0, 32 14.0 and 19.4, 40 16.4 and 19.3, 80 45.8 (one by one) and 21.8.
+constexpr int kLongSeg = 32;
+constexpr int kLongWaves = 4;   // waves, and so segments, of a workgroup
+__device__ __forceinline__ double lane_value(double v, int k) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), k), __builtin_amdgcn_readlane(__double2loint(v), k));
+}
+__device__ __forceinline__ double wave_sum(int32_t b, int32_t e, const uint32_t* __restrict__ src, const double* __restrict__ A,
+                                           const double* __restrict__ D) {
+    const uint32_t lane = threadIdx.x & 63, end = (uint32_t)__builtin_amdgcn_readfirstlane(e);
+    auto gather = [&](uint32_t p, double& x, double& y) {
+        x = y = 0.;
+        if (p + lane < end) {
+            const uint32_t q = src[p + lane];
+            x = A[q];
+            if (D) y = D[q];
+        }
+    };
+    double v = 0., x, y;
+    uint32_t p = (uint32_t)__builtin_amdgcn_readfirstlane(b);
+    gather(p, x, y);
+    for (; p < end; p += 64) {
+        double xn, yn;
+        gather(p + 64, xn, yn);
+        const int m = end - p < 64 ? (int)(end - p) : 64;
+        if (D) {
+#pragma unroll 4
+            for (int k = 0; k < m; ++k) { v += lane_value(x, k); v -= lane_value(y, k); }
+        } else {
+#pragma unroll 8
+            for (int k = 0; k < m; ++k) v += lane_value(x, k);
+        }
+        x = xn; y = yn;
+    }
+    return v;
+}
+// The long segment of this wave of workgroup `tile`, or −1.
+__device__ __forceinline__ int32_t long_of(int64_t tile, int64_t n, const int32_t* __restrict__ list) {
+    const int64_t q = tile * kLongWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    return q < n ? list[q] : -1;
+}
+static_assert(64 * kLongWaves == kBlock, "a wave per segment");
+int64_t long_tiles(int64_t n) { return (n + kLongWaves - 1) / kLongWaves; }
+// Prepare: of n segments (idx: those of these numbers) the ones of more than kLongSeg contributions are counted in
+// *count, and listed (in any order) unless list is null.
+__global__ __launch_bounds__(kBlock) void long_list_kernel(int64_t n, const int32_t* __restrict__ idx, const int32_t* __restrict__ seg,
+                                                           unsigned* __restrict__ count, int32_t* __restrict__ list) {
+    const int64_t q = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (q >= n) return;
+    const int32_t k = idx ? idx[q] : (int32_t)q;
+    if (seg[k + 1] - seg[k] <= kLongSeg) return;
+    const unsigned at = atomicAdd(count, 1u);
+    if (list) list[at] = k;
+}
+
 // The rhs: out[d] = Σ R[src[p]] (− dR[src[p]] after each, on :step: add_value! then
 // add_∂!{1,:minus}, src/SweepX.jl:56-57), a lane per dof in the order of
-// scatter_kernel, and, for the chain solve (pos), also into its right-hand side b or its λ pairs. The
-// first lane hands the NaN flag (the element kernels are done) to the host.
+// scatter_kernel (long segments: a wave), and, for the chain solve (pos), also into its right-hand side b or
+// its λ pairs. The first lane hands the NaN flag (the element kernels are done) to the host.
 struct RhsArgs {
-    int64_t n = 0;
-    const int32_t* seg = nullptr;
+    int64_t n = 0, nlong = 0;
+    const int32_t *seg = nullptr, *longs = nullptr;
     const uint32_t* src = nullptr;
     const double* R = nullptr;
     const double* dR = nullptr;
@@ -1413,15 +1496,8 @@ struct RhsArgs {
     const unsigned long long* flag = nullptr;
     unsigned long long* hflag = nullptr;
 };
-__device__ __forceinline__ void rhs_dof(const RhsArgs& a, int64_t d) {
-    if (d == 0 && a.hflag) *a.hflag = *a.flag;
-    if (d >= a.n) return;
-    double v = 0.;
-    for (int32_t p = a.seg[d], e = a.seg[d + 1]; p < e; ++p) {
-        const uint32_t q = a.src[p];
-        v += a.R[q];
-        if (a.dR) v -= a.dR[q];
-    }
+__host__ __device__ inline int64_t rhs_tiles(const RhsArgs& a) { return (a.n + kBlock - 1) / kBlock; }
+__device__ __forceinline__ void rhs_put(const RhsArgs& a, int64_t d, double v) {
     a.out[d] = v;
     if (a.pos) {
         const int32_t p = a.pos[d];
@@ -1429,7 +1505,24 @@ __device__ __forceinline__ void rhs_dof(const RhsArgs& a, int64_t d) {
         else a.pc[4 * (int64_t)(-p - 1) + 3] = v;
     }
 }
-__global__ __launch_bounds__(kBlock) void rhs_kernel(RhsArgs a) { rhs_dof(a, (int64_t)blockIdx.x * kBlock + threadIdx.x); }
+// Workgroup `tile` of rhs_tiles + long_tiles.
+__device__ __forceinline__ void rhs_tile(const RhsArgs& a, int64_t tile) {
+    const int64_t nt = rhs_tiles(a);
+    if (tile >= nt) {
+        const int32_t d = long_of(tile - nt, a.nlong, a.longs);
+        if (d < 0) return;
+        const double v = wave_sum(a.seg[d], a.seg[d + 1], a.src, a.R, a.dR);
+        if ((threadIdx.x & 63) == 0) rhs_put(a, d, v);
+        return;
+    }
+    const int64_t d = tile * kBlock + threadIdx.x;
+    if (d == 0 && a.hflag) *a.hflag = *a.flag;
+    if (d >= a.n) return;
+    const int32_t p0 = a.seg[d], p1 = a.seg[d + 1];
+    if (p1 - p0 > kLongSeg) return;
+    rhs_put(a, d, lane_sum(p0, p1, a.src, a.R, a.dR));
+}
+__global__ __launch_bounds__(kBlock) void rhs_kernel(RhsArgs a) { rhs_tile(a, blockIdx.x); }
 
 // ---- the nz scatter by nodes -------------------------------------------------
 // The six columns of a node whose elements are beams hold whole 6×6 blocks: one per neighbour and
@@ -1437,15 +1530,19 @@ __global__ __launch_bounds__(kBlock) void rhs_kernel(RhsArgs a) { rhs_dof(a, (in
 // per element and block stands for 36 sources and 36 segment starts. Blocks are numbered in the order
 // of their nz. A wave takes ten: lane 6b + r owns row r of block b and walks the six columns. Each nz is
 // summed in the same element order as in scatter_kernel. The nz of all other columns (Holds, loads,
-// nodes of other kinds) follow in the same launch, a lane each.
+// nodes of other kinds or of many elements) follow in the same launch, a lane each or, long, a wave.
 // Bound: HBM. The index traffic falls from 8 B a nz to 16 B a block; stores go through L2, where the
 // rows of a line meet (written past it they cost 244 µs instead of 180). 383,000 beams in chains: 237 µs
 // for the best segmented shape, 180 here.
 constexpr int kNodeWaves = 4, kWaveBlocks = 10;
+static_assert(64 * kNodeWaves == kBlock, "tiles of the rhs and of long segments");
 constexpr int kNodeUnits = 4;   // tens of blocks a wave takes one after another
+// Sources of a block gathered together, for their latency. One at a time, two, three and four: a hub of 63
+// beams 19.4, 14.1, 11.8 and 11.2 µs, 60,000 beams twelve between two nodes 25.1, 22.0, 20.9 and 21.2 µs.
+constexpr int kNodeGather = 4;
 struct NodeArgs {
     NodeMap m;
-    int64_t per_xcd, ntile, nrest;   // tiles of blocks, then of `rest`, then of the rhs
+    int64_t per_xcd, ntile, nrest, nlong;   // tiles of blocks, then of `rest`, of `longs`, then of the rhs
     int units;
     RhsArgs rhs;
     const int32_t* seg;
@@ -1462,20 +1559,28 @@ __global__ __launch_bounds__(64 * kNodeWaves) void node_scatter_kernel(NodeArgs 
         const int64_t o = IDX ? (int64_t)__builtin_nontemporal_load(a.dst + k) : k;
         a.out[o] = v;
     };
-    if (tile >= a.ntile + a.nrest) {
-        if (a.rhs.seg) rhs_dof(a.rhs, (tile - a.ntile - a.nrest) * (64 * kNodeWaves) + t);
-        return;
-    }
-    if (tile >= a.ntile) {
-        const int64_t q = (tile - a.ntile) * (64 * kNodeWaves) + t;
-        if (q >= a.m.nrest) return;
-        const int64_t k = a.m.rest[q];
-        double v = 0.;
-        for (int32_t p = a.seg[k], e = a.seg[k + 1]; p < e; ++p) v += a.K[a.src[p]];
-        put(k, v);
-        return;
-    }
     const int l = t & 63, w = t >> 6, r = l % 6;
+    if (tile >= a.ntile) {
+        int64_t q = tile - a.ntile;
+        if (q < a.nrest) {
+            const int64_t i = q * (64 * kNodeWaves) + t;
+            if (i >= a.m.nrest) return;
+            const int64_t k = a.m.rest[i];
+            const int32_t p0 = a.seg[k], p1 = a.seg[k + 1];
+            if (p1 - p0 <= kLongSeg) put(k, lane_sum(p0, p1, a.src, a.K, nullptr));
+            return;
+        }
+        q -= a.nrest;
+        if (q < a.nlong) {
+            const int32_t k = long_of(q, a.m.nlong, a.m.longs);
+            if (k < 0) return;
+            const double v = wave_sum(a.seg[k], a.seg[k + 1], a.src, a.K, nullptr);
+            if (l == 0) put(k, v);
+            return;
+        }
+        if (a.rhs.seg) rhs_tile(a.rhs, q - a.nlong);
+        return;
+    }
     if (l >= 6 * kWaveBlocks) return;   // no barrier below
     for (int u = 0; u < a.units; ++u) {
         const int64_t b = ((tile * kNodeWaves + w) * a.units + u) * kWaveBlocks + l / 6;
@@ -1485,8 +1590,23 @@ __global__ __launch_bounds__(64 * kNodeWaves) void node_scatter_kernel(NodeArgs 
         double v[6];
 #pragma unroll
         for (int c = 0; c < 6; ++c) v[c] = 0.;
-        for (int j = 0; j < n; ++j) {
-            const double* k = a.K + (uint32_t)(j == 0 ? h.w : (int)a.m.src[h.z + j]) + r;
+        const uint32_t* src = a.m.src + h.z;
+        int j = 0;
+        for (; j + kNodeGather <= n; j += kNodeGather) {
+            double x[kNodeGather][6];
+#pragma unroll
+            for (int i = 0; i < kNodeGather; ++i) {
+                const double* k = a.K + src[j + i] + r;
+#pragma unroll
+                for (int c = 0; c < 6; ++c) x[i][c] = k[12 * c];
+            }
+#pragma unroll
+            for (int i = 0; i < kNodeGather; ++i)
+#pragma unroll
+                for (int c = 0; c < 6; ++c) v[c] += x[i][c];
+        }
+        for (; j < n; ++j) {
+            const double* k = a.K + (j == 0 ? (uint32_t)h.w : src[j]) + r;
 #pragma unroll
             for (int c = 0; c < 6; ++c) v[c] += k[12 * c];
         }
@@ -1506,7 +1626,8 @@ void launch_node_scatter(const NodeMap& m, hipStream_t s, const int32_t* seg, co
     const int64_t per = (int64_t)kNodeWaves * a.units * kWaveBlocks;
     a.ntile = (m.nblock + per - 1) / per;
     a.nrest = (m.nrest + 64 * kNodeWaves - 1) / (64 * kNodeWaves);
-    const int64_t nt = a.ntile + a.nrest + (rhs.n + 64 * kNodeWaves - 1) / (64 * kNodeWaves);
+    a.nlong = long_tiles(m.nlong);
+    const int64_t nt = a.ntile + a.nrest + a.nlong + rhs_tiles(rhs) + long_tiles(rhs.nlong);
     a.per_xcd = (nt + kXCD - 1) / kXCD;
     const dim3 gr((unsigned)(a.per_xcd * kXCD)), bl(64 * kNodeWaves);
     if (dst) hipLaunchKernelGGL((node_scatter_kernel<true>), gr, bl, 0, s, a);
@@ -1527,45 +1648,49 @@ __global__ __launch_bounds__(kBlock) void node_base_kernel(int64_t nele, const i
             for (int k = 0; k < 6; ++k) atomicOr(f + idx[(int64_t)(6 * h + k) * nele + e], 2);
     }
 }
-// Whether J is the base of a node whose columns are whole blocks, every source where block_source
-// says; its blocks and sources counted. dp: the block of rows J.
-__device__ inline bool node_check(int64_t J, int64_t nX, const int32_t* __restrict__ f, const int32_t* __restrict__ colptr,
-                                  const int32_t* __restrict__ rowval, const int32_t* __restrict__ seg,
-                                  const uint32_t* __restrict__ src, int& m, int& ns, int& dp) {
-    if (J + 6 > nX || f[J] != 1) return false;
-    for (int k = 1; k < 6; ++k) if (f[J + k] != 0) return false;
+// Whether J is the base of a node whose columns are whole blocks, every source at its place in its element's
+// 12×12; its blocks m and sources ns counted. By a whole wave, a lane per nz: a node may have any number of blocks.
+__device__ inline bool node_check(int64_t J, const int32_t* __restrict__ colptr, const int32_t* __restrict__ rowval,
+                                  const int32_t* __restrict__ seg, const uint32_t* __restrict__ src, int& m, int& ns) {
+    const int lane = threadIdx.x & 63;
     const int32_t k0 = colptr[J], len = colptr[J + 1] - k0;
-    if (len % 6 != 0 || len == 0 || len > 6 * 64) return false;
-    m = len / 6; ns = 0; dp = -1;
+    m = ns = 0;
+    if (len % 6 != 0 || len == 0 || len > 0xffff) return false;
     for (int c = 1; c < 6; ++c) if (colptr[J + c + 1] - colptr[J + c] != len) return false;
-    for (int b = 0; b < m; ++b) {
-        const int32_t I = rowval[k0 + 6 * b], k00 = k0 + 6 * b;
-        if (I == J) dp = b;
-        const int nc = seg[k00 + 1] - seg[k00];
-        if (nc < 1 || nc > 0x7fff) return false;
-        ns += nc;
-        for (int c = 0; c < 6; ++c)
-            for (int r = 0; r < 6; ++r) {
-                const int32_t k = k00 + c * len + r;
-                if (rowval[k] != I + r || seg[k + 1] - seg[k] != nc) return false;
-            }
-        for (int j = 0; j < nc; ++j)   // element j's entries at their places in its 12×12
-            for (int c = 0; c < 6; ++c)
-                for (int r = 0; r < 6; ++r)
-                    if (src[seg[k00 + c * len + r] + j] != src[seg[k00] + j] + (uint32_t)(r + 12 * c)) return false;
+    m = len / 6;
+    bool diagonal = false;
+    for (int q0 = 0; q0 < 36 * m; q0 += 64) {
+        const int q = q0 + lane, b = q / 36, e = q - 36 * b, c = e / 6, r = e - 6 * c;
+        bool ok = true;
+        if (q < 36 * m) {
+            const int32_t k00 = k0 + 6 * b, k = k00 + c * len + r, I = rowval[k00], p0 = seg[k00], p = seg[k];
+            const int nc = seg[k00 + 1] - p0;
+            ok = nc >= 1 && nc <= 0x7fff && rowval[k] == I + r && seg[k + 1] - p == nc;
+            for (int j = 0; j < nc && ok; ++j) ok = src[p + j] == src[p0 + j] + (uint32_t)(r + 12 * c);
+            if (e == 0) ns += nc;
+            diagonal = diagonal || I == J;
+        }
+        if (__any(!ok)) return false;
     }
-    return dp >= 0;
+    for (int o = 32; o > 0; o /= 2) ns += __shfl_xor(ns, o);
+    return __any(diagonal);
 }
-// cnt: 4 × (nX + 1): node, blocks, sources, other nz of each column.
+// cnt: 4 × (nX + 1): node, blocks, sources, other nz of each column. A wave per 64 dofs takes the bases among them
+// one after the other.
 __global__ __launch_bounds__(kBlock) void node_count_kernel(int64_t nX, const int32_t* __restrict__ f, const int32_t* __restrict__ colptr,
                                                             const int32_t* __restrict__ rowval, const int32_t* __restrict__ seg,
                                                             const uint32_t* __restrict__ src, int32_t* __restrict__ cnt) {
-    const int64_t J = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (J > nX) return;
-    int m = 0, ns = 0, dp = 0;
-    const bool ok = J < nX && node_check(J, nX, f, colptr, rowval, seg, src, m, ns, dp);
-    const int64_t n1 = nX + 1;
-    cnt[J] = ok; cnt[n1 + J] = ok ? m : 0; cnt[2 * n1 + J] = ok ? ns : 0;
+    const int64_t J = (int64_t)blockIdx.x * kBlock + threadIdx.x, J0 = J - (threadIdx.x & 63), n1 = nX + 1;
+    bool base = J + 6 <= nX && f[J] == 1;
+    for (int k = 1; k < 6; ++k) base = base && f[J + k] == 0;
+    int ok = 0, m = 0, ns = 0;
+    for (unsigned long long todo = __ballot(base); todo; todo &= todo - 1) {
+        const int i = __builtin_ctzll(todo);
+        int mi, nsi;
+        const bool oki = node_check(J0 + i, colptr, rowval, seg, src, mi, nsi);
+        if ((int)(threadIdx.x & 63) == i && oki) { ok = 1; m = mi; ns = nsi; }
+    }
+    if (J <= nX) { cnt[J] = ok; cnt[n1 + J] = m; cnt[2 * n1 + J] = ns; }
 }
 __global__ __launch_bounds__(kBlock) void node_rest_kernel(int64_t nX, const int32_t* __restrict__ ok, const int32_t* __restrict__ colptr,
                                                            int32_t* __restrict__ rest) {
@@ -1584,11 +1709,12 @@ __global__ __launch_bounds__(kBlock) void node_fill_kernel(int64_t nX, const int
     const int64_t n1 = nX + 1;
     if (J == nX) return;
     if (cnt[J]) {
-        const int32_t b0 = pos[n1 + J], k0 = colptr[J], len = colptr[J + 1] - k0;
+        const int32_t k0 = colptr[J], len = colptr[J + 1] - k0;
+        const int32_t at = pos[n1 + J];
         int32_t p = pos[2 * n1 + J];
         for (int b = 0; b < len / 6; ++b) {
             const int32_t k00 = k0 + 6 * b, nc = seg[k00 + 1] - seg[k00];
-            o.blk[b0 + b] = make_int4(k00, len | nc << 16, p, (int)src[seg[k00]]);
+            o.blk[at + b] = make_int4(k00, len | nc << 16, p, (int)src[seg[k00]]);
             for (int j = 0; j < nc; ++j) o.src[p++] = src[seg[k00] + j];
         }
     }
@@ -1990,7 +2116,26 @@ static int tune_scatter(Ctx* c, double* out, bool pick) {
     return MH_OK;
 }
 
-// The node map of the prepared nz maps (nmap.nblock = 0 when no beam node has whole-block columns).
+// The long ones of n segments (idx: of those numbers), listed.
+static int build_long(Ctx* c, int64_t n, const int32_t* idx, const int32_t* seg, int64_t& nlong, int32_t*& list) {
+    hipStream_t s = c->stream;
+    unsigned* count = c->d_cflag;   // a word that every call that uses it resets
+    unsigned h = 0;
+    auto run = [&](int32_t* to) {
+        hipLaunchKernelGGL(fill_u64, dim3(1), dim3(1), 0, s, reinterpret_cast<unsigned long long*>(count), 0ull);
+        if (n) hipLaunchKernelGGL(long_list_kernel, dim3(grid(n)), dim3(kBlock), 0, s, n, idx, seg, count, to);
+    };
+    run(nullptr);
+    HIPCHK(c, hipMemcpyAsync(&h, count, sizeof(h), hipMemcpyDeviceToHost, s));
+    HIPCHK(c, hipStreamSynchronize(s));
+    nlong = h;
+    if (h == 0) return MH_OK;
+    HIPCHK(c, dneed(list, nlong));
+    run(list);
+    return check_launch(c, "long sums");
+}
+
+// The node map of the prepared nz maps (nblock = 0 when no beam node has whole-block columns).
 static int build_node_map(Ctx* c) {
     hipStream_t s = c->stream;
     const int64_t nX = c->nX, n1 = nX + 1;
@@ -2024,6 +2169,7 @@ static int build_node_map(Ctx* c) {
         HIPCHK(c, hipMalloc(&m.rest, sizeof(int32_t) * std::max(tot[3], 1)));
         hipLaunchKernelGGL(node_fill_kernel, dim3(grid(n1)), dim3(kBlock), 0, s, nX, cnt, pos, c->d_colptr, c->d_rowval,
                            c->d_kseg, c->d_ksrc, m);
+        if (int r = build_long(c, m.nrest, m.rest, c->d_kseg, m.nlong, m.longs)) return r;
     }
     if (int r = check_launch(c, "node map")) return r;
     HIPCHK(c, hipStreamSynchronize(s));
@@ -2510,6 +2656,7 @@ int mh_prepare_sweepx(mh_ctx* c, int OX, int64_t* nnz_out) {
     HIPCHK(c, hipStreamSynchronize(s));
     dfree(kin); dfree(kout); dfree(vin); dfree(head); dfree(id); dfree(colk);
     if (int r = build_rmap(c)) return r;
+    if (int r = build_long(c, nX, nullptr, c->d_rseg, c->nrlong, c->d_rlong)) return r;
     unsigned int *rkin = nullptr, *rkout = nullptr;
     uint32_t* rvin = nullptr;
     // ---- U-dof map (gradients ∂L/∂U of the adjoint), same construction over the U class
@@ -2738,7 +2885,7 @@ static int enqueue_sweepx(Ctx* c, int OX, bool step, const double* c6, bool time
     if (int r = check_launch(c, "element kernels")) return r;
     if (timed) HIPCHK(c, hipEventRecord(c->ev[1], s));
     RhsArgs rh;
-    rh.n = c->nX; rh.seg = c->d_rseg; rh.src = c->d_rsrc; rh.R = c->d_Rbuf; rh.dR = step ? c->d_dRbuf : nullptr; rh.out = c->d_rhs;
+    rh.n = c->nX; rh.nlong = c->nrlong; rh.longs = c->d_rlong; rh.seg = c->d_rseg; rh.src = c->d_rsrc; rh.R = c->d_Rbuf; rh.dR = step ? c->d_dRbuf : nullptr; rh.out = c->d_rhs;
     rh.flag = c->d_flag; rh.hflag = c->h_flag;
     if (fused) { rh.pos = c->d_cpos; rh.b = c->d_cbuf + 3 * c->cnb * c->cB * c->cB; rh.pc = pc; }
     double* out = fused ? c->d_cbuf : c->d_nzval;
@@ -2752,7 +2899,8 @@ static int enqueue_sweepx(Ctx* c, int OX, bool step, const double* c6, bool time
         else launch_scatter<false>(c->scatter_variant, s, c->nnz, c->d_kseg, c->d_ksrc, c->d_Kbuf, out, dst);
     }
     if (timed) HIPCHK(c, hipEventRecord(c->ev[2], s));
-    if (!joined) hipLaunchKernelGGL(rhs_kernel, dim3(std::max(grid(c->nX), 1u)), dim3(kBlock), 0, s, rh);
+    if (!joined)
+        hipLaunchKernelGGL(rhs_kernel, dim3((unsigned)std::max<int64_t>(rhs_tiles(rh) + long_tiles(rh.nlong), 1)), dim3(kBlock), 0, s, rh);
     if (timed) HIPCHK(c, hipEventRecord(c->ev[3], s));
     return check_launch(c, "scatter kernels");
 }
@@ -3070,6 +3218,8 @@ int mh_get_scatter(mh_ctx* c, int64_t* info) {
     info[2] = c->nmap.nrest;
     info[3] = c->use_nodes ? node_units(c->nmap) : 0;
     info[4] = joins_rhs(c);
+    info[5] = c->nmap.nlong;
+    info[6] = c->nrlong;
     return MH_OK;
 }
 

@@ -18,9 +18,9 @@ def mc():
 
 
 def info(mc, out):
-    v = np.zeros(5, np.int64)
+    v = np.zeros(7, np.int64)
     out.ctx.check(mc.lib.mh_get_scatter(out.ctx.h, mc._lib.i64ptr(v)), "scatter")
-    return dict(zip(("nodes", "blocks", "rest", "tens", "joined"), v.tolist()))
+    return dict(zip(("nodes", "blocks", "rest", "tens", "joined", "long", "rlong"), v.tolist()))
 
 
 def chain(mc, n):
