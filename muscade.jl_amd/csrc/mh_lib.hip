@@ -113,6 +113,7 @@ struct Ctx {
     int64_t nK = 0, nP = 0, nR = 0, nnz = 0;
     double* d_Kc = nullptr;      // dynamic beams: scaled compact static part, 45 per element
     double* d_rec = nullptr;     // dynamic beams: the elements' records (mh::DynRec), in tiles of kDynTile
+    int rec_nd = 0;              // time levels that d_rec has room for
     // words of one call: uploaded in one copy ahead of its kernels (upload_call), and the results its
     // last kernels leave in pinned host memory
     CallWords* d_call = nullptr;
@@ -283,7 +284,7 @@ void free_prepared(Ctx* c) {
     free_graph(c);
     free_chain(c);
     free_big(c);
-    dfree(c->d_Kbuf); dfree(c->d_Rbuf); dfree(c->d_dRbuf); dfree(c->d_nzval); dfree(c->d_rhs); dfree(c->d_Kc); dfree(c->d_rec);
+    dfree(c->d_Kbuf); dfree(c->d_Rbuf); dfree(c->d_dRbuf); dfree(c->d_nzval); dfree(c->d_rhs); dfree(c->d_Kc); dfree(c->d_rec); c->rec_nd = 0;
     dfree(c->d_colptr); dfree(c->d_rowval); dfree(c->d_kseg); dfree(c->d_ksrc); dfree(c->d_rseg); dfree(c->d_rsrc);
     dfree(c->nmap.blk); dfree(c->nmap.rest); dfree(c->nmap.src); dfree(c->nmap.longs); dfree(c->d_rlong); c->nrlong = 0;
     c->nmap = NodeMap(); c->use_nodes = false;
@@ -533,10 +534,13 @@ __device__ __forceinline__ void dyn_load(const BeamDynArgs& a, int64_t e, mh::Be
 // records (1,096 B an element at second order). From time jets it took 19,400 instructions and one
 // wave per SIMD, in closed form 8,800; 383,000 elements, second order: 362 µs before, 219 now.
 constexpr int kDynTile = 64;   // elements whose records lie together
-constexpr int kDynRecMax = mh::kDynRec<3>;
 constexpr int kValueBlock = 64;   // one wave: the LDS tile of the compact tangents lets seven share a CU
 static_assert(kValueBlock % kDynTile == 0, "whole tiles per workgroup");
-int64_t rec_numbers(int64_t nele) { return (nele + kDynTile - 1) / kDynTile * kDynTile * kDynRecMax; }
+// Numbers of a group's records for nd time levels.
+int64_t rec_numbers(int64_t nele, int nd) {
+    const int rec = nd == 1 ? mh::kDynRec<1> : nd == 2 ? mh::kDynRec<2> : mh::kDynRec<3>;
+    return (nele + kDynTile - 1) / kDynTile * kDynTile * rec;
+}
 template <int ND, bool UDOF>
 __global__ __launch_bounds__(kValueBlock, 2) void beam_dyn_value_kernel(BeamDynArgs a) {
     __shared__ double tile[kValueBlock * mh::kCompact];
@@ -2081,6 +2085,31 @@ static int upload_soa(Ctx* c, T** dst, const T* src, int n, int64_t nele) {
 }
 
 
+// The compact static parts and the records of the beams for nd time levels. Records of fewer levels make way
+// once there is room for the larger ones (an adjoint of a higher order than was prepared); what is left out of a
+// record at lower order is most of it: 456, 552 and 1,096 B a beam for one, two and three levels.
+static int dyn_buffers(Ctx* c, int nd) {
+    int64_t nKc = 0, nRec = 0;
+    auto beam = [](const Group& g) { return g.kind == MH_KIND_BEAM || g.kind == MH_KIND_BEAM_U; };
+    for (auto& g : c->groups)
+        if (beam(g)) { g.kcbase = nKc; nKc += g.nele * mh::kCompact; nRec += rec_numbers(g.nele, nd); }
+    if (nKc == 0) return MH_OK;
+    HIPCHK(c, dneed(c->d_Kc, nKc));
+    if (c->rec_nd >= nd) return MH_OK;
+    double* rec = nullptr;
+    HIPCHK(c, dneed(rec, nRec));
+    if (c->d_rec) {
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+        dfree(c->d_rec);
+        ++c->gen;   // a captured graph holds the old records
+    }
+    c->d_rec = rec; c->rec_nd = nd;
+    nRec = 0;
+    for (auto& g : c->groups)
+        if (beam(g)) { g.recbase = nRec; nRec += rec_numbers(g.nele, nd); }
+    return MH_OK;
+}
+
 // Tuner: time each shape of the segmented nz scatter on the prepared maps, into out, and keep (pick) the
 // fastest. The sums are identical for every shape (each segment is summed in the same order).
 static int tune_scatter(Ctx* c, double* out, bool pick) {
@@ -2571,7 +2600,7 @@ int mh_prepare_sweepx(mh_ctx* c, int OX, int64_t* nnz_out) {
     free_prepared(c);
     // contribution counts and buffer offsets, in eletype order. Static beams store the
     // compact tangent; dynamic beams (K + a₁C + b₁M is not symmetric) the full block.
-    int64_t nK = 0, nP = 0, nR = 0, nKc = 0, nRec = 0, nRU = 0, nRA = 0;
+    int64_t nK = 0, nP = 0, nR = 0, nRU = 0, nRA = 0;
     bool coded = false;
     for (auto& g : c->groups) {
         g.ubase = nRU;
@@ -2583,9 +2612,6 @@ int mh_prepare_sweepx(mh_ctx* c, int OX, int64_t* nnz_out) {
         coded = coded || g.compact;
         g.kper = g.compact ? mh::kCompact : (int64_t)g.nX * g.nX;
         g.kbase = nK; g.rbase = nR;
-        g.kcbase = nKc;
-        g.recbase = nRec;
-        if (beam && OX > 0) { nKc += g.nele * mh::kCompact; nRec += rec_numbers(g.nele); }
         nK += g.nele * g.kper;
         nP += g.nele * g.nX * g.nX;
         nR += g.nele * g.nX;
@@ -2601,8 +2627,8 @@ int mh_prepare_sweepx(mh_ctx* c, int OX, int64_t* nnz_out) {
     HIPCHK(c, hipMalloc(&c->d_Kbuf, sizeof(double) * std::max<int64_t>(nK, 1)));
     HIPCHK(c, hipMalloc(&c->d_Rbuf, sizeof(double) * std::max<int64_t>(nR, 1)));
     HIPCHK(c, hipMalloc(&c->d_dRbuf, sizeof(double) * std::max<int64_t>(nR, 1)));
-    if (nKc) HIPCHK(c, hipMalloc(&c->d_Kc, sizeof(double) * nKc));
-    if (nRec) HIPCHK(c, hipMalloc(&c->d_rec, sizeof(double) * nRec));
+    if (OX > 0)
+        if (int r = dyn_buffers(c, OX + 1)) return r;
     HIPCHK(c, hipMalloc(&c->d_rhs, sizeof(double) * std::max<int64_t>(nX, 1)));
     HIPCHK(c, hipMalloc(&c->d_colptr, sizeof(int32_t) * (nX + 1)));
     // ---- matrix pairs
@@ -3035,16 +3061,8 @@ int mh_vjp_lagrangian(mh_ctx* c, int OX, mh_err* err) {
         HIPCHK(c, dneed(c->d_gabuf, c->nRA));
         HIPCHK(c, dneed(c->d_gA, c->nA));
     }
-    if (OX > 0) {
-        int64_t nKc = 0, nRec = 0;
-        for (auto& g : c->groups)
-            if (g.kind == MH_KIND_BEAM || g.kind == MH_KIND_BEAM_U) {
-                g.kcbase = nKc; nKc += g.nele * mh::kCompact;
-                g.recbase = nRec; nRec += rec_numbers(g.nele);
-            }
-        if (nKc) HIPCHK(c, dneed(c->d_Kc, nKc));
-        if (nRec) HIPCHK(c, dneed(c->d_rec, nRec));
-    }
+    if (OX > 0)
+        if (int r = dyn_buffers(c, nd)) return r;
     hipLaunchKernelGGL(fill_u64, dim3(1), dim3(1), 0, s, c->d_flag, ~0ull);
     HIPCHK(c, hipEventRecord(c->ev[0], s));
     for (size_t gi = 0; gi < c->groups.size(); ++gi) {
@@ -3254,17 +3272,16 @@ int mh_prepare_direct(mh_ctx* c, int OX, int OU, int IA, int64_t* nnz4) {
     free_prepared(c);
     // A-dofs reach the device only through A-scaled beams: their section follows A (mh_set_A)
     // and their A column comes from mh_beam_dRdA, outside these blocks
-    int64_t nR = 0, nKd = 0, nKU = 0, nKc = 0, nRec = 0;
+    int64_t nR = 0, nKd = 0, nKU = 0;
     for (auto& g : c->groups) {
         if (g.kind == MH_KIND_ZERO || g.kind == MH_KIND_HOST) {
             c->err = "elements with user functions (DofCost, DofConstraint) are not evaluated on the device in AssemblyDirect";
             return MH_ERR_ARG;
         }
-        g.rbase = nR; g.kdbase = nKd; g.kubase = nKU; g.kcbase = nKc; g.recbase = nRec;
+        g.rbase = nR; g.kdbase = nKd; g.kubase = nKU;
         nR += g.nele * g.nX;
         nKd += g.nele * g.nX * g.nX;
         nKU += g.nele * g.nX * g.nU;
-        if (g.kind == MH_KIND_BEAM || g.kind == MH_KIND_BEAM_U) { nKc += g.nele * mh::kCompact; nRec += rec_numbers(g.nele); }
     }
     if (nR >= (int64_t)UINT32_MAX || nKd >= (int64_t)UINT32_MAX) { c->err = "too many element outputs for 32-bit maps"; return MH_ERR_SIZE; }
     c->nR = nR; c->nKd = nKd; c->nKU = nKU;
@@ -3286,8 +3303,7 @@ int mh_prepare_direct(mh_ctx* c, int OX, int OU, int IA, int64_t* nnz4) {
     if (int r = build_dmap(c, uu, c->nU, c->nU, false, false, c->dUU)) return r;
     HIPCHK(c, hipMalloc(&c->d_Kd, sizeof(double) * std::max<int64_t>((OX + 1) * nKd, 1)));
     HIPCHK(c, hipMalloc(&c->d_KU, sizeof(double) * std::max<int64_t>(nKU, 1)));
-    HIPCHK(c, hipMalloc(&c->d_Kc, sizeof(double) * std::max<int64_t>(nKc, 1)));
-    HIPCHK(c, hipMalloc(&c->d_rec, sizeof(double) * std::max<int64_t>(nRec, 1)));
+    if (int r = dyn_buffers(c, OX + 1)) return r;
     HIPCHK(c, hipMalloc(&c->d_Rd, sizeof(double) * std::max<int64_t>(nR, 1)));
     HIPCHK(c, hipMalloc(&c->d_L1x, sizeof(double) * std::max<int64_t>(nR, 1)));
     // residual-path elements (beams, bars) add nothing to L1[X] and never write their slots

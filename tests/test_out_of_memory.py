@@ -120,6 +120,35 @@ def with_newton(a):
     chained(a)
     newton(a)
 
+if sys.argv[3] == "records":   # 64 to a tile, 69 and 137 numbers a record at first and second order, 57 without derivatives
+    def records(numbers):
+        return 2 * 64 * numbers * 8      # the two groups' tiles
+    a = context(1)
+    with_lambda(a)
+    assert records(69) in live() and records(137) not in live(), live()
+    vjp(a, 1)
+    assert records(69) in live(), live()
+    vjp(a, 2)
+    assert records(137) in live() and records(69) not in live(), live()
+    vjp(a, 1)
+    assert records(137) in live(), live()
+    del a
+    a = context(1)                       # no room for the larger ones: the smaller ones stay
+    with_lambda(a)
+    vjp(a, 1)
+    stand_in.stand_in_fail_at(0)
+    assert "out of memory" in vjp(a, 2)
+    assert records(69) in live()
+    vjp(a, 2)
+    assert records(137) in live() and records(69) not in live(), live()
+    del a
+    a = context(0)
+    assert not {records(57), records(69), records(137)} & set(live()), live()
+    d = mc.AssemblyDirect(0, 0, 0, a.model, a.dis, nA=a.model.ndof["A"])
+    assert records(57) in live(), live()
+    print("checked")
+    sys.exit()
+
 cases = {"adjoint of a static preparation": (0, with_lambda, lambda a: vjp(a, 2)),
          "adjoint": (2, with_lambda, lambda a: vjp(a, 2)),
          "sparse adjoint solve": (0, with_newton, sparse),
@@ -166,4 +195,9 @@ def stand_in(tmp_path_factory):
 @pytest.mark.parametrize("call", ["adjoint of a static preparation", "adjoint", "sparse adjoint solve", "decrement"])
 def test_failed_allocation_leaves_nothing_half_made(stand_in, call):
     r = subprocess.run([sys.executable, "-c", PROGRAM, str(stand_in), ROOT, call], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0 and "checked" in r.stdout, r.stdout[-2000:] + r.stderr[-3000:]
+
+
+def test_records_take_the_order_in_use(stand_in):
+    r = subprocess.run([sys.executable, "-c", PROGRAM, str(stand_in), ROOT, "records"], capture_output=True, text=True, timeout=300)
     assert r.returncode == 0 and "checked" in r.stdout, r.stdout[-2000:] + r.stderr[-3000:]
