@@ -1134,10 +1134,11 @@ struct DirectArgs {
 // Beams, after the value pass with unit scales: a workgroup per tile of elements and lanes as in
 // the SweepX direction pass. The X₀ pass gives the Jacobian's rows (LDS) and ∂R/∂X₀; then the loads
 // are differentiated along X′ₖ and X″ₖ; ∂R/∂U = −Σ_gp dL J_xᵀ, a lane its two rows. Bound: latency (a
-// step's few beams fill a few CUs; the loop over orders spills 1,168 B a lane): 230 beams, second order,
-// 86 µs on jets, 82 here.
+// step's few beams fill a few CUs). One wave per SIMD: bounded to 256 registers for two, the loop over orders
+// spilled 1,168 B a lane at second order (148 now). With the value pass, second order, on jets, in two waves and in
+// one: 230 beams 131, 100 and 68 µs, 100,000 beams 2,498, 1,057 and 483 µs.
 template <int ND, bool UDOF>
-__global__ __launch_bounds__(kDirLanes, 2) void beam_direct_kernel(DirectArgs a) {
+__global__ __launch_bounds__(kDirLanes) void beam_direct_kernel(DirectArgs a) {
     __shared__ DynElem<ND> lds[kDirTile];
     __shared__ mh::DirRow rows[kDirTile][6];
     const int64_t e0 = xcd_tile(a.per_xcd) * kDirTile;
