@@ -6,7 +6,7 @@
 //   node spins      t_n = rᵀ T(v_n) δv_n  (T = I + bS + cS², the left Jacobian of Rodrigues)
 //   frame spin      ω   = ½(s − τ φ×Δ),  s = t₁+t₂, Δ = t₂−t₁, τ = tan(|φ|/4)/|φ|
 //   δvₗ             =  ½Δ + κ φ×(φ×Δ),   κ = ½e − ¼τ (e of T⁻¹),   φ = rᵀφ = 2vₗ
-// (W of beam_static is [Pᵀ T₁ | P T₂] with P = (I + Rodrigues(φ/2))⁻¹ = ½(I − τ spin φ), and a
+// (ω = Pᵀt₁ + Pt₂ with P = (I + Rodrigues(φ/2))⁻¹ = ½(I − τ spin φ), and a
 // rigid spin moves vₗ not at all), all of them time jets. Along a rotation
 //   δx_gp = r·((yu − ya) A + yv B),  A = (ω_y d_z − ω_z d_y, −d_x ω_z, d_x ω_y),
 //   B = (−ω_y v_y − ω_z v_z, ω_x v_y + δv_z, ω_x v_z − δv_y),  d = uₗ + (L/2, 0, 0), v = vₗ,

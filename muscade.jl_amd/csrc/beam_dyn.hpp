@@ -1,31 +1,23 @@
-// Dynamic EulerBeam3D (X with time derivatives, OX = 1 or 2): time jets of the
-// corotated kinematics and the inertia, added-mass, damping and roll-inertia loads.
+// Requestables and strain gauges of EulerBeam3D on jets: the corotated kinematics with their time
+// derivatives, the inertia, added-mass, damping and roll-inertia loads, and first and second derivatives of
+// the gauges' strains. (The solver's residual and tangent are in closed form: beam_math.hpp, beam_dir.hpp.)
 //
 // Reference: toolbox/BeamElement.jl:28-64 (resultants), :151-208 (residual,
 // kinematics, corotated), toolbox/Rotations.jl:13-182, src/Taylor.jl:24-65
-// (motion / motion⁻¹), src/SweepX.jl:45-74 (the solver's trial path).
+// (motion / motion⁻¹), src/Output.jl:131-181 (getresult).
 //
-// Muscade evaluates the element on nested forward-mode duals: two time levels
-// (motion{P}) around the solver partials. Two things follow, and are reproduced:
+// getresult evaluates the element on plain values, so every formula, squares among them, is exact calculus
+// on its time levels.
 //
-//   * time derivatives are exact calculus through every formula, except that
-//     the integer power rule of src/Adiff.jl:230 (a^0 → zero(a)) drops the
-//     cross-level term of a square taken on a two-level time jet: for the
-//     `sinc1(θ/2)^2` of Rodrigues (Rotations.jl:134) the second time
-//     derivative is 2·s·s̈ instead of 2·s·s̈ + 2·ṡ². `jsq_muscade` below;
-//   * the solver's tangent is the derivative along one trial direction ε:
-//     X₀ + ε·e, X₁ + ε·a₁e, X₂ + ε·b₁e (:iter) or X₁ + ε·a, X₂ + ε·b (the δr
-//     partial of :step).
-//
-// `Jet<NT,E>` carries q(t,ε) truncated at order NT-1 in t and 1 in ε:
-// v[n] = ∂ⁿq/∂tⁿ and e[n] = ∂(∂ⁿq/∂tⁿ)/∂ε.  With E = false it is the plain time
-// jet (value pass).
+// `Jet<NT,E>` carries q(t,ε) truncated at order NT-1 in t and 1 in ε, at most second order in all:
+// v[n] = ∂ⁿq/∂tⁿ and e[n] = ∂(∂ⁿq/∂tⁿ)/∂ε.  With E = false it is the plain time jet.
 #pragma once
 #include "beam_math.hpp"
 
 namespace mh {
 
 template <int NT, bool E> struct Jet {
+    static_assert(NT + (E ? 1 : 0) <= 3, "second order in all");
     double v[NT];
     double e[E ? NT : 1];
 };
@@ -88,14 +80,10 @@ template <int NT, bool E> MH_HD Jet<NT, E> operator*(const Jet<NT, E>& a, const 
     if constexpr (E) {
         r.e[0] = a.e[0] * b.v[0] + a.v[0] * b.e[0];
         if constexpr (NT > 1) r.e[1] = (a.e[1] * b.v[0] + a.v[1] * b.e[0]) + (a.e[0] * b.v[1] + a.v[0] * b.e[1]);
-        if constexpr (NT > 2)
-            r.e[2] = (a.e[2] * b.v[0] + a.v[2] * b.e[0]) + 2. * (a.e[1] * b.v[1] + a.v[1] * b.e[1]) +
-                     (a.e[0] * b.v[2] + a.v[0] * b.e[2]);
     } else r.e[0] = 0.;
     return r;
 }
-// Composition with a scalar function given f, f', f'', f''' at a.v[0] (chain rule
-// to third total order: two in t, one in ε).
+// Composition with a scalar function given f, f', f'' at a.v[0].
 template <int NT, bool E> MH_HD Jet<NT, E> jfun(const Jet<NT, E>& a, const double* f) {
     Jet<NT, E> r;
     r.v[0] = f[0];
@@ -104,26 +92,9 @@ template <int NT, bool E> MH_HD Jet<NT, E> jfun(const Jet<NT, E>& a, const doubl
     if constexpr (E) {
         r.e[0] = f[1] * a.e[0];
         if constexpr (NT > 1) r.e[1] = f[2] * (a.e[0] * a.v[1]) + f[1] * a.e[1];
-        if constexpr (NT > 2)
-            r.e[2] = f[3] * (a.e[0] * (a.v[1] * a.v[1])) + f[2] * (2. * (a.v[1] * a.e[1]) + a.e[0] * a.v[2]) + f[1] * a.e[2];
     } else r.e[0] = 0.;
     return r;
 }
-// x^2 as Muscade's integer power rule evaluates it on a time jet (src/Adiff.jl:230):
-// exact to first order in t; at second order only 2·a·ä survives (see header).
-template <int NT, bool E> MH_HD Jet<NT, E> jsq_muscade(const Jet<NT, E>& a) {
-    Jet<NT, E> r;
-    r.v[0] = a.v[0] * a.v[0];
-    if constexpr (NT > 1) r.v[1] = 2. * (a.v[0] * a.v[1]);
-    if constexpr (NT > 2) r.v[2] = 2. * (a.v[0] * a.v[2]);
-    if constexpr (E) {
-        r.e[0] = 2. * (a.v[0] * a.e[0]);
-        if constexpr (NT > 1) r.e[1] = 2. * (a.e[0] * a.v[1] + a.v[0] * a.e[1]);
-        if constexpr (NT > 2) r.e[2] = 2. * (a.e[0] * a.v[2] + a.v[0] * a.e[2]);
-    } else r.e[0] = 0.;
-    return r;
-}
-
 // ------------------------------------------------------------ scalar functions
 // Derivatives of sinc1 with the branches of Rotations.jl:14-45.
 MH_HD double sinc1_d1(double x) {
@@ -136,36 +107,27 @@ MH_HD double sinc1_d2(double x) {
     double x2 = x * x;
     return -1. / 3. + x2 * (1. / 10. + x2 * (-1. / 168. + x2 * (1. / 6480.)));
 }
-MH_HD double sinc1_d3(double x) {
-    if (fabs(x) > 0.4) {
-        double s = sin(x), c = cos(x);
-        return -c / x + 3. * s / (x * x) + 6. * c / (x * x * x) - 6. * s / (x * x * x * x);
-    }
-    double x2 = x * x;
-    return x * (1. / 5. + x2 * (-1. / 42. + x2 * (1. / 1080. + x2 * (-1. / 55440. + x2 * (1. / 4717440.)))));
-}
 template <int NT, bool E> MH_HD Jet<NT, E> jsinc1(const Jet<NT, E>& a) {
     const double x = a.v[0];
-    double f[4];
+    double f[3];
     f[0] = sinc1(x);
     f[1] = sinc1_d1(x);
     f[2] = (NT + (E ? 1 : 0) > 2) ? sinc1_d2(x) : 0.;
-    f[3] = (NT + (E ? 1 : 0) > 3) ? sinc1_d3(x) : 0.;
     return jfun(a, f);
 }
 template <int NT, bool E> MH_HD Jet<NT, E> jsqrt(const Jet<NT, E>& a) {
     const double x = a.v[0], s = sqrt(x);
-    double f[4] = {s, 0.5 / s, -0.25 / (x * s), 0.375 / (x * x * s)};
+    double f[3] = {s, 0.5 / s, -0.25 / (x * s)};
     return jfun(a, f);
 }
 template <int NT, bool E> MH_HD Jet<NT, E> jrecip(const Jet<NT, E>& a) {
     const double x = a.v[0], r = 1. / x;
-    double f[4] = {r, -(r * r), 2. * (r * r * r), -6. * (r * r * r * r)};
+    double f[3] = {r, -(r * r), 2. * (r * r * r)};
     return jfun(a, f);
 }
 template <int NT, bool E> MH_HD Jet<NT, E> jacos(const Jet<NT, E>& a) {
     const double x = a.v[0], q = 1. - x * x, sq = sqrt(q);
-    double f[4] = {acos(x), -1. / sq, -x / (q * sq), -(1. + 2. * x * x) / (q * q * sq)};
+    double f[3] = {acos(x), -1. / sq, -x / (q * sq)};
     return jfun(a, f);
 }
 // scac(x) = sinc1(acos x); 5th-order series in x-1 for |x-1| <= 1e-3 (Rotations.jl:61-68)
@@ -173,11 +135,10 @@ template <int NT, bool E> MH_HD Jet<NT, E> jscac(const Jet<NT, E>& a) {
     const double d = a.v[0] - 1.;
     if (fabs(d) > 1e-3) return jsinc1(jacos(a));
     const double c1 = 1. / 3., c2 = -2. / 90., c3 = 0.0052911879917544626, c4 = -0.0016229317117234072, c5 = 0.0005625;
-    double f[4];
+    double f[3];
     f[0] = 1. + d * (c1 + d * (c2 + d * (c3 + d * (c4 + d * c5))));
     f[1] = c1 + d * (2. * c2 + d * (3. * c3 + d * (4. * c4 + d * (5. * c5))));
     f[2] = 2. * c2 + d * (6. * c3 + d * (12. * c4 + d * (20. * c5)));
-    f[3] = 6. * c3 + d * (24. * c4 + d * (60. * c5));
     return jfun(a, f);
 }
 
@@ -187,9 +148,7 @@ template <int NT, bool E> struct JV3 { Jet<NT, E> a[3]; };
 
 // Rodrigues(v) = I + sinc1(θ) S + (sinc1(θ/2)²/2) spin²(S), θ = norm3(v) (Rotations.jl:106-135):
 // the coefficient jets a = sinc1(θ), b = sinc1(θ/2)²/2.
-// XSQ = false: the square by Muscade's power rule on jets over solver partials (the
-// assembly); XSQ = true: the exact square (jets over plain values, as getresult evaluates).
-template <int NT, bool E, bool XSQ = false>
+template <int NT, bool E>
 MH_HD void jrodrigues_coef(const JV3<NT, E>& v, Jet<NT, E>& a, Jet<NT, E>& b) {
     using J = Jet<NT, E>;
     const J& x = v.a[0]; const J& y = v.a[1]; const J& z = v.a[2];
@@ -199,8 +158,7 @@ MH_HD void jrodrigues_coef(const JV3<NT, E>& v, Jet<NT, E>& a, Jet<NT, E>& b) {
     else th = jsqrt(ss);
     a = jsinc1(th);
     J s = jsinc1(0.5 * th);
-    if constexpr (XSQ) b = 0.5 * (s * s);
-    else b = 0.5 * jsq_muscade(s);
+    b = 0.5 * (s * s);
 }
 // Column k of Rodrigues(v) from its coefficients, spin²(S) entrywise (Rotations.jl:114-122).
 template <int K, int NT, bool E>
@@ -222,9 +180,9 @@ MH_HD JV3<NT, E> jrodrigues_col(const JV3<NT, E>& v, const Jet<NT, E>& a, const 
     }
     return r;
 }
-template <int NT, bool E, bool XSQ = false> MH_HD JM3<NT, E> jrodrigues(const JV3<NT, E>& v) {
+template <int NT, bool E> MH_HD JM3<NT, E> jrodrigues(const JV3<NT, E>& v) {
     Jet<NT, E> a, b;
-    jrodrigues_coef<NT, E, XSQ>(v, a, b);
+    jrodrigues_coef<NT, E>(v, a, b);
     JV3<NT, E> c0 = jrodrigues_col<0>(v, a, b), c1 = jrodrigues_col<1>(v, a, b), c2 = jrodrigues_col<2>(v, a, b);
     JM3<NT, E> r;
 #pragma unroll
@@ -256,20 +214,13 @@ template <int NT, bool E> MH_HD JV3<NT, E> jmulv(const JM3<NT, E>& A, const JV3<
 
 // ------------------------------------------------------------ element dynamics
 // Per element, what the loads need from the kinematics jets.
-template <bool E> struct DynKin {
-    Jet<1, E> r0[9];          // rₛₘ
-    Jet<1, E> r1[9], r2[9];   // ṙₛₘ, r̈ₛₘ
-    Jet<1, E> xd[4][3];       // ẋ at the Gauss points
-    Jet<1, E> xdd[4][3];      // ẍ at the Gauss points
-    double xe[4][3];          // ∂x/∂ε at the Gauss points (a column of the Jacobian of x w.r.t. X₀)
+struct DynKin {
+    double r0[9];             // rₛₘ
+    double r1[9], r2[9];      // ṙₛₘ, r̈ₛₘ
+    double xd[4][3];          // ẋ at the Gauss points
+    double xdd[4][3];         // ẍ at the Gauss points
 };
-template <int NT, bool E> MH_HD Jet<1, E> jslice(const Jet<NT, E>& a, int n) {
-    Jet<1, E> r;
-    r.v[0] = n < NT ? a.v[n] : 0.;
-    if constexpr (E) r.e[0] = n < NT ? a.e[n] : 0.;
-    else r.e[0] = 0.;
-    return r;
-}
+template <int NT> MH_HD double jlevel(const Jet<NT, false>& a, int n) { return n < NT ? a.v[n] : 0.; }
 
 // The rotation chain (v₁,v₂) ↦ (rₛₘ, Δv) of BeamElement.jl:192-208 on time jets.
 // Neither R₂ = Rodrigues(v₂) nor the relative rotation M = R₂R₁ᵀ is held whole: φ = Rodrigues⁻¹(M)
@@ -277,15 +228,15 @@ template <int NT, bool E> MH_HD Jet<1, E> jslice(const Jet<NT, E>& a, int n) {
 // formed a column at a time; rₛₘ = Rodrigues(Δv)·(R₁ rₘ) applies Rodrigues(Δv) to one column
 // of R₁rₘ at a time, w ↦ w + a Δv×w + b (Δv (Δv·w) − |Δv|² w). This keeps the live jets
 // of the chain to about 21 instead of the 27 of three whole matrices.
-template <int NT, bool E, bool XSQ = false>
+template <int NT, bool E>
 MH_HD void dyn_rotation_chain(const BeamGeo& G, const JV3<NT, E>& v1, const JV3<NT, E>& v2, JM3<NT, E>& rsm,
                               JV3<NT, E>& dv) {
     using J = Jet<NT, E>;
-    JM3<NT, E> R1 = jrodrigues<NT, E, XSQ>(v1);
+    JM3<NT, E> R1 = jrodrigues<NT, E>(v1);
     J tr, ax[3];
     {
         J a2, b2;
-        jrodrigues_coef<NT, E, XSQ>(v2, a2, b2);
+        jrodrigues_coef<NT, E>(v2, a2, b2);
         auto add = [&](const JV3<NT, E>& c2, int k, bool first) {
             const J* c1 = &R1.a[3 * k];
             J d = (c1[0] * c2.a[0] + c1[1] * c2.a[1]) + c1[2] * c2.a[2];
@@ -305,7 +256,7 @@ MH_HD void dyn_rotation_chain(const BeamGeo& G, const JV3<NT, E>& v1, const JV3<
     for (int c = 0; c < 3; ++c) dv.a[c] = 0.5 * ((0.5 * ax[c]) * rs);
     JM3<NT, E> R1m = jmul_const(R1, G.rm);
     J ah, bh;
-    jrodrigues_coef<NT, E, XSQ>(dv, ah, bh);
+    jrodrigues_coef<NT, E>(dv, ah, bh);
     const J& x = dv.a[0]; const J& y = dv.a[1]; const J& z = dv.a[2];
     J n2 = (x * x + y * y) + z * z;
 #pragma unroll
@@ -319,49 +270,47 @@ MH_HD void dyn_rotation_chain(const BeamGeo& G, const JV3<NT, E>& v1, const JV3<
     }
 }
 // Kinematics (BeamElement.jl:176-208) on time jets. Xj: the 12 element dofs as jets.
-template <int NT, bool E, bool XSQ = false>
-MH_HD void dyn_kinematics(const BeamGeo& G, const Jet<NT, E>* Xj, DynKin<E>& k) {
-    using J = Jet<NT, E>;
+template <int NT>
+MH_HD void dyn_kinematics(const BeamGeo& G, const Jet<NT, false>* Xj, DynKin& k) {
+    using J = Jet<NT, false>;
     const double L = G.L;
-    JV3<NT, E> u1, u2;
+    JV3<NT, false> u1, u2;
 #pragma unroll
     for (int c = 0; c < 3; ++c) { u1.a[c] = Xj[c]; u2.a[c] = Xj[6 + c]; }
-    JM3<NT, E> rsm;
-    JV3<NT, E> dv;
-    JV3<NT, E> v1, v2;
+    JM3<NT, false> rsm;
+    JV3<NT, false> dv;
+    JV3<NT, false> v1, v2;
 #pragma unroll
     for (int c = 0; c < 3; ++c) { v1.a[c] = Xj[3 + c]; v2.a[c] = Xj[9 + c]; }
-    dyn_rotation_chain<NT, E, XSQ>(G, v1, v2, rsm, dv);
+    dyn_rotation_chain<NT, false>(G, v1, v2, rsm, dv);
     // uₗ₂ = rₛₘᵀ(u₂ + tgₘ/2 - cₛ) - tgₑ/2,  vₗ₂ = rₛₘᵀ Δv
-    JV3<NT, E> dd, cs;
+    JV3<NT, false> dd, cs;
     const double tg[3] = {G.tgm.x, G.tgm.y, G.tgm.z};
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
         cs.a[c] = 0.5 * (u1.a[c] + u2.a[c]);
         dd.a[c] = (u2.a[c] + tg[c] * 0.5) - cs.a[c];
     }
-    JV3<NT, E> ul = jmulT(rsm, dd), vl = jmulT(rsm, dv);
+    JV3<NT, false> ul = jmulT(rsm, dd), vl = jmulT(rsm, dv);
     ul.a[0] = ul.a[0] + (-(L * 0.5));
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
         const double z = G.zgp[g];
         const double ya = 2. * z, yu = -4. * (z * z * z) + 3. * z, yv = (z * z - 1. / 4.) * L;
-        JV3<NT, E> p;
+        JV3<NT, false> p;
         p.a[0] = ya * ul.a[0] + L * z;
         p.a[1] = yu * ul.a[1] + yv * vl.a[2];
         p.a[2] = yu * ul.a[2] - yv * vl.a[1];
-        JV3<NT, E> x = jmulv(rsm, p);
+        JV3<NT, false> x = jmulv(rsm, p);
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
             J xc = x.a[c] + cs.a[c];
-            k.xd[g][c] = jslice(xc, 1);
-            k.xdd[g][c] = jslice(xc, 2);
-            if constexpr (E) k.xe[g][c] = xc.e[0];
-            else k.xe[g][c] = 0.;
+            k.xd[g][c] = jlevel(xc, 1);
+            k.xdd[g][c] = jlevel(xc, 2);
         }
     }
 #pragma unroll
-    for (int i = 0; i < 9; ++i) { k.r0[i] = jslice(rsm.a[i], 0); k.r1[i] = jslice(rsm.a[i], 1); k.r2[i] = jslice(rsm.a[i], 2); }
+    for (int i = 0; i < 9; ++i) { k.r0[i] = jlevel(rsm.a[i], 0); k.r1[i] = jlevel(rsm.a[i], 1); k.r2[i] = jlevel(rsm.a[i], 2); }
 }
 
 struct BeamDynSection {
@@ -372,40 +321,38 @@ struct BeamDynSection {
 // External loads of the resultants (BeamElement.jl:28-64): per Gauss point the force
 // fₑ (fw, inertia, added mass, linear and quadratic damping, minus U) and the
 // element's roll-inertia couple mₑ (the same at every Gauss point).
-template <bool E> MH_HD void dyn_loads(const DynKin<E>& k, const BeamDynSection& S, const double* U, Jet<1, E> (*fe)[3],
-                                       Jet<1, E>* me) {
-    using J = Jet<1, E>;
-    const J* r0 = k.r0;
+MH_HD void dyn_loads(const DynKin& k, const BeamDynSection& S, const double* U, double (*fe)[3], double* me) {
+    const double* r0 = k.r0;
     for (int g = 0; g < 4; ++g) {
-        J xl1[3], xl2[3];
+        double xl1[3], xl2[3];
 #pragma unroll
         for (int j = 0; j < 3; ++j) {   // x ∘₁ r₀ = r₀ᵀx
             xl1[j] = (k.xd[g][0] * r0[3 * j] + k.xd[g][1] * r0[3 * j + 1]) + k.xd[g][2] * r0[3 * j + 2];
             xl2[j] = (k.xdd[g][0] * r0[3 * j] + k.xdd[g][1] * r0[3 * j + 1]) + k.xdd[g][2] * r0[3 * j + 2];
         }
-        J fal[3], fll[3], fql[3];
+        double fal[3], fll[3], fql[3];
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
             fal[j] = S.Ca[j] * xl2[j];
             fll[j] = S.Cl[j] * xl1[j];
-            J q = S.Cq[j] * (xl1[j] * xl1[j]);
-            fql[j] = xl1[j].v[0] < 0. ? -q : q;
+            double q = S.Cq[j] * (xl1[j] * xl1[j]);
+            fql[j] = xl1[j] < 0. ? -q : q;
         }
 #pragma unroll
         for (int i = 0; i < 3; ++i) {
-            J fa = (r0[i] * fal[0] + r0[i + 3] * fal[1]) + r0[i + 6] * fal[2];
-            J fl = (r0[i] * fll[0] + r0[i + 3] * fll[1]) + r0[i + 6] * fll[2];
-            J fq = (r0[i] * fql[0] + r0[i + 3] * fql[1]) + r0[i + 6] * fql[2];
-            J f = (((S.mu * k.xdd[g][i] + fa) + fl) + fq) + (i == 2 ? S.w : 0.);
+            double fa = (r0[i] * fal[0] + r0[i + 3] * fal[1]) + r0[i + 6] * fal[2];
+            double fl = (r0[i] * fll[0] + r0[i + 3] * fll[1]) + r0[i + 6] * fll[2];
+            double fq = (r0[i] * fql[0] + r0[i + 3] * fql[1]) + r0[i + 6] * fql[2];
+            double f = (((S.mu * k.xdd[g][i] + fa) + fl) + fq) + (i == 2 ? S.w : 0.);
             fe[g][i] = f + (-U[i]);
         }
     }
     // vᵢ₂ = spin⁻¹(ṙᵀṙ + r₀ᵀr̈) (Rotations.jl:177-182); only its first component is used
-    J a21 = ((k.r1[6] * k.r1[3] + k.r1[7] * k.r1[4]) + k.r1[8] * k.r1[5]) +
+    double a21 = ((k.r1[6] * k.r1[3] + k.r1[7] * k.r1[4]) + k.r1[8] * k.r1[5]) +
             ((r0[6] * k.r2[3] + r0[7] * k.r2[4]) + r0[8] * k.r2[5]);
-    J a12 = ((k.r1[3] * k.r1[6] + k.r1[4] * k.r1[7]) + k.r1[5] * k.r1[8]) +
+    double a12 = ((k.r1[3] * k.r1[6] + k.r1[4] * k.r1[7]) + k.r1[5] * k.r1[8]) +
             ((r0[3] * k.r2[6] + r0[4] * k.r2[7]) + r0[5] * k.r2[8]);
-    J m1 = S.iota1 * (0.5 * (a21 - a12));
+    double m1 = S.iota1 * (0.5 * (a21 - a12));
 #pragma unroll
     for (int i = 0; i < 3; ++i) me[i] = r0[i] * m1;
 }
@@ -416,43 +363,9 @@ MH_HD v3 rotvec(const m3& r) {
     return mk((at(r, 2, 1) - at(r, 1, 2)) / 2. / sc, (at(r, 0, 2) - at(r, 2, 0)) / 2. / sc, (at(r, 1, 0) - at(r, 0, 1)) / 2. / sc);
 }
 
-// The element dofs of the solver's trial path as jets.
-//   dir 0..11: δX along dof `dir`, with weights (w0·s, a₁s, b₁s), s = scale.X[dir]
-//              (w0 = 1 for the solver; w0 = 0 isolates the X′ or X″ partials);
-//   dir 12:    δr of :step, (0, a, b) with a = a₂X₁ + a₃X₂, b = b₂X₁ + b₃X₂ per dof;
-//   dir 13:    X₀ + ε·lam (a directional derivative along lam, 12 values);
-//   otherwise: no ε seed.
-// X: ND rows of 12; c = (a₁,a₂,a₃,b₁,b₂,b₃).
-template <int NT, bool E> MH_HD void dyn_seed(const double (*X)[12], const double* scale, const double* c, int dir,
-                                              Jet<NT, E>* Xj, double w0 = 1., const double* lam = nullptr) {
-#pragma unroll
-    for (int i = 0; i < 12; ++i) {
-        Jet<NT, E> q = jzero<NT, E>();
-#pragma unroll
-        for (int n = 0; n < NT; ++n) q.v[n] = X[n][i];
-        if constexpr (E) {
-            if (dir == 13) {
-                q.e[0] = lam[i];
-            } else if (dir == i) {
-                q.e[0] = w0 * scale[i];
-                if constexpr (NT > 1) q.e[1] = c[0] * scale[i];
-                if constexpr (NT > 2) q.e[2] = c[3] * scale[i];
-            } else if (dir == 12) {
-                if constexpr (NT == 2) q.e[1] = c[1] * X[1][i];
-                if constexpr (NT == 3) {
-                    q.e[1] = c[1] * X[1][i] + c[2] * X[2][i];
-                    q.e[2] = c[4] * X[1][i] + c[5] * X[2][i];
-                }
-            }
-        }
-        Xj[i] = q;
-    }
-}
-
 // Requestables of the element (BeamElement.jl:28-64,151-174) at X (ND time levels), what
 // getresult extracts (src/Output.jl:131-181). getresult evaluates the element on plain
-// values, so the time jets carry no solver partials and every square is exact (no
-// power-rule artefact). ☼ε and ♢κ = (vₗ₂[1], vₗ₂[3], −vₗ₂[2])·2/L
+// values. ☼ε and ♢κ = (vₗ₂[1], vₗ₂[3], −vₗ₂[2])·2/L
 // with their ND time levels, then per Gauss point ☼x and ☼κgp (ND levels each) and the
 // resultants' ☼fᵢ, ☼mᵢ, ☼fₑ (as returned by `resultants`, before the U-load is subtracted)
 // and ☼mₑ. Layout: ε[ND], κ[ND][3], then per Gauss point x[ND][3], κgp[ND][3], fᵢ, mᵢ[3],
@@ -462,14 +375,19 @@ template <int ND> MH_HD void dyn_requestables(const BeamGeo& G, const BeamSectio
                                               const double (*X)[12], double* __restrict__ out) {
     using J = Jet<ND, false>;
     J Xj[12];
-    dyn_seed<ND, false>(X, nullptr, nullptr, -1, Xj);
+#pragma unroll
+    for (int i = 0; i < 12; ++i) {
+        Xj[i] = jzero<ND, false>();
+#pragma unroll
+        for (int n = 0; n < ND; ++n) Xj[i].v[n] = X[n][i];
+    }
     const double L = G.L;
     JV3<ND, false> u1, u2, v1, v2;
 #pragma unroll
     for (int c = 0; c < 3; ++c) { u1.a[c] = Xj[c]; u2.a[c] = Xj[6 + c]; v1.a[c] = Xj[3 + c]; v2.a[c] = Xj[9 + c]; }
     JM3<ND, false> rsm;
     JV3<ND, false> dv;
-    dyn_rotation_chain<ND, false, true>(G, v1, v2, rsm, dv);
+    dyn_rotation_chain<ND, false>(G, v1, v2, rsm, dv);
     JV3<ND, false> dd, cs;
     const double tg[3] = {G.tgm.x, G.tgm.y, G.tgm.z};
     const double cm[3] = {G.cm.x, G.cm.y, G.cm.z};
@@ -492,11 +410,11 @@ template <int ND> MH_HD void dyn_requestables(const BeamGeo& G, const BeamSectio
 #pragma unroll
         for (int c = 0; c < 3; ++c) out[q++] = km[c].v[d];
     // loads (values) from the time jets of the Gauss points
-    DynKin<false> k;
-    dyn_kinematics<ND, false, true>(G, Xj, k);
-    Jet<1, false> fe[4][3], me[3];
+    DynKin k;
+    dyn_kinematics<ND>(G, Xj, k);
+    double fe[4][3], me[3];
     const double U0[3] = {0., 0., 0.};
-    dyn_loads<false>(k, D, U0, fe, me);
+    dyn_loads(k, D, U0, fe, me);
     const double ka = 2. / L, kv = 2. / L;
     for (int g = 0; g < 4; ++g) {
         const double z = G.zgp[g];
@@ -521,17 +439,16 @@ template <int ND> MH_HD void dyn_requestables(const BeamGeo& G, const BeamSectio
         out[q++] = S.EI3 * kg[1].v[0];
         out[q++] = S.EI2 * kg[2].v[0];
 #pragma unroll
-        for (int c = 0; c < 3; ++c) out[q++] = fe[g][c].v[0];
+        for (int c = 0; c < 3; ++c) out[q++] = fe[g][c];
 #pragma unroll
-        for (int c = 0; c < 3; ++c) out[q++] = me[c].v[0];
+        for (int c = 0; c < 3; ++c) out[q++] = me[c];
     }
 }
 
 // The strain-gauge requestables εₐₓ = ε and κ = ♢κ (BeamElement.jl:155,172;
 // StrainGaugeOnBeamElement.jl:73) on jets whose "time" level carries ∂/∂X_i and whose ε
 // level carries ∂/∂X_j: with the seeds X_k = X₀_k + t·δ_ki + ε·δ_kj, v[0] is the value,
-// v[1] = ∂/∂X_i, e[0] = ∂/∂X_j and e[1] = ∂²/∂X_i∂X_j (exact squares: second derivatives
-// at the value level, as revariate{2} forms them, have no power-rule artefact).
+// v[1] = ∂/∂X_i, e[0] = ∂/∂X_j and e[1] = ∂²/∂X_i∂X_j.
 MH_HD void gauge_jets(const BeamGeo& G, const double* X0, int i, int j, Jet<2, true>* q) {
     using J = Jet<2, true>;
     J Xj[12];
@@ -546,7 +463,7 @@ MH_HD void gauge_jets(const BeamGeo& G, const double* X0, int i, int j, Jet<2, t
     for (int c = 0; c < 3; ++c) { u1.a[c] = Xj[c]; u2.a[c] = Xj[6 + c]; v1.a[c] = Xj[3 + c]; v2.a[c] = Xj[9 + c]; }
     JM3<2, true> rsm;
     JV3<2, true> dv;
-    dyn_rotation_chain<2, true, true>(G, v1, v2, rsm, dv);
+    dyn_rotation_chain<2, true>(G, v1, v2, rsm, dv);
     JV3<2, true> dd;
     const double tg[3] = {G.tgm.x, G.tgm.y, G.tgm.z};
 #pragma unroll

@@ -348,7 +348,7 @@ struct BeamLoads { v3 e0, ea, eu, ev, m; };
 // out of Q (the ω-ω part) and of the coupling to translations.
 //
 // Bound: FP64 latency at two waves per SIMD, then HBM. Over six columns of global spins the same
-// Hessian took 6,299 operations and 462 registers (one wave per SIMD); here about 2,000 and 256.
+// element took 6,299 counted operations and 462 registers (one wave per SIMD); here 2,794 and 256.
 // 973,000 elements: 320 µs before, 142 now.
 struct BeamSpin {
     v3 Fb, N, Fv, ve, a, u;          // forces and moment, body loads
@@ -638,13 +638,6 @@ MH_HD int beam_static_vjp(const BeamGeo& G, const BeamSection& S, v3 fe, const d
     int nan = !((at(r, 0, 0) + at(r, 1, 1) + at(r, 2, 2) - 1.) / 2. > -1.);
     for (int i = 0; i < 12; ++i) nan |= g[i] != g[i];
     return nan;
-}
-
-// Full 12×12 entry from the compact form (host harnesses and checks).
-MH_HD double compact_entry(const double* Kc, int i, int j) {
-    double m;
-    int s = compact_slot(i, j, &m);
-    return m * Kc[s];
 }
 
 }  // namespace mh

@@ -20,13 +20,13 @@
 //
 // Block cyclic reduction (no pivoting between blocks, partial pivoting inside a block)
 //   level s = 1, 2, 4, …: blocks i ≡ s (mod 2s) are eliminated, blocks j ≡ 0 (mod 2s) kept.
-//   factor:  D_i = P⁻¹LU; L_i ← D_i⁻¹L_i, U_i ← D_i⁻¹U_i, b_i ← D_i⁻¹b_i        (in place)
-//   update:  D_j −= L_j U_{j−s} + U_j L_{j+s};  b_j −= L_j b_{j−s} + U_j b_{j+s};
-//            L_j ← −L_j L_{j−s} (couples j−2s),  U_j ← −U_j U_{j+s} (couples j+2s)
-//   top:     x_0 = D_0⁻¹ b_0
-//   back:    for s descending, x_i = b_i − L_i x_{i−s} − U_i x_{i+s}     (x overwrites b)
-//   Every eliminated block is written once and read-only afterwards, so the levels run
-//   in place without a second copy; a kept block is written only by its own lanes.
+//   eliminate: L_i ← D_i⁻¹L_i, U_i ← D_i⁻¹U_i, b_i ← D_i⁻¹b_i by Gauss-Jordan elimination    (in place)
+//   update:    D_j −= L_j U_{j−s} + U_j L_{j+s};  b_j −= L_j b_{j−s} + U_j b_{j+s};
+//              L_j ← −L_j L_{j−s} (couples j−2s),  U_j ← −U_j U_{j+s} (couples j+2s)
+//   top:       x_0 = D_0⁻¹ b_0
+//   back:      for s descending, x_i = b_i − L_i x_{i−s} − U_i x_{i+s}     (x overwrites b)
+//   Six levels run in a workgroup's LDS at a time (reduce_kernel): the eliminated blocks of a chunk
+//   go back in place, its first block to the system of the next phase.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <cmath>
