@@ -2236,7 +2236,7 @@ static int build_rmap(Ctx* c) {
     dfree(tmp);
     hipLaunchKernelGGL(rseg_kernel, dim3(grid(nR + 1)), dim3(kBlock), 0, s, nR, rkout, nX, c->d_rseg);
     if (int r = check_launch(c, "rhs pattern")) return r;
-    HIPCHK(c, hipStreamSynchronize(s));
+    if (int r = build_long(c, nX, nullptr, c->d_rseg, c->nrlong, c->d_rlong)) return r;   // waits for the stream
     dfree(rkin); dfree(rkout); dfree(rvin);
     return MH_OK;
 }
@@ -2683,7 +2683,6 @@ int mh_prepare_sweepx(mh_ctx* c, int OX, int64_t* nnz_out) {
     HIPCHK(c, hipStreamSynchronize(s));
     dfree(kin); dfree(kout); dfree(vin); dfree(head); dfree(id); dfree(colk);
     if (int r = build_rmap(c)) return r;
-    if (int r = build_long(c, nX, nullptr, c->d_rseg, c->nrlong, c->d_rlong)) return r;
     unsigned int *rkin = nullptr, *rkout = nullptr;
     uint32_t* rvin = nullptr;
     // ---- U-dof map (gradients ∂L/∂U of the adjoint), same construction over the U class
